@@ -13,25 +13,34 @@
 // node vector and block group (nn/kernels.py:575-603, over _block_weights
 // :506-536) and their gradients through autograd.
 //
-// All three are v_mfma_f32_16x16x4f32 products.  Lane l = 16 q + c of the
-// MFMA supplies A[c][q] and B[q][c] and holds D[4 q + i][c], i < 4.
+// All three are MFMA products in float32 accuracy: vectors of 17 to 128 reals
+// as split bf16 products over 32 contraction indices an instruction
+// (node_mix_*_deep), vectors up to 16 over 16 (node_mix_*_split), and under
+// GM_SPLIT_PRODUCTS=0 v_mfma_f32_16x16x4f32 (lane l = 16 q + c supplies A[c][q]
+// and B[q][c] and holds D[4 q + i][c], i < 4).
 //
 // * forward: the contraction is short, so each wave keeps its columns of M in
 //   registers for the whole launch and streams 64-row tiles of v through LDS;
 //   M is the A operand (D = mix^T), so a lane's four D entries are four
 //   consecutive columns of one row: one 16-byte store each.
-// * input gradient: 128-row tiles, each wave 32 rows over the whole
-//   contraction, dmix and M staged per 64-column chunk in LDS; the
-//   accumulators restart every four chunks into a running total, so no fp32
-//   sum runs sequentially over more than 256 columns.
-// * weight gradient: split over row ranges into partial (w, C) matrices, each
-//   from 64-row chunks staged in LDS (up to 64-wide vectors: one partial per
-//   wave, each wave a quarter of every chunk over the workgroup's whole
-//   w x 64 tile, so an operand read feeds four MFMAs); a second pass sums the
-//   partials in a fixed order.  No atomics anywhere: results are deterministic.
+// * input gradient: 128-row tiles, each wave 32 rows over the contraction, M
+//   staged per chunk of columns in LDS; the accumulators restart every 256
+//   columns into a running total, so no fp32 sum runs sequentially over more.
+// * weight gradient: split over row ranges into partial (w, C) matrices; a
+//   second pass sums the partials in a fixed order.  No atomics anywhere:
+//   results are deterministic.
+//
+// Bound: the bytes of the mixes, (N, C) written by the forward and read by each
+// gradient.  256x512, B = 4 (N = 524,288), w = 64, C = 5,440 (11.4 GB; a plain
+// read of them takes 1.85 ms, a plain write 2.0), 16-deep -> 32-deep: forward
+// 3.21 -> 2.60 ms, input gradient 3.06 -> 2.61, weight gradient 3.35 -> 2.48;
+// w = 32, C = 2,720: 1.25 -> 1.06, 1.12 -> 1.10, 1.14 -> 1.05; w = 128, N =
+// 65,536, C = 26,112 (6.8 GB): 3.82 -> 2.57, 3.98 -> 2.50, 5.55 -> 2.75.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "split.hpp"
@@ -499,17 +508,12 @@ __device__ __forceinline__ float4 load_dm4(const uint16_t* src) {
 // fp32 accuracy: split.hpp).  A 16-deep contraction chunk kc gives lane
 // (c, q) the indices 16 kc + 4 q + s, s < 4, in both operands.
 
-// The split kernels' tiling by vector width: columns a forward wave owns
-// (16 SplitCT), rows an input-gradient wave owns (16 SplitRT) and columns a
-// weight-gradient workgroup owns (16 SplitJT); the widest vectors take the
-// narrower tiles so the accumulators and held operands stay within a wave's
-// registers.
-template <int W>
-constexpr int SplitCT = W == 128 ? 1 : 2;
-template <int W>
-constexpr int SplitRT = W == 128 ? 1 : 2;
-template <int W>
-constexpr int SplitJT = W == 128 ? 2 : 4;
+// These 16-deep forms serve vectors up to 16 reals (a 32-deep operand would be
+// half zeros); wider ones take the 32-deep forms below.  The split kernels'
+// tiling: columns a forward wave owns (16 kSplitCT), rows an input-gradient
+// wave owns (16 kSplitRT) and columns a weight-gradient workgroup owns
+// (16 kSplitJT).
+constexpr int kSplitCT = 2, kSplitRT = 2, kSplitJT = 4;
 
 // A SplitB operand from three bf16 planes (four contraction indices each).
 __device__ __forceinline__ SplitB split_b_planes(uint2 hi, uint2 mid, uint2 lo) {
@@ -525,42 +529,44 @@ __device__ __forceinline__ void store_planes(uint16_t* plane0, uint16_t* plane1,
   *reinterpret_cast<uint2*>(plane2 + at) = make_uint2(sp.lo[0], sp.lo[1]);
 }
 
-// Four values' pieces as the three B operands themselves, one 16-byte record
-// each ([hi, hi], [mid, mid], [lo, hi] slot pairs): a wave then reads an
-// operand straight into its registers instead of assembling it from planes.
-__device__ __forceinline__ void store_operands(uint4* rec, float4 x) {
-  const Split4 sp = split4(x.x, x.y, x.z, x.w);
-  rec[0] = make_uint4(sp.hi[0], sp.hi[1], sp.hi[0], sp.hi[1]);
-  rec[1] = make_uint4(sp.mid[0], sp.mid[1], sp.mid[0], sp.mid[1]);
-  rec[2] = make_uint4(sp.lo[0], sp.lo[1], sp.hi[0], sp.hi[1]);
-}
-
-__device__ __forceinline__ SplitB load_operands(const uint4* rec) {
-  const uint4 hh = rec[0], mm = rec[1], lh = rec[2];
-  return SplitB{u32x4{hh.x, hh.y, hh.z, hh.w}, u32x4{mm.x, mm.y, mm.z, mm.w}, u32x4{lh.x, lh.y, lh.z, lh.w}};
+// Four consecutive columns of an output row; FULL: a whole row tile and whole
+// aligned columns (no checks, so the stores do not break up the product's
+// code: 3.86 -> 2.6 ms for 64 reals at N = 524,288 against a check a store),
+// else those below C of the rows below N.
+template <bool FULL>
+__device__ __forceinline__ void store4(float* out, int64_t row, int64_t col, int64_t N, int64_t C, floatx4 x,
+                                       int vec_out) {
+  float* dst = out + row * C + col;
+  if constexpr (FULL) {
+    *reinterpret_cast<floatx4*>(dst) = x;
+  } else {
+    if (row >= N) return;
+    if (vec_out && col + 3 < C) {
+      *reinterpret_cast<floatx4*>(dst) = x;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (col + i < C) dst[i] = x[i];
+    }
+  }
 }
 
 // Forward: wave wv of workgroup x owns columns x * 64 CT + 16 CT wv + 16 j + c
 // (j < CT); the pieces of M at those columns are split once per wave and held
 // in registers; each 64-row tile of v is split once per workgroup into LDS, from
-// which every wave takes its B operands: for 64 reals as the operands
-// themselves (48 bytes a four-value group, rows of W / 4 + 1 groups so neither
-// the staging writes nor a 16-lane read meet in a bank), for the other widths
-// as three bf16 planes (row stride W + 4 halfwords: a 16-lane 8-byte read
-// covers 32 banks once) assembled into operands by each wave.
+// which every wave takes its B operands: three bf16 planes (row stride W + 4
+// halfwords: a 16-lane 8-byte read covers 32 banks once) assembled into
+// operands by each wave.
 template <int W, typename V = float>
 __global__ __launch_bounds__(kThreads) void node_mix_forward_split(const V* __restrict__ v, int64_t ldv,
                                                                    const float* __restrict__ M, int64_t N, int w,
                                                                    int64_t C, float* __restrict__ out, int vec_v,
                                                                    int vec_out) {
-  constexpr int KC = W / 16, CT = SplitCT<W>;
+  constexpr int KC = W / 16, CT = kSplitCT;
   constexpr int LDP = W + 4;
   constexpr int QUADS = 64 * W / 4;
   constexpr int PER = (QUADS + kThreads - 1) / kThreads;
-  constexpr bool OPS = W == 64;       // operands staged as records (w = 64: 3.39 -> 3.32 ms at NS; w = 32 slower)
-  constexpr int GP = W / 4 + 1;       // record groups a staged row
-  __shared__ __align__(16) uint16_t vp[OPS ? 1 : 3][OPS ? 8 : 64 * LDP];
-  __shared__ __align__(16) uint4 vr[OPS ? 64 * GP * 3 : 1];
+  __shared__ __align__(16) uint16_t vp[3][64 * LDP];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
   const int64_t col0 = (int64_t)blockIdx.x * (64 * CT) + 16 * CT * wv;
   SplitA ma[KC][CT];
@@ -594,81 +600,46 @@ __global__ __launch_bounds__(kThreads) void node_mix_forward_split(const V* __re
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
       const int idx = threadIdx.x + p * kThreads;
-      if (idx < QUADS) {
-        if constexpr (OPS)
-          store_operands(&vr[((idx / (W / 4)) * GP + idx % (W / 4)) * 3], pre[p]);
-        else
-          store_planes(vp[0], vp[1], vp[2], (idx / (W / 4)) * LDP + 4 * (idx % (W / 4)), pre[p]);
-      }
+      if (idx < QUADS) store_planes(vp[0], vp[1], vp[2], (idx / (W / 4)) * LDP + 4 * (idx % (W / 4)), pre[p]);
     }
     __syncthreads();
     if (tile + gridDim.y < n_tiles) fetch(tile + gridDim.y);
     const int64_t row0 = tile * 64;
+    auto product = [&](auto full) {
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      floatx4 acc[CT];
+      for (int rt = 0; rt < 4; ++rt) {
+        floatx4 acc[CT];
 #pragma unroll
-      for (int j = 0; j < CT; ++j) acc[j] = kZero4;
+        for (int j = 0; j < CT; ++j) acc[j] = kZero4;
 #pragma unroll
-      for (int kc = 0; kc < KC; ++kc) {
-        SplitB b;
-        if constexpr (OPS) {
-          b = load_operands(&vr[((16 * rt + c) * GP + 4 * kc + q) * 3]);
-        } else {
+        for (int kc = 0; kc < KC; ++kc) {
           const int at = (16 * rt + c) * LDP + 16 * kc + 4 * q;
-          b = split_b_planes(*reinterpret_cast<const uint2*>(&vp[0][at]), *reinterpret_cast<const uint2*>(&vp[1][at]),
-                             *reinterpret_cast<const uint2*>(&vp[2][at]));
-        }
+          const SplitB b = split_b_planes(*reinterpret_cast<const uint2*>(&vp[0][at]),
+                                          *reinterpret_cast<const uint2*>(&vp[1][at]),
+                                          *reinterpret_cast<const uint2*>(&vp[2][at]));
 #pragma unroll
-        for (int j = 0; j < CT; ++j) acc[j] = mfma_split(ma[kc][j], b, acc[j]);
-      }
-      if constexpr (CT == 2 && !OPS) {
+          for (int j = 0; j < CT; ++j) acc[j] = mfma_split(ma[kc][j], b, acc[j]);
+        }
         // Lane (c, q) holds row c's columns 4q.. of both 16-column tiles.  Lanes c and c ^ 8
         // trade halves (c < 8 gives its second tile, c >= 8 its first; one DPP rotate by 8
         // within each 16-lane row), so each of the two stores writes eight whole rows of the
-        // wave's 32 columns (128 contiguous bytes a row) instead of 64-byte halves of sixteen:
-        // 1.44 -> 1.23 ms for w = 32 at 256x512, B = 4.  The 64-real form keeps its stores
-        // (3.31 vs 3.35 ms with the trade: its stores then wait for both tiles' longer chains).
+        // wave's 32 columns (128 contiguous bytes a row) instead of 64-byte halves of sixteen.
         const bool lo = c < 8;
         floatx4 sw;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           sw[i] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(lo ? acc[1][i] : acc[0][i]),
                                                              kDppRowRor8, 0xF, 0xF, false));
-        const int64_t col = col0 + 16 * (c >> 3) + 4 * q;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int64_t row = row0 + 16 * rt + 8 * h + (c & 7);
-          const floatx4 val = (h == 0) == lo ? acc[h] : sw;
-          if (row < N) {
-            float* dst = out + row * C;
-            if (vec_out && col + 3 < C) {
-              *reinterpret_cast<float4*>(dst + col) = make_float4(val[0], val[1], val[2], val[3]);
-            } else {
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (col + i < C) dst[col + i] = val[i];
-            }
-          }
-        }
-      } else {
-        const int64_t row = row0 + 16 * rt + c;
-        if (row < N) {
-          float* dst = out + row * C;
-#pragma unroll
-          for (int j = 0; j < CT; ++j) {
-            const int64_t col = col0 + 16 * j + 4 * q;
-            if (vec_out && col + 3 < C) {
-              *reinterpret_cast<float4*>(dst + col) = make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
-            } else {
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (col + i < C) dst[col + i] = acc[j][i];
-            }
-          }
-        }
+        for (int h = 0; h < 2; ++h)
+          store4<full()>(out, row0 + 16 * rt + 8 * h + (c & 7), col0 + 16 * (c >> 3) + 4 * q, N, C,
+                         (h == 0) == lo ? acc[h] : sw, vec_out);
       }
-    }
+    };
+    if (vec_out && row0 + 64 <= N && col0 + 16 * CT <= C)
+      product(std::true_type{});
+    else
+      product(std::false_type{});
   }
 }
 
@@ -680,14 +651,12 @@ template <int W>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void node_mix_dinput_split(const float* __restrict__ dmix,
                                                                   const float* __restrict__ M, int64_t N, int w,
                                                                   int64_t C, float* __restrict__ dv, int64_t lddv) {
-  constexpr int RT = SplitRT<W>, ROWS = 64 * RT;
-  // chunks of KC columns (32 for the widest vectors: fewer staged registers); LDM: a 16-lane 8-byte read
-  // covers 32 banks once
-  constexpr int KC = W == 128 ? 32 : 64, LDM = KC + 4, JW = W / 16, KS = KC / 16;
-  // 64-column chunks of dmix unpadded, 16-byte unit u of row r at u ^ (r mod 16): a 16-byte read's set of
+  constexpr int RT = kSplitRT, ROWS = 64 * RT;
+  // LDM: a 16-lane 8-byte read covers 32 banks once
+  constexpr int KC = 64, LDM = KC + 4, JW = W / 16, KS = KC / 16;
+  // dmix rows unpadded, 16-byte unit u of row r at u ^ (r mod 16): a 16-byte read's set of
   // 16 lanes (c < 8 of one lane row, c >= 8 of another) then meets 16 distinct bank quads
-  constexpr bool SWZ = KC == 64;
-  constexpr int LDD = SWZ ? KC : KC + 4;
+  constexpr int LDD = KC;
   constexpr int TOTAL_EVERY = 256 / KC;  // chunks a running sum spans before it joins the total
   constexpr int DQ = ROWS * KC / 4 / kThreads;
   constexpr int MQ = W * KC / 4 / kThreads;
@@ -726,7 +695,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int p = 0; p < DQ; ++p) {
       const int idx = threadIdx.x + p * kThreads;
-      const int u = SWZ ? (idx % CQ) ^ ((idx / CQ) & 15) : idx % CQ;
+      const int u = (idx % CQ) ^ ((idx / CQ) & 15);
       *reinterpret_cast<float4*>(&dt[(idx / CQ) * LDD + 4 * u]) = pd[p];
     }
 #pragma unroll
@@ -741,7 +710,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       SplitA a[RT];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        const int u = SWZ ? (4 * kc + q) ^ c : 4 * kc + q;
+        const int u = (4 * kc + q) ^ c;
         const float4 x = *reinterpret_cast<const float4*>(&dt[(16 * RT * wv + 16 * rt + c) * LDD + 4 * u]);
         a[rt] = split_a(x.x, x.y, x.z, x.w);
       }
@@ -789,7 +758,7 @@ __global__ __launch_bounds__(kThreads) void node_mix_dweight_split(const V* __re
                                                                    const DM* __restrict__ dmix, int64_t N, int w,
                                                                    int64_t C, int64_t rps, float* __restrict__ partial,
                                                                    int vec_v) {
-  constexpr int JT = SplitJT<W>, COLS = 16 * JT;
+  constexpr int JT = kSplitJT, COLS = 16 * JT;
   // lanes (c, q) read rows 16 wv + 4 q + s: strides with 4 LD = 16 (mod 64) words put a quarter-wave's
   // rows in distinct banks
   constexpr int RC = 64, LDV = W + 4, LDM = COLS + 4, IW = W / 16;
@@ -866,6 +835,402 @@ __global__ __launch_bounds__(kThreads) void node_mix_dweight_split(const V* __re
     }
 }
 
+// ---------------------------------------------------------------- 32-deep split products
+//
+// The same products for vectors of 17 to 128 reals with each operand register
+// holding one piece of 32 contraction indices (lane (c, q) the indices 32 kd +
+// 8 q + s, s < 8): six instructions per 32 indices, three operand registers
+// sets a side (hi, mid, lo) and none of them assembled from halves, so half the
+// LDS reads and no register copies next to the 16-deep form.  Bfloat16 operands
+// are their own hi piece (P = 1): the products with their mid and lo pieces,
+// exact zeros, are left out.
+//
+// LDS operands are 16-byte units of eight bf16 values of one piece; a row of U
+// units keeps unit u at u ^ (row mod U), so that neither the staging writes
+// nor a 16-lane set of operand reads meet in a bank.
+template <int P>
+struct Pieces {
+  u32x4 p[P];
+};
+
+template <int P>
+__device__ __forceinline__ Pieces<P> pieces8(const float (&x)[8]) {
+  Pieces<P> r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (P == 1) {
+      r.p[0][i] = pack_bf16(x[2 * i], x[2 * i + 1]);
+    } else {
+      const SplitPair sp = split_pair(x[2 * i], x[2 * i + 1]);
+      r.p[0][i] = sp.hi;
+      r.p[1][i] = sp.mid;
+      r.p[2][i] = sp.lo;
+    }
+  }
+  return r;
+}
+
+// acc[t] += A[t] B over 32 contraction indices for T tiles, the smallest
+// products first (pieces of order i + j = 2, 1, 0), the tiles' chains side by side.
+template <int T, int PA, int PB>
+__device__ __forceinline__ void mfma_pieces(const Pieces<PA> (&a)[T], const Pieces<PB>& b, floatx4 (&acc)[T]) {
+#pragma unroll
+  for (int order = 2; order >= 0; --order)
+#pragma unroll
+    for (int i = 0; i <= order; ++i) {
+      if (i >= PA || order - i >= PB) continue;
+#pragma unroll
+      for (int t = 0; t < T; ++t) acc[t] = mfma_bf16(a[t].p[i], b.p[order - i], acc[t]);
+    }
+}
+
+template <int W>
+constexpr int DeepCT = W == 128 ? 2 : 4;  // 16-column tiles a forward wave holds
+template <int W>
+constexpr int DeepJT = W == 128 ? 2 : 4;  // column tiles a weight-gradient wave owns
+template <int U>
+__device__ __forceinline__ int deep_unit(int row, int u) {
+  return row * U + (u ^ (U >= 8 ? row & (U - 1) : (row >> 2) & (U - 1)));
+}
+
+// Eight consecutive reals k .. k + 7 (zero at and past w).
+template <typename V>
+__device__ __forceinline__ void load8(const V* src, int k, int w, int vec, float (&x)[8]) {
+  const float4 a = load_v4(src, k, w, vec), b = load_v4(src + 4, k + 4, w, vec);
+  x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w;
+  x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+}
+
+// Forward: wave wv of workgroup x owns columns x 64 CT + 16 CT wv + 16 j + c
+// (j < CT), M's pieces at them held in registers; each 64-row tile of v is split
+// once per workgroup into LDS.
+template <int W, typename V = float>
+__global__ __launch_bounds__(kThreads, 2) void node_mix_forward_deep(const V* __restrict__ v, int64_t ldv,
+                                                                     const float* __restrict__ M, int64_t N, int w,
+                                                                     int64_t C, float* __restrict__ out, int vec_v,
+                                                                     int vec_out) {
+  constexpr int KD = W / 32, CT = DeepCT<W>, U = W / 8, PV = sizeof(V) == 2 ? 1 : 3;
+  constexpr int PER = 64 * U / kThreads;  // staged units a thread
+  static_assert(PER * kThreads == 64 * U, "whole units a thread");
+  __shared__ __align__(16) u32x4 vs[PV][64 * U];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
+  const int64_t col0 = (int64_t)blockIdx.x * (64 * CT) + 16 * CT * wv;
+  Pieces<3> ma[KD][CT];
+#pragma unroll
+  for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      const int64_t col = col0 + 16 * j + c;
+      float x[8];
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) {
+        const int k = 32 * kd + 8 * q + s8;
+        x[s8] = (k < w && col < C) ? M[(int64_t)k * C + col] : 0.f;
+      }
+      ma[kd][j] = pieces8<3>(x);
+    }
+  const int64_t n_tiles = (N + 63) / 64;
+  float pre[PER][8];
+  auto fetch = [&](int64_t tile) {
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int idx = threadIdx.x + p * kThreads, row = idx / U, k = 8 * (idx % U);
+      const int64_t r = tile * 64 + row;
+      if (r < N) {
+        load8(v + r * ldv + k, k, w, vec_v, pre[p]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pre[p][i] = 0.f;
+      }
+    }
+  };
+  if ((int64_t)blockIdx.y < n_tiles) fetch(blockIdx.y);
+  for (int64_t tile = blockIdx.y; tile < n_tiles; tile += gridDim.y) {
+    __syncthreads();  // the previous tile's LDS reads are done
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int idx = threadIdx.x + p * kThreads;
+      const Pieces<PV> x = pieces8<PV>(pre[p]);
+#pragma unroll
+      for (int i = 0; i < PV; ++i) vs[i][deep_unit<U>(idx / U, idx % U)] = x.p[i];
+    }
+    __syncthreads();
+    if (tile + gridDim.y < n_tiles) fetch(tile + gridDim.y);
+    auto product = [&](auto full) {
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        floatx4 acc[CT];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) acc[j] = kZero4;
+#pragma unroll
+        for (int kd = 0; kd < KD; ++kd) {
+          Pieces<PV> b;
+#pragma unroll
+          for (int i = 0; i < PV; ++i) b.p[i] = vs[i][deep_unit<U>(16 * rt + c, 4 * kd + q)];
+          mfma_pieces(ma[kd], b, acc);
+        }
+        if constexpr (W == 32) {
+          // lanes c and c ^ 8 trade tile halves by one DPP rotate, so a store writes eight whole
+          // 128-byte row runs instead of sixteen 64-byte halves (1.25 -> 1.07 ms; no gain for wider vectors)
+          const bool lo = c < 8;
+#pragma unroll
+          for (int j = 0; j < CT; j += 2) {
+            floatx4 sw;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              sw[i] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(lo ? acc[j + 1][i] : acc[j][i]),
+                                                                 kDppRowRor8, 0xF, 0xF, false));
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              store4<full()>(out, tile * 64 + 16 * rt + 8 * h + (c & 7), col0 + 16 * (j + (c >> 3)) + 4 * q, N, C,
+                             (h == 0) == lo ? acc[j + h] : sw, vec_out);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < CT; ++j)
+            store4<full()>(out, tile * 64 + 16 * rt + c, col0 + 16 * j + 4 * q, N, C, acc[j], vec_out);
+        }
+        // a row tile's stores leave before the next one's products (2.93 -> 2.62 ms for 64 reals: interleaved,
+        // the held results take 232 registers and leave in bursts)
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (vec_out && tile * 64 + 64 <= N && col0 + 16 * CT <= C)
+      product(std::true_type{});
+    else
+      product(std::false_type{});
+  }
+}
+
+// Input gradient: tiles of 128 rows, each wave 32 rows over the workgroup's
+// chunks of the contraction (per_split of them; few rows are split over several
+// workgroups, their sums added in order by node_mix_dinput_reduce); its dmix rows come straight from memory into the lanes that
+// split them, M's chunk of KC columns is split once per workgroup into LDS
+// (two buffers, one barrier a chunk); running totals every 256 columns.
+template <int W>
+__global__ __launch_bounds__(kThreads, 2) void node_mix_dinput_deep(const float* __restrict__ dmix,
+                                                                    const float* __restrict__ M, int64_t N, int w,
+                                                                    int64_t C, float* __restrict__ dv, int64_t lddv,
+                                                                    int64_t per_split) {
+  constexpr int RT = 2, KC = W == 32 ? 64 : 32, KD = KC / 32, JW = W / 16, U = KC / 8;
+  constexpr int TOTAL_EVERY = 256 / KC;
+  constexpr int MP = (W * U + kThreads - 1) / kThreads;  // units of M's chunk a thread stages
+  __shared__ __align__(16) u32x4 ms[2][3][W * U];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
+  const int64_t row0 = (int64_t)blockIdx.x * (64 * RT) + 16 * RT * wv;
+  const int64_t all = (C + KC - 1) / KC, ch0 = (int64_t)blockIdx.y * per_split;
+  const int64_t n_chunks = ch0 + per_split < all ? ch0 + per_split : all;
+  dv += (int64_t)blockIdx.y * N * lddv;  // a split's partial sums (one split: the gradient itself)
+  float4 pd[RT][KD][2], pm[MP][2];
+  auto fetch = [&](int64_t ch) {
+    const int64_t c0 = ch * KC;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int64_t r = row0 + 16 * rt + c;
+#pragma unroll
+      for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int64_t col = c0 + 32 * kd + 8 * q + 4 * h;
+          pd[rt][kd][h] = (r < N && col < C) ? *reinterpret_cast<const float4*>(dmix + r * C + col)
+                                             : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < MP; ++p) {
+      const int idx = threadIdx.x + p * kThreads, row = idx / U;  // rows past w (and past W) load zeros
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int64_t col = c0 + 8 * (idx % U) + 4 * h;
+        pm[p][h] = (row < w && col < C) ? *reinterpret_cast<const float4*>(M + (int64_t)row * C + col)
+                                        : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
+  };
+  auto split8 = [](const float4 (&x)[2]) {
+    const float y[8] = {x[0].x, x[0].y, x[0].z, x[0].w, x[1].x, x[1].y, x[1].z, x[1].w};
+    return pieces8<3>(y);
+  };
+  floatx4 acc[JW][RT], tot[JW][RT];
+#pragma unroll
+  for (int j = 0; j < JW; ++j)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[j][rt] = tot[j][rt] = kZero4;
+  if (ch0 < n_chunks) fetch(ch0);
+  for (int64_t ch = ch0; ch < n_chunks; ++ch) {
+    auto& buf = ms[ch & 1];  // last read two chunks ago, before every wave's last barrier
+    Pieces<3> a[KD][RT];
+#pragma unroll
+    for (int p = 0; p < MP; ++p) {
+      const int idx = threadIdx.x + p * kThreads;
+      const Pieces<3> x = split8(pm[p]);
+      if (idx < W * U) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) buf[i][deep_unit<U>(idx / U, idx % U)] = x.p[i];
+      }
+    }
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) a[kd][rt] = split8(pd[rt][kd]);
+    if (ch + 1 < n_chunks) fetch(ch + 1);
+    __syncthreads();
+#pragma unroll
+    for (int kd = 0; kd < KD; ++kd)
+#pragma unroll
+      for (int j = 0; j < JW; ++j) {
+        Pieces<3> b;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) b.p[i] = buf[i][deep_unit<U>(16 * j + c, 4 * kd + q)];
+        mfma_pieces(a[kd], b, acc[j]);
+      }
+    if (ch % TOTAL_EVERY == TOTAL_EVERY - 1 || ch + 1 == n_chunks) {
+#pragma unroll
+      for (int j = 0; j < JW; ++j)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          tot[j][rt] += acc[j][rt];
+          acc[j][rt] = kZero4;
+        }
+    }
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int j = 0; j < JW; ++j) {
+      const int col = 16 * j + c;
+      if (col >= w) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t r = row0 + 16 * rt + 4 * q + i;
+        if (r < N) dv[r * lddv + col] = tot[j][rt][i];
+      }
+    }
+}
+
+// dv[r][k] = the sum of the splits' partial sums (rows of w reals), in order.
+__global__ __launch_bounds__(kThreads) void node_mix_dinput_reduce(const float* __restrict__ partial, int64_t N, int w,
+                                                                   int splits, float* __restrict__ dv, int64_t lddv) {
+  const int64_t e = (int64_t)blockIdx.x * kThreads + threadIdx.x, n = N * w;
+  if (e >= n) return;
+  float s = partial[e];
+  for (int y = 1; y < splits; ++y) s += partial[y * n + e];
+  dv[e / w * lddv + e % w] = s;
+}
+
+// Weight gradient: workgroup (x, y) owns 64 JT columns over rows [y rps,
+// min(N, (y + 1) rps)), wave wv the columns x 64 JT + 16 JT wv + JT c + j (so a
+// lane's tiles are consecutive columns: one load a row, no LDS), in chunks of
+// 32 rows; the chunk of v is split once per workgroup into LDS, transposed
+// (a thread splits eight rows of one column: one operand unit), two buffers,
+// one barrier a chunk.  One partial matrix a workgroup row.
+template <int W, typename V = float, typename DM = float>
+__global__ __launch_bounds__(kThreads, 2) void node_mix_dweight_deep(const V* __restrict__ v, int64_t ldv,
+                                                                     const DM* __restrict__ dmix, int64_t N, int w,
+                                                                     int64_t C, int64_t rps,
+                                                                     float* __restrict__ partial, int vec_p) {
+  constexpr int JT = DeepJT<W>, IW = W / 16, RC = 32, PV = sizeof(V) == 2 ? 1 : 3, PD = sizeof(DM) == 2 ? 1 : 3;
+  constexpr int UNITS = 4 * W, VQ = (UNITS + kThreads - 1) / kThreads;
+  __shared__ __align__(16) u32x4 vs[2][PV][UNITS];  // unit (octet o, column k) at o W + k
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, c = lane & 15, q = lane >> 4;
+  const int64_t col = (int64_t)blockIdx.x * (64 * JT) + 16 * JT * wv + JT * c;
+  const int64_t first = (int64_t)blockIdx.y * rps, last = first + rps < N ? first + rps : N;
+  float pv[VQ][8], pd[8][JT];
+  auto fetch = [&](int64_t r0) {
+#pragma unroll
+    for (int p = 0; p < VQ; ++p) {
+      const int idx = threadIdx.x + p * kThreads, k = idx % W, o = idx / W;
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) {
+        const int64_t r = r0 + 8 * o + s8;
+        float x = 0.f;
+        if (idx < UNITS && r < last && k < w) {
+          if constexpr (sizeof(V) == 2)
+            x = bf16_at(v + r * ldv + k);
+          else
+            x = v[r * ldv + k];
+        }
+        pv[p][s8] = x;
+      }
+    }
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) {
+      const int64_t r = r0 + 8 * q + s8;
+      const bool in = r < last && col < C;  // C is a multiple of 4, so a lane's columns are in or out together
+      const DM* src = dmix + r * C + col;
+      if constexpr (JT == 4) {
+        const float4 x = in ? load_dm4(src) : make_float4(0.f, 0.f, 0.f, 0.f);
+        pd[s8][0] = x.x, pd[s8][1] = x.y, pd[s8][2] = x.z, pd[s8][3] = x.w;
+      } else if constexpr (sizeof(DM) == 2) {
+        const uint32_t x = in ? *reinterpret_cast<const uint32_t*>(src) : 0u;
+        pd[s8][0] = bf16_lo(x), pd[s8][1] = bf16_hi(x);
+      } else {
+        const float2 x = in ? *reinterpret_cast<const float2*>(src) : make_float2(0.f, 0.f);
+        pd[s8][0] = x.x, pd[s8][1] = x.y;
+      }
+    }
+  };
+  floatx4 acc[IW][JT];
+#pragma unroll
+  for (int i = 0; i < IW; ++i)
+#pragma unroll
+    for (int j = 0; j < JT; ++j) acc[i][j] = kZero4;
+  if (first < last) fetch(first);
+  int cur = 0;
+  for (int64_t r0 = first; r0 < last; r0 += RC, cur ^= 1) {
+    auto& buf = vs[cur];  // last read two chunks ago, before every wave's last barrier
+#pragma unroll
+    for (int p = 0; p < VQ; ++p) {
+      const int idx = threadIdx.x + p * kThreads;
+      const Pieces<PV> x = pieces8<PV>(pv[p]);
+      if (idx < UNITS) {
+#pragma unroll
+        for (int i = 0; i < PV; ++i) buf[i][idx] = x.p[i];
+      }
+    }
+    Pieces<PD> b[JT];
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      float x[8];
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) x[s8] = pd[s8][j];
+      b[j] = pieces8<PD>(x);
+    }
+    if (r0 + RC < last) fetch(r0 + RC);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IW; ++i) {
+      Pieces<PV> a;
+#pragma unroll
+      for (int p = 0; p < PV; ++p) a.p[p] = buf[p][q * W + 16 * i + c];
+#pragma unroll
+      for (int order = 2; order >= 0; --order)
+#pragma unroll
+        for (int p = 0; p <= order; ++p) {
+          if (p >= PV || order - p >= PD) continue;
+#pragma unroll
+          for (int j = 0; j < JT; ++j) acc[i][j] = mfma_bf16(a.p[p], b[j].p[order - p], acc[i][j]);
+        }
+    }
+  }
+  if (col >= C) return;
+  float* out = partial + (int64_t)blockIdx.y * w * C;
+#pragma unroll
+  for (int i = 0; i < IW; ++i)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+      const int row = 16 * i + 4 * q + ii;
+      if (row >= w) continue;
+      float* dst = out + (int64_t)row * C + col;
+      if (vec_p && JT == 4) {
+        *reinterpret_cast<float4*>(dst) = make_float4(acc[i][0][ii], acc[i][1][ii], acc[i][JT - 2][ii], acc[i][JT - 1][ii]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < JT; ++j) dst[j] = acc[i][j][ii];
+      }
+    }
+}
+
 // dM[e] = sum over y = 0, 1, ..., count - 1 of partial[y stride][e], in that order.
 __global__ __launch_bounds__(kThreads) void node_mix_reduce_kernel(const float* __restrict__ partial, int64_t n,
                                                                    int64_t count, int64_t stride,
@@ -920,13 +1285,19 @@ int check_shapes(int64_t N, int64_t w, int64_t C) {
 
 int width_class(int64_t w) { return w <= 16 ? 16 : (w <= 32 ? 32 : (w <= 64 ? 64 : 128)); }
 
+// Whether vectors of w reals take the 32-deep kernels.
+bool deep(int64_t w) { return split_products() && w > 16; }
+
 // Column tile of the weight gradient's workgroups: 64 columns for vectors up to
 // 64 reals; above, 32 for the split kernel and 128 for the fp32 one.
-int64_t weight_tile(int64_t w) { return w <= 64 ? 64 : (split_products() ? 32 : 128); }
+int64_t weight_tile(int64_t w) {
+  if (deep(w)) return 64 * (w <= 64 ? DeepJT<64> : DeepJT<128>);
+  return w <= 64 ? 64 : 128;
+}
 
 // Partial matrices a workgroup row writes: four (one a wave) but for the fp32
 // kernel of vectors above 64 reals (one).
-int64_t weight_partials_per_split(int64_t w) { return (w <= 64 || split_products()) ? 4 : 1; }
+int64_t weight_partials_per_split(int64_t w) { return w <= 64 && !deep(w) ? 4 : 1; }
 
 // Row groups g of a grid of nx x g workgroups whose rows each workgroup loops
 // over in equal shares: about `want` workgroups in whole rounds of the
@@ -948,18 +1319,26 @@ const void* dweight_kernel(int64_t w) {
   const bool sp = split_products();
   switch (width_class(w)) {
     case 16: return sp ? (const void*)node_mix_dweight_split<16> : (const void*)node_mix_dweight_k_kernel<16>;
-    case 32: return sp ? (const void*)node_mix_dweight_split<32> : (const void*)node_mix_dweight_k_kernel<32>;
-    case 64: return sp ? (const void*)node_mix_dweight_split<64> : (const void*)node_mix_dweight_k_kernel<64>;
-    default: return sp ? (const void*)node_mix_dweight_split<128> : (const void*)node_mix_dweight_kernel<128>;
+    case 32: return sp ? (const void*)node_mix_dweight_deep<32> : (const void*)node_mix_dweight_k_kernel<32>;
+    case 64: return sp ? (const void*)node_mix_dweight_deep<64> : (const void*)node_mix_dweight_k_kernel<64>;
+    default: return sp ? (const void*)node_mix_dweight_deep<128> : (const void*)node_mix_dweight_kernel<128>;
   }
 }
+
+// Rows one accumulator of the 32-deep weight gradient sums at most (about): a
+// longer chain costs accuracy (the error of a sequential float sum grows with
+// its length), a shorter one partial matrices.  4,096 rows: 2.1e-6 relative
+// (2-norm) over 524,288 rows against 3.7e-6 for the 16-deep form's 10,900.
+constexpr int64_t kMaxChainRows = 4096;
 
 // The weight gradient's row splits: about 1024 workgroups in whole rounds, whole 64-row chunks per split.
 void weight_splits(int64_t N, int64_t w, int64_t C, int64_t max_splits, int64_t& splits, int64_t& rps) {
   const int64_t tile = weight_tile(w);
   const int64_t nx = (C + tile - 1) / tile > 0 ? (C + tile - 1) / tile : 1;
   const int64_t chunks = (N + 63) / 64;
-  int64_t s = round_groups(nx, 1024, resident_blocks(dweight_kernel(w), kThreads));
+  int64_t want = 1024;
+  if (deep(w)) want = std::max(want, nx * ((N + kMaxChainRows - 1) / kMaxChainRows));
+  int64_t s = round_groups(nx, want, resident_blocks(dweight_kernel(w), kThreads));
   if (s > chunks) s = chunks;
   if (s > max_splits) s = max_splits;
   if (s < 1) s = 1;
@@ -968,12 +1347,59 @@ void weight_splits(int64_t N, int64_t w, int64_t C, int64_t max_splits, int64_t&
   if (splits < 1) splits = 1;
 }
 
+const void* dinput_kernel(int64_t w) {
+  switch (width_class(w)) {
+    case 32: return (const void*)node_mix_dinput_deep<32>;
+    case 64: return (const void*)node_mix_dinput_deep<64>;
+    default: return (const void*)node_mix_dinput_deep<128>;
+  }
+}
+
+// Splits of the input gradient's contraction: a workgroup walks its chunks one
+// after the other, so a launch takes about (rounds of resident workgroups) x
+// (chunks a split + kSplitCost): the splits that make this least.  16 row tiles
+// (2,048 rows, w = 64, C = 5,440): 191 us whole, 38 us in 16 splits; from four
+// rounds of row tiles up the tail is small and the contraction stays whole.
+constexpr int64_t kMaxInputSplits = 16, kSplitCost = 6;
+
+void input_splits(int64_t N, int64_t w, int64_t C, int64_t& splits, int64_t& per_split) {
+  const int64_t kc = width_class(w) == 32 ? 64 : 32, chunks = (C + kc - 1) / kc, blocks = (N + 127) / 128;
+  const int64_t slots = resident_blocks(dinput_kernel(w), kThreads);
+  splits = 1;
+  if (slots > 0 && blocks < 4 * slots) {
+    int64_t best = 0;
+    for (int64_t s = 1; s <= kMaxInputSplits && 4 * s <= chunks; ++s) {
+      const int64_t cost = (blocks * s + slots - 1) / slots * ((chunks + s - 1) / s + (s > 1 ? kSplitCost : 0));
+      if (best == 0 || cost < best) best = cost, splits = s;
+    }
+  }
+  per_split = chunks > 0 ? (chunks + splits - 1) / splits : 1;
+  if (chunks > 0) splits = (chunks + per_split - 1) / per_split;
+}
+
+int launch_dinput(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C, int64_t splits,
+                  int64_t per_split, float* partial, float* dv, int64_t lddv, hipStream_t s) {
+  const dim3 grid((unsigned)((N + 127) / 128), (unsigned)splits), block(kThreads);
+  float* to = splits > 1 ? partial : dv;
+  const int64_t ld = splits > 1 ? w : lddv;
+  switch (width_class(w)) {
+    case 32: hipLaunchKernelGGL(node_mix_dinput_deep<32>, grid, block, 0, s, dmix, M, N, (int)w, C, to, ld, per_split); break;
+    case 64: hipLaunchKernelGGL(node_mix_dinput_deep<64>, grid, block, 0, s, dmix, M, N, (int)w, C, to, ld, per_split); break;
+    default: hipLaunchKernelGGL(node_mix_dinput_deep<128>, grid, block, 0, s, dmix, M, N, (int)w, C, to, ld, per_split); break;
+  }
+  const int rc = check_launch("node_mix_backward_input");
+  if (rc != GM_OK || splits == 1) return rc;
+  hipLaunchKernelGGL(node_mix_dinput_reduce, dim3((unsigned)((N * w + kThreads - 1) / kThreads)), block, 0, s, partial,
+                     N, (int)w, (int)splits, dv, lddv);
+  return check_launch("node_mix_backward_input (reduce)");
+}
+
 int launch_dweight(const float* v, int64_t ldv, const float* dmix, int64_t N, int64_t w, int64_t C, int64_t splits,
                    int64_t rps, float* partial, float* dM, hipStream_t stream) {
   const int64_t tile = weight_tile(w), nx = (C + tile - 1) / tile;
   if (N > 0 && nx > 0) {
     const dim3 grid((unsigned)nx, (unsigned)splits), block(kThreads);
-    const int vec = aligned(v, 16) && ldv % 4 == 0;
+    const int vec = aligned(v, 16) && ldv % 4 == 0, vec_p = aligned(partial, 16);
     const bool sp = split_products();
     switch (width_class(w)) {
       case 16:
@@ -981,15 +1407,15 @@ int launch_dweight(const float* v, int64_t ldv, const float* dmix, int64_t N, in
         else hipLaunchKernelGGL(node_mix_dweight_k_kernel<16>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
         break;
       case 32:
-        if (sp) hipLaunchKernelGGL(node_mix_dweight_split<32>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
+        if (sp) hipLaunchKernelGGL(node_mix_dweight_deep<32>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec_p);
         else hipLaunchKernelGGL(node_mix_dweight_k_kernel<32>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
         break;
       case 64:
-        if (sp) hipLaunchKernelGGL(node_mix_dweight_split<64>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
+        if (sp) hipLaunchKernelGGL(node_mix_dweight_deep<64>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec_p);
         else hipLaunchKernelGGL(node_mix_dweight_k_kernel<64>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
         break;
       default:
-        if (sp) hipLaunchKernelGGL(node_mix_dweight_split<128>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
+        if (sp) hipLaunchKernelGGL(node_mix_dweight_deep<128>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec_p);
         else hipLaunchKernelGGL(node_mix_dweight_kernel<128>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
         break;
     }
@@ -1054,14 +1480,14 @@ extern "C" int gm_node_mix_forward_f32(const float* v, int64_t ldv, const float*
   const int vec_out = gm::aligned(out, 16) && C % 4 == 0;
   const int W = gm::width_class(w);
   const bool sp = gm::split_products();
-  const int CT = sp ? (W == 128 ? gm::SplitCT<128> : gm::SplitCT<64>) : (W == 128 ? 2 : 4);
+  const int CT = sp ? (W == 16 ? gm::kSplitCT : (W == 128 ? gm::DeepCT<128> : gm::DeepCT<64>)) : (W == 128 ? 2 : 4);
   const int64_t nx = (C + 64 * CT - 1) / (64 * CT), n_tiles = (N + 63) / 64;
   const void* kernel = nullptr;
   switch (W) {
     case 16: kernel = sp ? (const void*)gm::node_mix_forward_split<16> : (const void*)gm::node_mix_forward_kernel<16, 4>; break;
-    case 32: kernel = sp ? (const void*)gm::node_mix_forward_split<32> : (const void*)gm::node_mix_forward_kernel<32, 4>; break;
-    case 64: kernel = sp ? (const void*)gm::node_mix_forward_split<64> : (const void*)gm::node_mix_forward_kernel<64, 4>; break;
-    default: kernel = sp ? (const void*)gm::node_mix_forward_split<128> : (const void*)gm::node_mix_forward_kernel<128, 2>; break;
+    case 32: kernel = sp ? (const void*)gm::node_mix_forward_deep<32> : (const void*)gm::node_mix_forward_kernel<32, 4>; break;
+    case 64: kernel = sp ? (const void*)gm::node_mix_forward_deep<64> : (const void*)gm::node_mix_forward_kernel<64, 4>; break;
+    default: kernel = sp ? (const void*)gm::node_mix_forward_deep<128> : (const void*)gm::node_mix_forward_kernel<128, 2>; break;
   }
   int64_t ny = gm::round_groups(nx, 2048, gm::resident_blocks(kernel, gm::kThreads));
   if (ny > n_tiles) ny = n_tiles;
@@ -1070,9 +1496,9 @@ extern "C" int gm_node_mix_forward_f32(const float* v, int64_t ldv, const float*
   if (sp) {
     switch (W) {
       case 16: hipLaunchKernelGGL((gm::node_mix_forward_split<16>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
-      case 32: hipLaunchKernelGGL((gm::node_mix_forward_split<32>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
-      case 64: hipLaunchKernelGGL((gm::node_mix_forward_split<64>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
-      default: hipLaunchKernelGGL((gm::node_mix_forward_split<128>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
+      case 32: hipLaunchKernelGGL((gm::node_mix_forward_deep<32>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
+      case 64: hipLaunchKernelGGL((gm::node_mix_forward_deep<64>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
+      default: hipLaunchKernelGGL((gm::node_mix_forward_deep<128>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
     }
     return gm::check_launch("node_mix_forward");
   }
@@ -1085,34 +1511,59 @@ extern "C" int gm_node_mix_forward_f32(const float* v, int64_t ldv, const float*
   return gm::check_launch("node_mix_forward");
 }
 
-extern "C" int gm_node_mix_backward_input_f32(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C,
-                                              float* dv, int64_t lddv, void* stream) {
-  int rc = gm::check_shapes(N, w, C);
+namespace gm {
+namespace {
+
+int backward_input(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C, float* partial, float* dv,
+                   int64_t lddv, hipStream_t s) {
+  const int rc = check_shapes(N, w, C);
   if (rc != GM_OK) return rc;
   if (N == 0) return GM_OK;
   GM_REQUIRE(dv && lddv >= w, "dv must be a device pointer with lddv >= w");
   GM_REQUIRE(C == 0 || (dmix && M), "dmix and M must be device pointers");
-  GM_REQUIRE(C % 4 == 0 && gm::aligned(dmix, 16) && gm::aligned(M, 16),
+  GM_REQUIRE(C % 4 == 0 && aligned(dmix, 16) && aligned(M, 16),
              "dmix and M must be 16-byte aligned with C a multiple of 4");
-  const hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)((N + 127) / 128)), block(gm::kThreads);
-  if (gm::split_products()) {
-    const dim3 grid128((unsigned)((N + 64 * gm::SplitRT<128> - 1) / (64 * gm::SplitRT<128>)));
-    switch (gm::width_class(w)) {
-      case 16: hipLaunchKernelGGL(gm::node_mix_dinput_split<16>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
-      case 32: hipLaunchKernelGGL(gm::node_mix_dinput_split<32>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
-      case 64: hipLaunchKernelGGL(gm::node_mix_dinput_split<64>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
-      default: hipLaunchKernelGGL(gm::node_mix_dinput_split<128>, grid128, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
+  if (deep(w)) {
+    int64_t splits = 1, per_split = 0;
+    if (partial != nullptr) {
+      input_splits(N, w, C, splits, per_split);
+    } else {
+      per_split = C;  // chunks are of 32 columns or more: every chunk
     }
-    return gm::check_launch("node_mix_backward_input");
+    return launch_dinput(dmix, M, N, w, C, splits, per_split, partial, dv, lddv, s);
   }
-  switch (gm::width_class(w)) {
-    case 16: hipLaunchKernelGGL(gm::node_mix_dinput_kernel<16>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
-    case 32: hipLaunchKernelGGL(gm::node_mix_dinput_kernel<32>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
-    case 64: hipLaunchKernelGGL(gm::node_mix_dinput_kernel<64>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
-    default: hipLaunchKernelGGL(gm::node_mix_dinput_kernel<128>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
+  const dim3 grid((unsigned)((N + 127) / 128)), block(kThreads);
+  if (split_products()) {
+    hipLaunchKernelGGL(node_mix_dinput_split<16>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv);
+    return check_launch("node_mix_backward_input");
   }
-  return gm::check_launch("node_mix_backward_input");
+  switch (width_class(w)) {
+    case 16: hipLaunchKernelGGL(node_mix_dinput_kernel<16>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
+    case 32: hipLaunchKernelGGL(node_mix_dinput_kernel<32>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
+    case 64: hipLaunchKernelGGL(node_mix_dinput_kernel<64>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
+    default: hipLaunchKernelGGL(node_mix_dinput_kernel<128>, grid, block, 0, s, dmix, M, N, (int)w, C, dv, lddv); break;
+  }
+  return check_launch("node_mix_backward_input");
+}
+
+}  // namespace
+}  // namespace gm
+
+extern "C" int gm_node_mix_backward_input_f32(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C,
+                                              float* dv, int64_t lddv, void* stream) {
+  return gm::backward_input(dmix, M, N, w, C, nullptr, dv, lddv, (hipStream_t)stream);
+}
+
+extern "C" int64_t gm_node_mix_input_partials(int64_t N, int64_t w, int64_t C) {
+  if (N <= 0 || w < 1 || w > 128 || C <= 0 || !gm::deep(w)) return 0;
+  int64_t splits = 1, per_split = 0;
+  gm::input_splits(N, w, C, splits, per_split);
+  return splits > 1 ? splits * N * w : 0;
+}
+
+extern "C" int gm_node_mix_backward_input_split_f32(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C,
+                                                    float* partial, float* dv, int64_t lddv, void* stream) {
+  return gm::backward_input(dmix, M, N, w, C, partial, dv, lddv, (hipStream_t)stream);
 }
 
 extern "C" int64_t gm_node_mix_weight_partials(int64_t N, int64_t w, int64_t C) {
@@ -1143,9 +1594,10 @@ extern "C" int gm_node_mix_backward_weight_noalloc_f32(const float* v, int64_t l
   GM_REQUIRE(N == 0 || (v && dmix && ldv >= w), "v (ldv >= w) and dmix must be device pointers");
   GM_REQUIRE(C % 4 == 0 && (N == 0 || gm::aligned(dmix, 16)), "dmix must be 16-byte aligned with C a multiple of 4");
   const int64_t per_split = gm::weight_partials_per_split(w) * w * C;
-  GM_REQUIRE(per_split <= gm::kScratchFloats,
+  const int64_t needed = (w <= 64 || gm::split_products() ? 4 : 1) * w * C;
+  GM_REQUIRE(needed <= gm::kScratchFloats,
              "w * C is too large for the no-allocation weight gradient: its partials need " +
-                 std::to_string(per_split) + " floats a row split, the scratch holds " +
+                 std::to_string(needed) + " floats a row split, the scratch holds " +
                  std::to_string(gm::kScratchFloats));
   const hipStream_t s = (hipStream_t)stream;
   std::lock_guard<std::mutex> lock(gm::scratch_mutex);
@@ -1189,18 +1641,19 @@ extern "C" int gm_node_mix_forward_bf16(const uint16_t* v, int64_t ldv, const fl
   const int vec_v = gm::aligned(v, 8) && ldv % 4 == 0;
   const int vec_out = gm::aligned(out, 16) && C % 4 == 0;
   const int W = gm::width_class(w);
-  const int64_t nx = (C + 127) / 128, n_tiles = (N + 63) / 64;
+  const int CT = W == 16 ? gm::kSplitCT : gm::DeepCT<64>;
+  const int64_t nx = (C + 64 * CT - 1) / (64 * CT), n_tiles = (N + 63) / 64;
   const void* kernel = W == 16 ? (const void*)gm::node_mix_forward_split<16, uint16_t>
-                       : W == 32 ? (const void*)gm::node_mix_forward_split<32, uint16_t>
-                                 : (const void*)gm::node_mix_forward_split<64, uint16_t>;
+                       : W == 32 ? (const void*)gm::node_mix_forward_deep<32, uint16_t>
+                                 : (const void*)gm::node_mix_forward_deep<64, uint16_t>;
   int64_t ny = gm::round_groups(nx, 2048, gm::resident_blocks(kernel, gm::kThreads));
   if (ny > n_tiles) ny = n_tiles;
   if (ny > 65535) ny = 65535;
   const dim3 grid((unsigned)nx, (unsigned)ny), block(gm::kThreads);
   switch (W) {
     case 16: hipLaunchKernelGGL((gm::node_mix_forward_split<16, uint16_t>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
-    case 32: hipLaunchKernelGGL((gm::node_mix_forward_split<32, uint16_t>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
-    default: hipLaunchKernelGGL((gm::node_mix_forward_split<64, uint16_t>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
+    case 32: hipLaunchKernelGGL((gm::node_mix_forward_deep<32, uint16_t>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
+    default: hipLaunchKernelGGL((gm::node_mix_forward_deep<64, uint16_t>), grid, block, 0, s, v, ldv, M, N, (int)w, C, out, vec_v, vec_out); break;
   }
   return gm::check_launch("node_mix_forward (bfloat16 vectors)");
 }
@@ -1219,14 +1672,14 @@ int split_dweight(const V* v, int64_t ldv, const DM* dmix, int64_t N, int64_t w,
   const int64_t tile = weight_tile(w), nx = (C + tile - 1) / tile;
   if (N > 0 && nx > 0) {
     const dim3 grid((unsigned)nx, (unsigned)splits), block(kThreads);
-    const int vec = aligned(v, sizeof(V) == 2 ? 8 : 16) && ldv % 4 == 0;
+    const int vec = aligned(v, sizeof(V) == 2 ? 8 : 16) && ldv % 4 == 0, vec_p = aligned(partial, 16);
     switch (width_class(w)) {
       case 16: hipLaunchKernelGGL((node_mix_dweight_split<16, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec); break;
-      case 32: hipLaunchKernelGGL((node_mix_dweight_split<32, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec); break;
-      case 64: hipLaunchKernelGGL((node_mix_dweight_split<64, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec); break;
+      case 32: hipLaunchKernelGGL((node_mix_dweight_deep<32, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec_p); break;
+      case 64: hipLaunchKernelGGL((node_mix_dweight_deep<64, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec_p); break;
       default:
         if constexpr (sizeof(V) == 4)
-          hipLaunchKernelGGL((node_mix_dweight_split<128, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
+          hipLaunchKernelGGL((node_mix_dweight_deep<128, V, DM>), grid, block, 0, s, v, ldv, dmix, N, (int)w, C, rps, partial, vec_p);
         break;
     }
     const int rc = check_launch("node_mix_backward_weight");

@@ -59,6 +59,8 @@ SIGNATURES_F32 = {
     "gm_radial_trunk_backward_bf16": (ctypes.c_int, [_P] * 5 + [_I] * 4 + [_D, _P, _P, _P]),
     "gm_node_mix_forward_f32": (ctypes.c_int, [_P, _I, _P, _I, _I, _I, _P, _P]),
     "gm_node_mix_backward_input_f32": (ctypes.c_int, [_P, _P, _I, _I, _I, _P, _I, _P]),
+    "gm_node_mix_backward_input_split_f32": (ctypes.c_int, [_P, _P, _I, _I, _I, _P, _P, _I, _P]),
+    "gm_node_mix_input_partials": (ctypes.c_int64, [_I, _I, _I]),
     "gm_node_mix_weight_partials": (ctypes.c_int64, [_I, _I, _I]),
     "gm_node_mix_backward_weight_f32": (ctypes.c_int, [_P, _I, _P, _I, _I, _I, _P, _P, _P]),
     "gm_node_mix_backward_weight_noalloc_f32": (ctypes.c_int, [_P, _I, _P, _I, _I, _I, _P, _P]),
@@ -718,7 +720,10 @@ def node_mix_backward_input(dmix: Tensor, m: Tensor, dv: Tensor) -> None:
     w, C = m.shape
     _require_device(dmix, m)
     _check(dmix.shape == (N, C) and dv.shape[1] == w, "dmix must be (N, C) for m (w, C) and dv (N, w)")
-    _call("gm_node_mix_backward_input_f32", _ptr(dmix), _ptr(m), N, w, C, _ptr(dv), max(lddv, w), _stream(dv.device))
+    floats = int(library().gm_node_mix_input_partials(N, w, C))  # few rows: the contraction in splits
+    partial = torch.empty(floats, dtype=torch.float32, device=dv.device) if floats else None
+    _call("gm_node_mix_backward_input_split_f32", _ptr(dmix), _ptr(m), N, w, C, _ptr(partial), _ptr(dv), max(lddv, w),
+          _stream(dv.device))
 
 
 def node_mix_backward_weight(v: Tensor, dmix: Tensor) -> Tensor:

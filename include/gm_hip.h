@@ -612,6 +612,13 @@ int gm_node_mix_forward_f32(const float* v, int64_t ldv, const float* M, int64_t
  * aligned.  The reference takes it from autograd through the einsum. */
 int gm_node_mix_backward_input_f32(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C, float* dv,
                                    int64_t lddv, void* stream);
+/* The same with a workspace `partial` of gm_node_mix_input_partials(N, w, C)
+ * floats (it may be null, and is not read, where that is 0): few rows have
+ * their contraction split over several workgroups, the splits' sums added in
+ * a fixed order. */
+int gm_node_mix_backward_input_split_f32(const float* dmix, const float* M, int64_t N, int64_t w, int64_t C,
+                                         float* partial, float* dv, int64_t lddv, void* stream);
+int64_t gm_node_mix_input_partials(int64_t N, int64_t w, int64_t C);
 
 /* Its weight gradient dM (w, C) = v^T dmix, summed over row ranges into
  * `partial` (a workspace of gm_node_mix_weight_partials(N, w, C) floats) and

@@ -60,6 +60,54 @@ def test_node_mix_kernels_match_float64_products(case, cuda):
     _close(dm, v.T @ dmix.double(), "dM", 5e-6)
 
 
+# (N, row width, offset, w, C) at the edges of the 32-deep kernels' tiles: one row, the first and last width of
+# each class, columns past the last whole tile, a contraction split over several workgroups (few rows, many
+# columns) and not split, several chunks of rows for the weight gradient's splits
+DEEP = [
+    (1, 20, 2, 17, 4),
+    (33, 32, 0, 32, 260),
+    (128, 40, 3, 33, 1028),
+    (2048, 64, 0, 64, 5440),
+    (4100, 130, 1, 65, 388),
+    (130, 128, 0, 128, 2308),
+    (9000, 40, 4, 24, 132),
+]
+
+
+@pytest.mark.parametrize("case", DEEP)
+@pytest.mark.parametrize("rows16", [False, True])
+def test_node_mix_32_deep_kernels_match_float64_products(case, rows16, cuda):
+    """Float32 and bfloat16 node vectors (bfloat16: up to 64 reals) against
+    float64 products of the same rounded values.  The bound on each product is
+    the split's (2^-22 of the sum of |products|) plus a float32 chain's: its
+    length times 2^-24 of the sum of |products| (the first-order bound of a
+    sequential sum), so taken entry by entry."""
+    N, D, off, w, C = case
+    if rows16 and w > 64:
+        pytest.skip("bfloat16 node vectors are at most 64 reals wide")
+    print(f"node mix 32-deep N={N} w={w} C={C} bf16={rows16}", flush=True)
+    rows, m, dmix = _inputs(N, D, off, w, C, 17 * N + w + C)
+    rows = rows.bfloat16() if rows16 else rows
+    v = rows[:, off:off + w].double()
+    rd, md, dd = rows.to(cuda), m.to(cuda), dmix.to(cuda)
+
+    def check(got, a, b, chain, name):
+        want, size = a @ b, a.abs() @ b.abs()
+        ratio = ((got.double().cpu() - want).abs() / (size * (2.0 ** -22 + chain * 2.0 ** -24) + 1e-30)).max()
+        assert float(ratio) <= 1.0, f"{name}: {float(ratio):.2f} of the bound"
+
+    check(_native.node_mix_forward(rd[:, off:off + w], md), v, m.double(), 6 * 4, "mix")
+    dx = torch.full((N, D), 7.0, device=cuda)
+    _native.node_mix_backward_input(dd, md, dx[:, off:off + w])
+    check(dx[:, off:off + w], dmix.double(), m.double().T, 6 * 8 + C // 256 + 16, "dv")
+    assert bool((torch.cat([dx[:, :off], dx[:, off + w:]], dim=1) == 7.0).all()), "wrote outside its columns"
+    whole = torch.full((N, D), 7.0, device=cuda)  # the entry point without a workspace never splits
+    assert _native.library().gm_node_mix_backward_input_f32(
+        dd.data_ptr(), md.data_ptr(), N, w, C, whole[:, off:].data_ptr(), D, torch.cuda.current_stream().cuda_stream) == 0
+    check(whole[:, off:off + w], dmix.double(), m.double().T, 6 * 8 + C // 256 + 16, "dv (whole)")
+    check(_native.node_mix_backward_weight(rd[:, off:off + w], dd), v.T, dmix.double(), 6 * 128 + N // 4096 + 64, "dM")
+
+
 def test_node_mix_backward_weight_is_deterministic(cuda):
     rows, m, dmix = _inputs(4096, 64, 0, 64, 1088, 3)
     v, dd = rows.to(cuda), dmix.to(cuda)
