@@ -57,6 +57,7 @@ SIGNATURES_F32 = {
     "gm_radial_trunk_partials": (ctypes.c_int64, [_I]),
     "gm_radial_trunk_forward_bf16": (ctypes.c_int, [_P] * 4 + [_I] * 4 + [_D, _P, _P]),
     "gm_radial_trunk_backward_bf16": (ctypes.c_int, [_P] * 5 + [_I] * 4 + [_D, _P, _P, _P]),
+    "gm_signed_gather_f32": (ctypes.c_int, [_P, _I, _P, _I, _I, _P, _P]),
     "gm_node_mix_forward_f32": (ctypes.c_int, [_P, _I, _P, _I, _I, _I, _P, _P]),
     "gm_node_mix_backward_input_f32": (ctypes.c_int, [_P, _P, _I, _I, _I, _P, _I, _P]),
     "gm_node_mix_backward_input_split_f32": (ctypes.c_int, [_P, _P, _I, _I, _I, _P, _P, _I, _P]),
@@ -698,6 +699,17 @@ def _column_view(v: Tensor) -> tuple[int, int]:
            "node vectors must be a 2-D float32 or bfloat16 tensor on the GPU")
     _check(v.stride(1) == 1 or v.shape[1] == 1, "node vectors must have contiguous columns")
     return v.shape[0], (v.stride(0) if v.shape[0] > 1 else v.shape[1])
+
+
+def signed_gather(sources: Any, codes: Tensor) -> Tensor:
+    """``(n,)`` sums of the entries ``codes (uses, n)`` names among ``sources``
+    (float32, contiguous, None for zeros; ``gm_signed_gather_f32``)."""
+    uses, n = codes.shape
+    out = torch.empty(n, dtype=torch.float32, device=codes.device)
+    pointers = (_P * len(sources))(*[_ptr(t) for t in sources])
+    _call("gm_signed_gather_f32", pointers, len(sources), codes.data_ptr(), uses, n, out.data_ptr(),
+          _stream(codes.device))
+    return out
 
 
 def node_mix_forward(v: Tensor, m: Tensor) -> Tensor:

@@ -1,0 +1,126 @@
+"""A layer's parameters in the forms its kernels read, in one launch each way.
+
+The layers' kernels take block matrices, mixing matrices and stacked trunks
+whose every entry is one parameter entry, possibly negated, or zero (the
+reference concatenates and stacks them per head and block on every call,
+nn/attention.py:653-669, nn/kernels.py:506-546).  :func:`assembled` runs such a
+construction once on the parameters' positions in place of their values, keeps
+where every entry comes from, and from then on fills every form with one
+``gm_signed_gather_f32`` launch; the gradient is the transposed gather, each
+parameter entry's uses added in a fixed order.  The numbers are the
+construction's own, bit for bit (moves and sign changes only).
+
+Parameters the kernel does not take -- CPU tensors, other types, parameters on
+several devices or not contiguous -- go through the construction itself.
+"""
+
+from __future__ import annotations
+
+import itertools
+from collections.abc import Callable, Sequence
+from typing import Any
+
+import torch
+from torch import Tensor
+
+from gm_attention_amd import _native
+
+MAX_SOURCES = 256  # tensors a launch reads
+MAX_USES = 16  # uses of one parameter entry the gradient's padded table holds
+_ALIGN = 64  # entries a form starts at a multiple of (256 bytes: whole cache lines)
+
+
+def _starts(sizes: Sequence[int], align: int) -> list[int]:
+    """Starts of consecutive ranges of ``sizes``, each rounded up to ``align``, then the total."""
+    return list(itertools.accumulate((-(-n // align) * align for n in sizes), initial=0))
+
+
+class Plan:
+    """Where every entry of a construction's forms comes from, found on the
+    parameters' device."""
+
+    def __init__(self, shapes: tuple[torch.Size, ...], build: Callable[[list[Tensor]], list[Tensor]],
+                 device: torch.device) -> None:
+        self.shapes = shapes
+        sizes = [s.numel() for s in shapes]
+        self.in_starts = _starts(sizes, 4)  # a gradient starts on 16 bytes
+        at = torch.arange(1, self.in_starts[-1] + 1, dtype=torch.float64, device=device)
+        with torch.no_grad():
+            forms = build([at[a:a + n].view(s) for a, n, s in zip(self.in_starts, sizes, shapes)])
+        self.form_shapes = [m.shape for m in forms]
+        self.out_starts = _starts([m.numel() for m in forms], _ALIGN)
+        flat = torch.zeros(self.out_starts[-1], dtype=torch.float64, device=device)
+        for a, m in zip(self.out_starts, forms):
+            flat[a:a + m.numel()] = m.reshape(-1)
+        position = flat.abs().long() - 1  # -1: zero
+        self._used = (position, flat < 0)
+        self.codes = torch.where(position < 0, -1, self._code(self.in_starts, position, flat < 0)).reshape(1, -1)
+        counts = torch.bincount(position.clamp_min(-1) + 1, minlength=2)[1:]
+        self.most = int(counts.max())  # uses of one parameter entry
+        self.back: Tensor | None = None
+
+    @staticmethod
+    def _code(starts: list[int], position: Tensor, negative: Tensor) -> Tensor:
+        edges = torch.tensor(starts[:-1], dtype=torch.int64, device=position.device)
+        tensor = torch.searchsorted(edges, position, right=True) - 1
+        # an empty tensor shares its start with the next one: searchsorted takes the last of them, which holds it
+        offset = position - edges[tensor.clamp_min(0)]
+        return (tensor << 40) | (offset << 1) | negative.long()
+
+    def gradient_codes(self) -> Tensor:
+        """``(uses, parameter entries)``: entry p's j-th use among the forms' entries."""
+        if self.back is None:
+            position, negative = self._used
+            used = torch.nonzero(position >= 0).squeeze(1)
+            at, order = torch.sort(position[used], stable=True)
+            used = used[order]
+            rank = torch.arange(at.numel(), device=at.device) - torch.searchsorted(at, at)
+            table = torch.full((max(self.most, 1), self.in_starts[-1]), -1, dtype=torch.int64, device=at.device)
+            table[rank, at] = self._code(self.out_starts, used, negative[used])
+            self.back = table
+            self._used = None
+        return self.back
+
+
+class _Assemble(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx: Any, plan: Plan, *params: Tensor) -> tuple:
+        ctx.plan = plan
+        out = _native.signed_gather(params, plan.codes)
+        return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.out_starts, plan.form_shapes))
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx: Any, *grads: Tensor | None) -> tuple:
+        plan = ctx.plan
+        held = [None if g is None else g.to(torch.float32).contiguous() for g in grads]
+        flat = _native.signed_gather(held, plan.gradient_codes())
+        return (None, *(flat[a:a + s.numel()].view(s) if need else None
+                        for a, s, need in zip(plan.in_starts, plan.shapes, ctx.needs_input_grad[1:])))
+
+
+def takes(params: Sequence[Tensor]) -> bool:
+    """Whether :func:`assembled` fills the forms of ``params`` in one launch."""
+    if not 0 < len(params) <= MAX_SOURCES:
+        return False
+    device = params[0].device
+    return device.type == "cuda" and all(p.dtype == torch.float32 and p.device == device and p.is_contiguous()
+                                         for p in params)
+
+
+def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[list[Tensor]], list[Tensor]]) -> list:
+    """``build(params)``, a list of forms whose every entry is an entry of
+    ``params``, negated or not, or zero.  The plan is kept on ``owner`` under
+    ``name`` (which also names whatever else ``build`` depends on) for the
+    parameters' shapes and device."""
+    if not takes(params):
+        return build(list(params))
+    shapes = tuple(p.shape for p in params)
+    key = ("_assembly", name, str(params[0].device))
+    plan = owner.__dict__.get(key)
+    if plan is None or plan.shapes != shapes:
+        plan = Plan(shapes, build, params[0].device)
+        owner.__dict__[key] = plan
+    if plan.most > MAX_USES:
+        return build(list(params))
+    return list(_Assemble.apply(plan, *params))

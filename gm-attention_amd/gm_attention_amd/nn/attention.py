@@ -37,9 +37,11 @@ import torch.utils.checkpoint
 from torch import Tensor, nn
 
 from gm_attention_amd.discretization.discretization import SphericalDiscretization
-from gm_attention_amd.nn import fused_attention, fused_factored, kernels, radial
+from gm_attention_amd.nn import assembly, fused_attention, fused_factored, kernels, radial
 from gm_attention_amd.nn.kernels import SO2SteerableKernel
-from gm_attention_amd.nn.linear import FlatLinear, SO2Linear, apply_linear, block_matrix, flat_bias, weights_matrix
+from gm_attention_amd.nn.linear import (
+    FlatLinear, SO2Linear, apply_linear, block_matrix, flat_bias, linear_parameters, matrix_and_bias, weights_matrix,
+)
 from gm_attention_amd.representations.field_type import SO2FeatureField, SO2FieldType
 
 REMATERIALIZE_CHUNKS = os.environ.get("GM_CHUNK_REMATERIALIZE", "1") != "0"
@@ -214,6 +216,75 @@ def _stacked_flat(linears: Sequence[SO2Linear], field_type_out: SO2FieldType, ro
     return FlatLinear.apply(rows, m, flat_bias(bias, field_type_out))
 
 
+class _LayerForms:
+    """The batched layer's parameters as its kernels read them: the stacked
+    query and key maps and the output projection on flat rows (matrix, bias or
+    None), every head's node mixes (one matrix per input frequency) and, where
+    the fused trunk serves, the heads' stacked trunks -- one launch for all of
+    them (:mod:`assembly`)."""
+
+    def __init__(self, mhsa: SO2MHSA, values: list[SO2SteerableKernel], layout: fused_factored.HeadsLayout,
+                 trunk: bool) -> None:
+        heads = [cast(SO2Attention, h) for h in mhsa.heads]
+        maps = [[h.query for h in heads], [h.key for h in heads]]
+        proj = mhsa.output_projection
+        counts, params = [], []
+
+        def add(group: Sequence[Tensor]) -> None:
+            counts.append(len(group))
+            params.extend(group)
+
+        for lins in maps:
+            for lin in lins:
+                add(linear_parameters(lin))
+        add(linear_parameters(proj))
+        readouts = [k.readout_parameters() for k in values]
+        for r in readouts:
+            add([p for p in r if p is not None])
+        if trunk:
+            for k in values:
+                add(radial.trunk_parameters(k))
+
+        def build(ps: list[Tensor]) -> list[Tensor]:
+            groups = iter([ps[sum(counts[:i]):sum(counts[:i + 1])] for i in range(len(counts))])
+            forms = []
+            for lins in maps:
+                forms += _stacked_matrix(lins, mhsa.field_type_in, [next(groups) for _ in lins])
+            m, *bias = matrix_and_bias(proj, next(groups))
+            forms += [m.index_select(0, _heads_permutation(mhsa, m.device)), *bias]
+            given = []
+            for r in readouts:
+                it = iter(next(groups))
+                given.append([None if p is None else next(it) for p in r])
+            forms += fused_factored.mixing_forms(values, layout, given)
+            if trunk:
+                forms += radial.stacked_forms([next(groups) for _ in values])
+            return forms
+
+        self.served = assembly.takes(params)
+        if not self.served:
+            return
+        forms = iter(assembly.assembled(mhsa, f"layer {layout.split} {trunk}", params, build))
+
+        def pair(lin: SO2Linear) -> tuple[Tensor, Tensor | None]:
+            return next(forms), next(forms) if lin.has_bias else None
+
+        self.query, self.key, self.projection = pair(heads[0].query), pair(heads[0].key), pair(proj)
+        self.mixing = [next(forms) for _ in layout.hp.groups]
+        self.trunk = list(forms)
+
+
+def _stacked_matrix(linears: Sequence[SO2Linear], field_type_out: SO2FieldType,
+                    params: Sequence[Sequence[Tensor]]) -> list[Tensor]:
+    """The heads' stacked intertwiner on flat rows and its flat bias (where they
+    have one) from each head's parameters in ``linear_parameters`` order."""
+    lin = linears[0]
+    n = len(lin.common_frequencies)
+    weights = {str(f): torch.cat([p[i] for p in params], dim=0) for i, f in enumerate(lin.common_frequencies)}
+    m = weights_matrix(lin.field_type_in, field_type_out, lin.common_frequencies, weights)
+    return [m, flat_bias(torch.cat([p[n] for p in params]), field_type_out)] if lin.has_bias else [m]
+
+
 def _heads_permutation(mhsa: SO2MHSA, device: torch.device) -> Tensor:
     """For column ``head * d + c`` of the heads' outputs ``(N, H, d)`` (each in the
     per-head flat layout), its column in the direct sum's flat layout."""
@@ -259,21 +330,32 @@ def _attend_batched_flat(mhsa: SO2MHSA, x: SO2FeatureField, edges) -> Tensor | N
     rows = x._rows()
     if rows.ndim != 2:
         return None
+    compute = torch.float32 if x.dtype == torch.bfloat16 else x.dtype
+    fused_trunk = radial.eligible(values, compute, x.device)
+    layout = fused_factored.heads_layout(values, compute)
+    forms = _LayerForms(mhsa, values, layout, fused_trunk)
+    proj = mhsa.output_projection
     with torch.profiler.record_function("gm::attention/attend"):
-        queries = _stacked_flat([h.query for h in heads], mhsa.field_type_in, rows)
-        keys = _stacked_flat([h.key for h in heads], mhsa.field_type_in, rows)
+        if forms.served:
+            queries, keys = FlatLinear.apply(rows, *forms.query), FlatLinear.apply(rows, *forms.key)
+        else:
+            queries = _stacked_flat([h.query for h in heads], mhsa.field_type_in, rows)
+            keys = _stacked_flat([h.key for h in heads], mhsa.field_type_in, rows)
         alpha = fused_attention.softmax(mhsa, queries, keys, edges)  # (n_edges, n_heads)
         groups = fused_factored.groups_for(edges, edges.source_index)
-        compute = torch.float32 if x.dtype == torch.bfloat16 else x.dtype
-        if radial.eligible(values, compute, x.device):
-            h, trunk = None, functools.partial(radial.trunk_hidden_heads, values)
+        if fused_trunk:
+            h, trunk = None, functools.partial(radial.trunk_hidden_heads, values,
+                                               forms=forms.trunk if forms.served else None)
         else:
             h, trunk = torch.stack([k._trunk_hidden(edges.distances) for k in values]), None
-        out = fused_factored.forward_aggregated_heads(values, x, edges, alpha, h, groups, trunk)  # (N, H, d)
-    proj = mhsa.output_projection
-    m = block_matrix(proj).index_select(0, _heads_permutation(mhsa, rows.device))
-    return FlatLinear.apply(out.reshape(out.shape[0], -1), m,
-                            flat_bias(proj.bias if proj.has_bias else None, proj.field_type_out))
+        out = fused_factored.forward_aggregated_heads(values, x, edges, alpha, h, groups, trunk,
+                                                      forms.mixing if forms.served else None)  # (N, H, d)
+    if forms.served:
+        m, bias = forms.projection
+    else:
+        m = block_matrix(proj).index_select(0, _heads_permutation(mhsa, rows.device))
+        bias = flat_bias(proj.bias if proj.has_bias else None, proj.field_type_out)
+    return FlatLinear.apply(out.reshape(out.shape[0], -1), m, bias)
 
 
 def _attend_batched(mhsa: SO2MHSA, x: SO2FeatureField, edges) -> dict[int, Tensor]:

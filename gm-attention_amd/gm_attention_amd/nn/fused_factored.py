@@ -32,6 +32,7 @@ import torch
 from torch import Tensor
 
 from gm_attention_amd import _native
+from gm_attention_amd.nn import assembly
 from gm_attention_amd.representations.field_type import SO2FeatureField, SO2FieldType
 
 MAX_K, MAX_OUT, MAX_BM, MAX_C, DESC = 20, 128, 32, 320, 8
@@ -789,6 +790,15 @@ def heads_mixing(kernels: list[Any], hp: HeadsPlan, split: int = 1) -> list[Tens
     kernels, differentiable) rather than a per-head, per-block build.  With
     ``split > 1``, ``hp`` is the shares' plan and the columns run over
     ``H * split`` shares."""
+    readouts = [k.readout_parameters() for k in kernels]
+    params = [p for r in readouts for p in r if p is not None]
+    if assembly.takes(params):
+        def build(ps: list[Tensor]) -> list[Tensor]:
+            it = iter(ps)
+            return _heads_mixing_from(kernels, hp, [[None if p is None else next(it) for p in r] for r in readouts],
+                                      split)
+
+        return assembly.assembled(kernels[0], f"mixing {len(kernels)} {split}", params, build)
     plan = _mixing_maps(kernels, hp, split)
     flat = torch.cat([p.reshape(-1) for k in kernels for p in k.readout_parameters() if p is not None])
     return list(_SignedGather.apply(flat, plan))
@@ -814,6 +824,37 @@ def heads_mixes(x: SO2FeatureField, hp: HeadsPlan, mats: list[Tensor]) -> list[T
     vecs = node_vectors(x, hp)
     with torch.profiler.record_function("gm::kernel/node_products"):
         return [v @ m.to(v.dtype) for v, m in zip(vecs, mats, strict=True)]
+
+
+@dataclass(frozen=True)
+class HeadsLayout:
+    """How :func:`forward_aggregated_heads` runs a layer's heads: the plan of one
+    share (``split`` shares a head; 1 and ``grouped`` False for the kernels
+    that are not grouped), the phase orders of the grouped streams."""
+
+    hp: HeadsPlan
+    split: int
+    grouped: bool
+    pa: int
+    pt: int
+
+
+def heads_layout(kernels: list[Any], dtype: torch.dtype, K: int | None = None) -> HeadsLayout:
+    """The layout of the heads' value kernels for trunk features of ``dtype`` (K - 1 of them)."""
+    if K is None:
+        first = kernels[0]
+        K = (first.complex_head if first.complex_head is not None else first.real_head).in_features + 1
+    split = head_split(kernels[0], K) if dtype == torch.float32 else 0
+    hp = heads_plan(sub_head(kernels[0], max(split, 1)))
+    ok, pa, pt = grouped_eligible(hp, dtype, K)
+    if ok and split:
+        return HeadsLayout(hp, split, True, pa, pt)
+    return HeadsLayout(heads_plan(kernels[0]), 1, False, pa, pt)
+
+
+def mixing_forms(kernels: list[Any], layout: HeadsLayout, params: list[list[Tensor | None]]) -> list[Tensor]:
+    """:func:`heads_mixing`'s matrices for ``layout`` from the heads' readout parameters or stand-ins."""
+    return _heads_mixing_from(kernels, layout.hp, params, layout.split)
 
 
 class FactoredHeads(torch.autograd.Function):
@@ -1130,8 +1171,11 @@ def head_split(kernel: Any, K: int) -> int:
 
 
 def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any, alpha: Tensor, h: Tensor | None,
-                             groups: tuple[Tensor, Tensor, Tensor], trunk=None) -> Tensor:
-    """Every head's ``forward_factored_aggregated`` at once: ``(N, H, d_out)``.
+                             groups: tuple[Tensor, Tensor, Tensor], trunk=None,
+                             mats: list[Tensor] | None = None) -> Tensor:
+    """Every head's ``forward_factored_aggregated`` at once: ``(N, H, d_out)``
+    (``mats``: the heads' mixing matrices for their :func:`heads_layout`, formed
+    here when not given).
 
     ``h`` is every head's trunk features in edge order; alternatively
     ``trunk(rho, dtype)`` computes them from ``rho = d / cutoff`` in whatever
@@ -1143,13 +1187,14 @@ def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any,
     K = (h.shape[2] if h is not None else kernels[0].complex_head.in_features) + 1
     # bfloat16 rows: the node mixes read them as they are, everything after runs in float32
     dtype = h.dtype if h is not None else (torch.float32 if x.dtype == torch.bfloat16 else x.dtype)
-    split = head_split(kernels[0], K) if dtype == torch.float32 else 0
-    hp = heads_plan(sub_head(kernels[0], max(split, 1)))
-    ok, pa, pt = grouped_eligible(hp, dtype, K)
-    if ok and split:
+    layout = heads_layout(kernels, dtype, K)
+    hp, split, pa, pt = layout.hp, layout.split, layout.pa, layout.pt
+    if mats is None:
+        mats = heads_mixing(kernels, hp, split)
+    mixes = heads_mixes(x, hp, mats)
+    if layout.grouped:
         p = hp.plan
         unit = sub_head(kernels[0], split)
-        mixes = heads_mixes(x, hp, heads_mixing(kernels, hp, split))
         order, group_ptr, group_source = groups
         st = grouped_streams(edges, order, kernels[0].radial_basis.cutoff, pa, pt, dtype)
         fused = (FUSED_TRUNK and split == 1 and len(kernels) <= 8 and trunk is not None
@@ -1183,7 +1228,7 @@ def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any,
         return out.reshape(n, -1).index_select(1, cols).reshape(n, len(kernels), -1)
     if h is None:
         h = trunk((edges.distances / kernels[0].radial_basis.cutoff).to(dtype).contiguous())
-    return _forward_aggregated_heads_seg(kernels, x, edges, alpha, h, groups)
+    return _forward_aggregated_heads_seg(kernels, x, edges, alpha, h, groups, mixes)
 
 
 def forward_aggregated_shares(kernel: Any, x: SO2FeatureField, edges: Any, weights: Tensor,
@@ -1220,11 +1265,10 @@ def _heads_desc(kernel: Any, hp: HeadsPlan, device: torch.device) -> Tensor:
 
 
 def _forward_aggregated_heads_seg(kernels: list[Any], x: SO2FeatureField, edges: Any, alpha: Tensor, h: Tensor,
-                                  groups: tuple[Tensor, Tensor, Tensor]) -> Tensor:
-    """Every head's ``forward_factored_aggregated`` at once: ``(N, H, d_out)``."""
+                                  groups: tuple[Tensor, Tensor, Tensor], mixes: list[Tensor]) -> Tensor:
+    """Every head's ``forward_factored_aggregated`` at once on the heads' ``mixes``: ``(N, H, d_out)``."""
     hp = heads_plan(kernels[0])
     p = hp.plan
-    mixes = heads_mixes(x, hp, heads_mixing(kernels, hp))
     order, group_ptr, group_source = groups
     angular = torch.view_as_real(edges.angular_phases.contiguous()).contiguous().to(h.dtype)
     transport = torch.view_as_real(edges.transport_phases.contiguous()).contiguous().to(h.dtype)

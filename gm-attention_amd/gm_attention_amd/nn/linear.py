@@ -12,11 +12,13 @@ library GEMM on MFMA.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
 from torch import Tensor, nn
 
+from gm_attention_amd.nn.assembly import assembled
 from gm_attention_amd.representations import so2
 from gm_attention_amd.representations.field_type import SO2FeatureField, SO2FieldType
 
@@ -122,10 +124,27 @@ def flat_bias(bias: Tensor | None, fout: SO2FieldType) -> Tensor | None:
     return torch.cat([bias, bias.new_zeros(fout.dimension - fout.multiplicity(0))])
 
 
+def linear_parameters(lin: "SO2Linear") -> list[Tensor]:
+    """The layer's weights by frequency, then its bias where it has one."""
+    weights = [lin.weight[str(f)] for f in lin.common_frequencies]
+    return [*weights, lin.bias] if lin.has_bias else weights
+
+
+def matrix_and_bias(lin: "SO2Linear", params: list[Tensor]) -> list[Tensor]:
+    """The layer's matrix on flat rows, and its flat bias where it has one, from
+    its parameters (or stand-ins) in :func:`linear_parameters` order."""
+    common = lin.common_frequencies
+    m = weights_matrix(lin.field_type_in, lin.field_type_out, common, dict(zip(map(str, common), params)))
+    return [m, flat_bias(params[len(common)], lin.field_type_out)] if lin.has_bias else [m]
+
+
 def flat_forward(lin: "SO2Linear", flat: Tensor) -> Tensor:
     """``lin`` on flat rows ``(N, D_in)`` -> ``(N, D_out)``."""
-    bias = flat_bias(lin.bias if lin.has_bias else None, lin.field_type_out)
-    return FlatLinear.apply(flat, block_matrix(lin), bias)
+    if not lin.common_frequencies:  # no weights: the construction has nothing to read its type from
+        return FlatLinear.apply(flat, block_matrix(lin), flat_bias(lin.bias if lin.has_bias else None,
+                                                                   lin.field_type_out))
+    m, *bias = assembled(lin, "flat", linear_parameters(lin), functools.partial(matrix_and_bias, lin))
+    return FlatLinear.apply(flat, m, bias[0] if bias else None)
 
 
 class SO2Linear(nn.Module):

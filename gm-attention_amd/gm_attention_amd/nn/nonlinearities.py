@@ -22,6 +22,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from gm_attention_amd import _native
+from gm_attention_amd.nn.assembly import assembled
 from gm_attention_amd.nn.linear import FlatLinear
 from gm_attention_amd.representations.field_type import SO2FeatureField, SO2FieldType
 
@@ -86,10 +87,15 @@ class SO2ScalarGatedNonlinearity(nn.Module):
     def pre_activations(self, scalars: Tensor) -> Tensor:
         """Every frequency's gate pre-activations ``(N, sum a_n)``, frequency-major:
         one product with the stacked gate weights (``(a_0, sum a_n)``)."""
-        order = [str(f) for f in self.field_type.frequencies if f != 0]
-        weight = torch.cat([self.gates[k].weight for k in order]).t()
-        biases = [self.gates[k].bias for k in order]
-        return FlatLinear.apply(scalars, weight, None if biases[0] is None else torch.cat(biases))
+        gates = [self.gates[str(f)] for f in self.field_type.frequencies if f != 0]
+        biased = gates[0].bias is not None
+        params = [g.weight for g in gates] + ([g.bias for g in gates] if biased else [])
+
+        def build(ps: list[Tensor]) -> list[Tensor]:
+            return [torch.cat(ps[:len(gates)]).t()] + ([torch.cat(ps[len(gates):])] if biased else [])
+
+        weight, *bias = assembled(self, f"gates {biased}", params, build)
+        return FlatLinear.apply(scalars, weight, bias[0] if bias else None)
 
     def forward_flat(self, flat: Tensor) -> Tensor:
         """The nonlinearity on flat rows ``(N, D)``."""

@@ -19,6 +19,7 @@ import torch
 from torch import Tensor, nn
 
 from gm_attention_amd import _native
+from gm_attention_amd.nn.assembly import assembled
 from gm_attention_amd.representations.field_type import SO2FeatureField, SO2FieldType
 
 MAX_WIDTH = 1024  # flat width the HIP pass serves
@@ -81,9 +82,11 @@ class SO2LayerNorm(nn.Module):
 
     def gamma_flat(self, dtype: torch.dtype) -> Tensor:
         """The gains per flat coordinate (a copy's gain for both of its coordinates)."""
-        parts = [self.gamma[str(f)] if f == 0 else self.gamma[str(f)].repeat_interleave(2)
-                 for f in self.field_type.frequencies]
-        return torch.cat(parts).to(dtype)
+        def build(gains: list[Tensor]) -> list[Tensor]:
+            return [torch.cat([g if f == 0 else g.repeat_interleave(2)
+                               for f, g in zip(self.field_type.frequencies, gains, strict=True)])]
+
+        return assembled(self, "gamma", [self.gamma[str(f)] for f in self.field_type.frequencies], build)[0].to(dtype)
 
     def uses_hip(self, flat: Tensor) -> bool:
         return flat.device.type == "cuda" and flat.dtype in (torch.float32, torch.float64, torch.bfloat16) \

@@ -75,17 +75,31 @@ def stacked_trunk(kernels: list[Any]) -> tuple[Tensor, Tensor | None, Any]:
 HEADS_PER_LAUNCH = 8
 
 
-def trunk_hidden_heads(kernels: list[Any], rho: Tensor, dtype: torch.dtype | None = None) -> Tensor:
+def trunk_parameters(kernel: Any) -> list[Tensor]:
+    """The trunk's weight, then its bias where it has one."""
+    lin = list(kernel.radial_trunk)[0]
+    return [lin.weight] if lin.bias is None else [lin.weight, lin.bias]
+
+
+def stacked_forms(params: list[list[Tensor]]) -> list[Tensor]:
+    """Per launch of at most ``HEADS_PER_LAUNCH`` heads, the heads' stacked
+    weights and (where they have one) biases, from ``trunk_parameters``."""
+    return [torch.stack([p[i] for p in params[h0:h0 + HEADS_PER_LAUNCH]])
+            for h0 in range(0, len(params), HEADS_PER_LAUNCH) for i in range(len(params[0]))]
+
+
+def trunk_hidden_heads(kernels: list[Any], rho: Tensor, dtype: torch.dtype | None = None,
+                       forms: list[Tensor] | None = None) -> Tensor:
     """The stacked heads' trunk features ``(H, E, 16)`` on ``rho = d / cutoff``,
     at most ``HEADS_PER_LAUNCH`` heads a launch, in rho's dtype or ``dtype``
-    (bfloat16: float32 arithmetic, the features rounded as stored)."""
+    (bfloat16: float32 arithmetic, the features rounded as stored), from the
+    trunks' ``stacked_forms`` (stacked here when not given)."""
     rb = kernels[0].radial_basis
     rho = rho.contiguous()
+    params = [trunk_parameters(k) for k in kernels]
+    stacked = iter(stacked_forms(params) if forms is None else forms)
     parts = []
-    for h0 in range(0, len(kernels), HEADS_PER_LAUNCH):
-        chunk = kernels[h0:h0 + HEADS_PER_LAUNCH]
-        weight = torch.stack([list(k.radial_trunk)[0].weight for k in chunk])
-        biases = [list(k.radial_trunk)[0].bias for k in chunk]
-        bias = None if biases[0] is None else torch.stack(biases)
+    for _ in range(0, len(kernels), HEADS_PER_LAUNCH):
+        weight, bias = next(stacked), next(stacked) if len(params[0]) == 2 else None
         parts.append(RadialTrunk.apply(rho, weight, bias, rb.centers.contiguous(), float(rb.width), dtype))
     return parts[0] if len(parts) == 1 else torch.cat(parts, dim=0)

@@ -594,6 +594,18 @@ int gm_radial_trunk_backward_bf16(const uint16_t* dh, const float* rho, const fl
                                   const float* centers, int64_t n_edges, int64_t H, int64_t T, int64_t B, double width,
                                   float* partial, float* dparams, void* stream);
 
+/* ---------------- assembled parameters ----------------
+ *
+ * out[e] = the sum over u < uses, in order, of +-src[t][o] for codes[u][e] =
+ * t << 40 | o << 1 | negative (-1: no term): the assembled forms of a layer's
+ * parameters (and, with the roles exchanged, their gradients) in one launch.
+ * `src` is a host array of n_src <= 256 device pointers (null: zeros), codes a
+ * device array (uses, n) whose tensor numbers are below n_src and whose
+ * offsets lie within their tensors.  Stands for the concatenations and stacks
+ * of the reference's nn/attention.py:653-669 and nn/kernels.py:506-546. */
+int gm_signed_gather_f32(const float* const* src, int64_t n_src, const int64_t* codes, int64_t uses, int64_t n,
+                         float* out, void* stream);
+
 /* ---------------- node mixes (the factored kernel's channel mixing) ----------------
  *
  * Every head's node mixes for one input frequency n as one real product over

@@ -1,0 +1,122 @@
+"""Assembled parameter forms (nn/assembly.py): the plan's gather and its
+transposed gather against the construction itself and its autograd gradient,
+by evaluating the codes in torch on the CPU, and the HIP launch on the GPU
+(moves and sign changes: bit for bit; gradients: the uses of an entry added)."""
+
+import pytest
+import torch
+
+from gm_attention_amd.nn import assembly
+from gm_attention_amd.nn.attention import SO2MHSA, _LayerForms
+from gm_attention_amd.nn.linear import complex_as_real
+from gm_attention_amd.representations.field_type import SO2FieldType
+
+
+def _build(ps):
+    """Stacks, transposes, negated entries, repeats, zeros, an unused and a repeatedly used parameter."""
+    a, b, c, _unused, d = ps
+    m = a.new_zeros(9, 8)
+    m[:4, :6] = complex_as_real(a)
+    m[5:, 2:5] = b.t()
+    return [m, torch.cat([c, -c, c.new_zeros(3)]), torch.stack([d] * 5), d.reshape(1, 1)]
+
+
+SHAPES = [(3, 2, 2), (3, 4), (7,), (5, 5), (1,)]
+
+
+def _params(device="cpu", dtype=torch.float32):
+    g = torch.Generator().manual_seed(3)
+    return [torch.randn(s, generator=g).to(device, dtype) for s in SHAPES]
+
+
+def _gather(sources, codes):
+    """What gm_signed_gather_f32 computes, by its definition."""
+    out = torch.zeros(codes.shape[1], dtype=torch.float64)
+    for row in codes.cpu():
+        for e, code in enumerate(row.tolist()):
+            if code >= 0 and sources[code >> 40] is not None:
+                x = float(sources[code >> 40].reshape(-1)[(code >> 1) & ((1 << 39) - 1)])
+                out[e] += -x if code & 1 else x
+    return out
+
+
+def test_plan_codes_restate_the_construction_and_its_gradient():
+    params = [p.double().requires_grad_(True) for p in _params()]
+    plan = assembly.Plan(tuple(p.shape for p in params), _build, torch.device("cpu"))
+    want = _build(params)
+    flat = _gather([p.detach() for p in params], plan.codes)
+    for w, start, shape in zip(want, plan.out_starts, plan.form_shapes):
+        assert torch.equal(flat[start:start + shape.numel()].view(shape), w.detach())
+    up = [torch.randn_like(w) for w in want]
+    up[1] = None  # a form nothing reads has no gradient
+    grads = torch.autograd.grad([w for w, u in zip(want, up) if u is not None], params,
+                                [u for u in up if u is not None], allow_unused=True)
+    back = _gather(up, plan.gradient_codes())
+    for p, g, start in zip(params, grads, plan.in_starts):
+        got = back[start:start + p.numel()].view(p.shape)
+        assert torch.allclose(got, torch.zeros_like(p) if g is None else g, rtol=0, atol=1e-14)
+
+
+def test_parameters_the_kernel_does_not_take_go_through_the_construction():
+    class Owner:
+        pass
+
+    params = [p.requires_grad_(True) for p in _params()]
+    got = assembly.assembled(Owner(), "x", params, _build)  # CPU
+    for g, w in zip(got, _build(params)):
+        assert torch.equal(g, w) and g.grad_fn is not None
+
+
+@pytest.mark.gpu
+def test_forms_and_gradients_on_the_gpu(cuda):
+    class Owner:
+        pass
+
+    owner = Owner()
+    base = torch.empty(64, device=cuda)
+    params = _params(cuda)
+    params[2] = base[1:8].copy_(params[2])  # a view that starts off any alignment
+    params = [p.requires_grad_(True) for p in params]
+    got = assembly.assembled(owner, "x", params, _build)
+    want = _build(params)
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    up = [torch.randn_like(w) for w in want]
+    grads = torch.autograd.grad(got, params, up)
+    ref = torch.autograd.grad([w.double() for w in want], params, [u.double() for u in up], allow_unused=True)
+    for g, r in zip(grads, ref):
+        assert torch.allclose(g, torch.zeros_like(g) if r is None else r, rtol=0, atol=1e-6)
+    few = assembly.assembled(owner, "x", [p.detach() for p in params], _build)
+    assert not any(f.requires_grad for f in few)
+    wider = [p.repeat(2, *([1] * (p.dim() - 1))) if i == 2 else p for i, p in enumerate(params)]
+    again = assembly.assembled(owner, "x", wider, _build)  # other shapes under the same name: a plan of their own
+    for g, w in zip(again, _build(wider)):
+        assert torch.equal(g, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("field,heads,bias", [({0: 16, 1: 16, 2: 16}, 4, True), ({0: 6, 1: 4, 2: 2}, 2, False),
+                                              ({0: 4, 1: 4}, 2, True)])
+def test_layer_forms_equal_the_layers_own_constructions(field, heads, bias, cuda):
+    from gm_attention_amd.nn import fused_factored, radial
+    from gm_attention_amd.nn.attention import _heads_permutation, _stacked_matrix
+    from gm_attention_amd.nn.linear import linear_parameters, matrix_and_bias
+
+    torch.manual_seed(1)
+    mhsa = SO2MHSA(SO2FieldType(field), heads, cutoff=0.3, bias=bias, batched=True, dtype=torch.float32, device=cuda)
+    values = [h.value for h in mhsa.heads]
+    layout = fused_factored.heads_layout(values, torch.float32)
+    forms = _LayerForms(mhsa, values, layout, True)
+    assert forms.served
+    for form, lins in ((forms.query, [h.query for h in mhsa.heads]), (forms.key, [h.key for h in mhsa.heads])):
+        want = _stacked_matrix(lins, mhsa.field_type_in, [linear_parameters(lin) for lin in lins])
+        assert torch.equal(form[0], want[0])
+        assert torch.equal(form[1], want[1]) if bias else form[1] is None
+    m, *b = matrix_and_bias(mhsa.output_projection, linear_parameters(mhsa.output_projection))
+    assert torch.equal(forms.projection[0], m.index_select(0, _heads_permutation(mhsa, m.device)))
+    assert torch.equal(forms.projection[1], b[0]) if bias else forms.projection[1] is None
+    for got, want in zip(forms.mixing, fused_factored.mixing_forms(values, layout,
+                                                                   [k.readout_parameters() for k in values])):
+        assert torch.equal(got, want)
+    for got, want in zip(forms.trunk, radial.stacked_forms([radial.trunk_parameters(k) for k in values]), strict=True):
+        assert torch.equal(got, want)
