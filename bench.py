@@ -147,18 +147,20 @@ def cost_factored_forward_grouped(a, kw, out):
     E = rho_g.shape[0]
     es = _es(h_g) if h_g is not None else 4  # bfloat16 streams: h and the rows at 2 bytes
     h_bytes = es * (K - 1) if h_g is not None else 4
-    return E * (h_bytes + 16 + es * d_out) + n_nodes * 4 * K * C, E * (2.0 * K * C + 8 * wc)
+    H = h_g.shape[0] if h_g is not None and h_g.dim() == 3 else 1  # heads in the launch
+    return H * (E * (h_bytes + 16 + es * d_out) + n_nodes * 4 * K * C), H * E * (2.0 * K * C + 8 * wc)
 
 
 def cost_factored_backward_grouped(a, kw, out):
     g, target_g, weights_g, rows_g, h_g, runs, n_nodes, phase_g, rho_g = a[:9]
     K, C, wc = _factored_shape(*a[16:19])
-    d_out = g.shape[1]
+    d_out = g.shape[-1]
     E = rho_g.shape[0]
+    H = h_g.shape[0] if h_g is not None and h_g.dim() == 3 else 1  # heads in the launch
     es = _es(h_g) if h_g is not None else 4  # bfloat16 streams: h, the rows and dh at 2 bytes
     h_bytes = es * (K - 1) if h_g is not None else 4
     per_edge = h_bytes + 16 + 4 + 8 + 4 * d_out + es * d_out + es * (K - 1) + 4
-    return E * per_edge + 2 * n_nodes * 4 * K * C, E * (4.0 * K * C + 8 * wc)
+    return H * (E * per_edge + 2 * n_nodes * 4 * K * C), H * E * (4.0 * K * C + 8 * wc)
 
 
 def cost_factored_forward(a, kw, out):

@@ -123,6 +123,12 @@ struct FactArgs {
   // lane-owned kernels with compiled-in slots: h, the rows and dh are
   // bfloat16 (the pointers above then address 2-byte elements)
   int b16;
+  // grouped kernels: several heads in one launch, head v's streams at v times
+  // these elements from the pointers above (h and dh, the rows, the weights
+  // and dweights, g) and its mixes those of "node" j n_heads + v (the runs'
+  // node strides then step over one head)
+  int n_heads;
+  int64_t h_hs, rows_hs, w_hs, g_hs;
 };
 
 template <typename T>
@@ -999,6 +1005,30 @@ __device__ __forceinline__ void factors_grouped(const FactArgs<float>& a, const 
   }
 }
 
+// A grouped kernel's workgroup: its source group (negative: none) and head.
+// The heads of a group run on one XCD one after the other, so the streams
+// they share (phases, targets, the targets' gradient rows) meet in its L2.
+struct GroupHead {
+  int64_t gi;
+  int head;
+};
+__device__ __forceinline__ GroupHead group_head(const FactArgs<float>& a) {
+  int64_t b = blockIdx.x, nb = gridDim.x;
+  int head = 0;
+  if (a.n_heads > 1) {
+    const uint32_t i = blockIdx.x >> 3, heads = (uint32_t)a.n_heads;
+    head = (int)(i % heads);
+    b = (int64_t)(i / heads) * 8 + (blockIdx.x & 7);
+    nb = a.n_groups;
+    if (b >= nb) return {-1, 0};
+  }
+  return {a.group_order ? a.group_order[b] : xcd_spread_block(b, nb), head};
+}
+// Workgroups of a grouped launch: every head's groups, the groups in whole rounds of the XCDs.
+inline unsigned group_blocks(const FactArgs<float>& a) {
+  return (unsigned)(a.n_heads > 1 ? (a.n_groups + 7) / 8 * 8 * a.n_heads : a.n_groups);
+}
+
 struct TileIn {
   floatx4 h;    // this lane's slice of h: forward h(g = base + m)[4 q .. 4 q + 3]; backward h(base + l / 4)[4 (l % 4) ..]
   floatx4 ph;   // phase row of edge base + l / 4, floats 4 (l % 4) .. + 3
@@ -1008,7 +1038,7 @@ struct TileIn {
 };
 
 template <bool BACKWARD>
-__device__ __forceinline__ TileIn load_tile(const FactArgs<float>& a, int64_t base, int n, int lane) {
+__device__ __forceinline__ TileIn load_tile(const FactArgs<float>& a, int64_t hv, int64_t base, int n, int lane) {
   const int m = lane & 15, q = lane >> 4, e4 = lane >> 2, part = lane & 3;
   TileIn t;
   t.h = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -1017,15 +1047,15 @@ __device__ __forceinline__ TileIn load_tile(const FactArgs<float>& a, int64_t ba
   t.w = 0.f;
   t.tgt = 0;
   if (!BACKWARD) {
-    if (m < n) t.h = *reinterpret_cast<const floatx4*>(a.h + (base + m) * 16 + 4 * q);
+    if (m < n) t.h = *reinterpret_cast<const floatx4*>(a.h + hv * a.h_hs + (base + m) * 16 + 4 * q);
   } else {
-    if (e4 < n) t.h = *reinterpret_cast<const floatx4*>(a.h + (base + e4) * 16 + 4 * part);
+    if (e4 < n) t.h = *reinterpret_cast<const floatx4*>(a.h + hv * a.h_hs + (base + e4) * 16 + 4 * part);
   }
   if (e4 < n) t.ph = *reinterpret_cast<const floatx4*>(a.phase_g + (base + e4) * kPhaseRow + 4 * part);
   if (lane < n) {
     t.rho = a.rho_g[base + lane];
     if (BACKWARD) {
-      t.w = a.weights[base + lane];
+      t.w = a.weights[hv * a.w_hs + base + lane];
       t.tgt = a.target_g[base + lane];
     }
   }
@@ -1047,9 +1077,10 @@ __global__ __launch_bounds__(64) void factored_forward_grouped(FactArgs<float> a
   for (int i = lane; i <= d_out; i += kWave) optr[i] = a.optr[i];
   for (int i = lane; i < a.optr[d_out]; i += kWave) olist[i] = a.olist[i];
   stage_desc(a, Bd, lane);
-  const int64_t gi = a.group_order ? a.group_order[blockIdx.x] : xcd_spread_block(blockIdx.x, gridDim.x);
+  const GroupHead gh = group_head(a);
+  const int64_t gi = gh.gi, hv = gh.head;
   if (gi < 0 || gi >= a.n_groups) return;  // a malformed order names no group
-  const int64_t j = a.group_source[gi];
+  const int64_t j = a.group_source[gi] * a.n_heads + hv;
   const int64_t g0 = a.group_ptr[gi], g1 = a.group_ptr[gi + 1];
   float za[NT][4], z0[NT][4];
   int vb[NT][2];
@@ -1066,13 +1097,13 @@ __global__ __launch_bounds__(64) void factored_forward_grouped(FactArgs<float> a
       vb[nt][p] = c < wc2 ? (int)a.cmap[c >> 1] : -1;
     }
   }
-  TileIn next = load_tile<false>(a, g0, (int)((g1 - g0) < kMT ? (g1 - g0) : kMT), lane);
+  TileIn next = load_tile<false>(a, hv, g0, (int)((g1 - g0) < kMT ? (g1 - g0) : kMT), lane);
   for (int64_t base = g0; base < g1; base += kMT) {
     const int n = (int)((g1 - base) < kMT ? (g1 - base) : kMT);
     const TileIn cur = next;
     if (base + kMT < g1) {
       const int64_t nb2 = base + kMT;
-      next = load_tile<false>(a, nb2, (int)((g1 - nb2) < kMT ? (g1 - nb2) : kMT), lane);
+      next = load_tile<false>(a, hv, nb2, (int)((g1 - nb2) < kMT ? (g1 - nb2) : kMT), lane);
     }
     *reinterpret_cast<floatx4*>(Ph + 4 * lane) = cur.ph;
     if (lane < kMT) Rh[lane] = cur.rho;
@@ -1104,7 +1135,7 @@ __global__ __launch_bounds__(64) void factored_forward_grouped(FactArgs<float> a
     wave_sync();
     for (int e = q; e < n; e += 4) {
       const float* v = Vt + e * VP;
-      float* row = a.out + (base + e) * d_out;
+      float* row = a.out + hv * a.rows_hs + (base + e) * d_out;
       for (int o = m; o < d_out; o += kMT) {
         float sum = 0.f;
         for (int k = optr[o]; k < optr[o + 1]; ++k) sum += v[olist[k]];
@@ -1130,9 +1161,10 @@ __global__ __launch_bounds__(64) void factored_backward_grouped(FactArgs<float> 
   float* Ht = Wt + kMT * WP;                                       // [kMT][16]
   const int lane = threadIdx.x, m = lane & 15, q = lane >> 4;
   stage_desc(a, Bd, lane);
-  const int64_t gi = a.group_order ? a.group_order[blockIdx.x] : xcd_spread_block(blockIdx.x, gridDim.x);
+  const GroupHead gh = group_head(a);
+  const int64_t gi = gh.gi, hv = gh.head;
   if (gi < 0 || gi >= a.n_groups) return;  // a malformed order names no group
-  const int64_t j = a.group_source[gi];
+  const int64_t j = a.group_source[gi] * a.n_heads + hv;
   const int64_t g0 = a.group_ptr[gi], g1 = a.group_ptr[gi + 1];
   float zb[4 * NT];
 #pragma unroll
@@ -1147,13 +1179,13 @@ __global__ __launch_bounds__(64) void factored_backward_grouped(FactArgs<float> 
     dz[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
     dz0[nt] = 0.f;
   }
-  TileIn next = load_tile<true>(a, g0, (int)((g1 - g0) < kMT ? (g1 - g0) : kMT), lane);
+  TileIn next = load_tile<true>(a, hv, g0, (int)((g1 - g0) < kMT ? (g1 - g0) : kMT), lane);
   for (int64_t base = g0; base < g1; base += kMT) {
     const int n = (int)((g1 - base) < kMT ? (g1 - base) : kMT);
     const TileIn cur = next;
     if (base + kMT < g1) {
       const int64_t nb2 = base + kMT;
-      next = load_tile<true>(a, nb2, (int)((g1 - nb2) < kMT ? (g1 - nb2) : kMT), lane);
+      next = load_tile<true>(a, hv, nb2, (int)((g1 - nb2) < kMT ? (g1 - nb2) : kMT), lane);
     }
     *reinterpret_cast<floatx4*>(Ph + 4 * lane) = cur.ph;
     *reinterpret_cast<floatx4*>(Ht + 4 * lane) = cur.h;  // Ht[e = l / 4][4 (l % 4) ..]
@@ -1164,17 +1196,18 @@ __global__ __launch_bounds__(64) void factored_backward_grouped(FactArgs<float> 
     }
     wave_sync();
     for (int e = q; e < kMT; e += 4) {
-      const float* grow = e < n ? a.g + Tg[e] * a.g_ld : nullptr;
+      const float* grow = e < n ? a.g + hv * a.g_hs + Tg[e] * a.g_ld : nullptr;
       for (int o = m; o < d_out; o += kMT) Gt[e * d_out + o] = grow ? grow[o] : 0.f;
     }
     factors_grouped(a, Bd, Ph, Rh, Ft, lane);
     wave_sync();
     if (lane < n) {
-      const float* r = a.rows + (base + lane) * d_out;
+      const float* r = a.rows + hv * a.rows_hs + (base + lane) * d_out;
       const float* gr = Gt + lane * d_out;
       float sum = 0.f;
       for (int o = 0; o < d_out; ++o) sum += gr[o] * r[o];
-      a.dweights[base + lane] = a.accumulate ? a.dweights[base + lane] + sum : sum;
+      float* dw = a.dweights + hv * a.w_hs + base + lane;
+      *dw = a.accumulate ? *dw + sum : sum;
     }
     float w[NT][4];
 #pragma unroll
@@ -1207,7 +1240,10 @@ __global__ __launch_bounds__(64) void factored_backward_grouped(FactArgs<float> 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int e = 4 * q + r;
-      if (e < n && m + 1 < a.K) a.dh[(base + e) * 16 + m] = a.accumulate ? a.dh[(base + e) * 16 + m] + dh[r] : dh[r];
+      if (e < n && m + 1 < a.K) {
+        float* to = a.dh + hv * a.h_hs + (base + e) * 16 + m;
+        *to = a.accumulate ? *to + dh[r] : dh[r];
+      }
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -1931,15 +1967,16 @@ factored_forward_lanes(FactArgs<float> a) {
   __shared__ __align__(16) uint8_t colslot[128];
   const int lane = threadIdx.x, m = lane & 15, q = lane >> 4;
   const int d_out = P::kStatic ? P::kDout : a.d_out;
-  const int64_t gi = a.group_order ? a.group_order[blockIdx.x] : xcd_spread_block(blockIdx.x, gridDim.x);
+  const GroupHead gh = group_head(a);
+  const int64_t gi = gh.gi, hv = gh.head;
   if (gi < 0 || gi >= a.n_groups) return;  // a malformed order names no group
-  const int64_t j = a.group_source[gi];
+  const int64_t j = a.group_source[gi] * a.n_heads + hv;
   const int64_t g0 = a.group_ptr[gi];
   const int ng = (int)(a.group_ptr[gi + 1] - g0);
   constexpr bool fused = FUSED;
   // h and the rows: float32, or bfloat16 (B16) at half the bytes
-  const char* h_b = reinterpret_cast<const char*>(a.h);
-  char* out_b = reinterpret_cast<char*>(a.out);
+  const char* h_b = reinterpret_cast<const char*>(a.h) + stream_bytes<B16>(hv * a.h_hs);
+  char* out_b = reinterpret_cast<char*>(a.out) + stream_bytes<B16>(hv * a.rows_hs);
   const auto h_r = span(fused ? nullptr : h_b + stream_bytes<B16>(g0 * 16), fused ? 0 : stream_bytes<B16>((int64_t)ng * 16));
   const auto ph_r = P::kStatic ? span(a.zw_g + g0 * 4, (int64_t)ng * 16)
                                : span(a.phase_g + g0 * kPhaseRow, (int64_t)ng * kPhaseRow * 4);
@@ -2072,7 +2109,7 @@ __device__ __forceinline__ void backward_tile(const FactArgs<float>& a, const Bw
                                               const floatx4 (&zb)[NT], floatx4 (&dz)[NT], float (&dz0)[NT], float* Sh,
                                               float* Ph, float* Gt, int64_t* Tg, float* Hs, const BwdSpans& sp,
                                               int d_out, int ng, int tb, int m, int q, const TrunkLane& tl,
-                                              bool fused) {
+                                              bool fused, const float* g_b) {
   const int row = (tb + m) * d_out;
   // edge m's features 4 q .. 4 q + 3 (read as one 16-byte piece, or the fused trunk's),
   // handed to the dZ operand's layout (feature m of edges 4 q + i) through Hs with the
@@ -2131,7 +2168,7 @@ __device__ __forceinline__ void backward_tile(const FactArgs<float>& a, const Bw
     if (q == 0) Tg[m] = cur.tgt;
     wave_sync();
     for (int e = q; e < kMT; e += 4) {
-      const float* grow = tb + e < ng ? a.g + Tg[e] * a.g_ld : nullptr;
+      const float* grow = tb + e < ng ? g_b + Tg[e] * a.g_ld : nullptr;
       for (int o = m; o < GS; o += kMT) Gt[e * GS + o] = grow && o < d_out ? grow[o] : 0.f;
     }
     wave_sync();
@@ -2235,26 +2272,28 @@ factored_backward_lanes(FactArgs<float> a) {
   __shared__ __align__(16) uint32_t zsl[ZDMA ? 16 * NT : 1];  // ZDMA: where each slot column's rows sit
   const int lane = threadIdx.x, m = lane & 15, q = lane >> 4;
   const int d_out = P::kStatic ? P::kDout : a.d_out;
-  const int64_t gi = a.group_order ? a.group_order[blockIdx.x] : xcd_spread_block(blockIdx.x, gridDim.x);
+  const GroupHead gh = group_head(a);
+  const int64_t gi = gh.gi, hv = gh.head;
   if (gi < 0 || gi >= a.n_groups) return;  // a malformed order names no group
-  const int64_t j = a.group_source[gi];
+  const int64_t j = a.group_source[gi] * a.n_heads + hv;
   const int64_t g0 = a.group_ptr[gi];
   const int ng = (int)(a.group_ptr[gi + 1] - g0);
   constexpr bool fused = FUSED;
   BwdSpans sp;
   // h, the rows and dh: float32, or bfloat16 (B16) at half the bytes
-  const char* h_b = reinterpret_cast<const char*>(a.h);
-  const char* rows_b = reinterpret_cast<const char*>(a.rows);
-  char* dh_b = reinterpret_cast<char*>(a.dh);
+  const char* h_b = reinterpret_cast<const char*>(a.h) + stream_bytes<B16>(hv * a.h_hs);
+  const char* rows_b = reinterpret_cast<const char*>(a.rows) + stream_bytes<B16>(hv * a.rows_hs);
+  char* dh_b = reinterpret_cast<char*>(a.dh) + stream_bytes<B16>(hv * a.h_hs);
+  const float* g_b = a.g + hv * a.g_hs;
   sp.h = span(fused ? nullptr : h_b + stream_bytes<B16>(g0 * 16), fused ? 0 : stream_bytes<B16>((int64_t)ng * 16));
   sp.ph = P::kStatic ? span(a.zw_g + g0 * 4, (int64_t)ng * 16)
                      : span(a.phase_g + g0 * kPhaseRow, (int64_t)ng * kPhaseRow * 4);
   sp.rho = span(a.rho_g + g0, (int64_t)ng * 4);
-  sp.w = span(a.weights + g0, (int64_t)ng * 4);
+  sp.w = span(a.weights + hv * a.w_hs + g0, (int64_t)ng * 4);
   sp.t = span(a.target_g + g0, (int64_t)ng * 8);
   sp.rows = span(rows_b + stream_bytes<B16>(g0 * d_out), stream_bytes<B16>((int64_t)ng * d_out));
   sp.dh = span(dh_b + stream_bytes<B16>(g0 * 16), stream_bytes<B16>((int64_t)ng * 16));
-  sp.dw = span(a.dweights + g0, (int64_t)ng * 4);
+  sp.dw = span(a.dweights + hv * a.w_hs + g0, (int64_t)ng * 4);
   constexpr bool acc = ACC;
   // Two tiles in flight (buffers A and B, each refilled right after its
   // tile's stores); with static slots the targets run three tiles ahead and
@@ -2281,8 +2320,8 @@ factored_backward_lanes(FactArgs<float> a) {
   OutVals<P::kStatic ? NT : 1> oa, ob;
   int64_t tn = 0;  // static slots: the targets of the tile two ahead of the current one
   if constexpr (P::kStatic) {
-    load_outs<NT, P, B16>(oa, a.g + t0 * a.g_ld, sp.rows, m * d_out, q);
-    load_outs<NT, P, B16>(ob, a.g + t1 * a.g_ld, sp.rows, (kMT + m) * d_out, q);
+    load_outs<NT, P, B16>(oa, g_b + t0 * a.g_ld, sp.rows, m * d_out, q);
+    load_outs<NT, P, B16>(ob, g_b + t1 * a.g_ld, sp.rows, (kMT + m) * d_out, q);
     tn = bload_i64(sp.t, (2 * kMT + m) * 8);
   }
   // Z_t(j) for t = 1 + m at the lane's slot columns 16 nt + 4 q + r
@@ -2315,18 +2354,18 @@ factored_backward_lanes(FactArgs<float> a) {
   if (fused) tl = trunk_lane(a, m, q);
   for (int tb = 0;;) {
     backward_tile<NT, P, decltype(oa), B16>(a, ta, oa, zb, dz, dz0, Sh, Ph, Gt, Tg, Hs, sp, d_out, ng, tb, m, q, tl,
-                                            fused);
+                                            fused, g_b);
     if constexpr (P::kStatic) {
-      load_outs<NT, P, B16>(oa, a.g + tn * a.g_ld, sp.rows, (tb + 2 * kMT + m) * d_out, q);
+      load_outs<NT, P, B16>(oa, g_b + tn * a.g_ld, sp.rows, (tb + 2 * kMT + m) * d_out, q);
       tn = bload_i64(sp.t, (tb + 3 * kMT + m) * 8);
     }
     ta = load_bwd<P, B16>(sp.h, sp.ph, sp.rho, sp.w, sp.t, tb + 2 * kMT, m, q, fused, sp.dh, sp.dw, acc);
     tb += kMT;
     if (tb >= ng) break;
     backward_tile<NT, P, decltype(ob), B16>(a, tbf, ob, zb, dz, dz0, Sh, Ph, Gt, Tg, Hs, sp, d_out, ng, tb, m, q, tl,
-                                            fused);
+                                            fused, g_b);
     if constexpr (P::kStatic) {
-      load_outs<NT, P, B16>(ob, a.g + tn * a.g_ld, sp.rows, (tb + 2 * kMT + m) * d_out, q);
+      load_outs<NT, P, B16>(ob, g_b + tn * a.g_ld, sp.rows, (tb + 2 * kMT + m) * d_out, q);
       tn = bload_i64(sp.t, (tb + 3 * kMT + m) * 8);
     }
     tbf = load_bwd<P, B16>(sp.h, sp.ph, sp.rho, sp.w, sp.t, tb + 2 * kMT, m, q, fused, sp.dh, sp.dw, acc);
@@ -2387,6 +2426,7 @@ int prepare(FactArgs<T>& a, const T* h, const Runs<T>& runs, const T* angular, c
   a.d_out = (int)d_out;
   a.g_ld = d_out;
   a.n_groups = n_groups;
+  a.n_heads = 1;
   // Every packed column belongs to exactly one block, and the blocks sharing
   // an output slot are consecutive, alike in width and kind of output.
   int covered_c = 0, covered_r = 0, open = -1;
@@ -2687,7 +2727,7 @@ size_t lds_backward_grouped(const FactArgs<float>& a, int NT) {
 
 template <int NT>
 void launch_grouped_nt(bool forward, const FactArgs<float>& a, hipStream_t stream) {
-  const dim3 grid((unsigned)a.n_groups), block(64);
+  const dim3 grid(group_blocks(a)), block(64);
   if (forward)
     hipLaunchKernelGGL(factored_forward_grouped<NT>, grid, block, lds_forward_grouped(a, NT), stream, a);
   else
@@ -2754,7 +2794,7 @@ inline bool zdma_backward() {
 // The lane-owned kernels over bfloat16 streams (compiled-in slots, trunk features read).
 template <int NT, class P>
 void launch_lanes_b16(bool forward, const FactArgs<float>& a, hipStream_t stream) {
-  const dim3 grid((unsigned)a.n_groups), block(64);
+  const dim3 grid(group_blocks(a)), block(64);
   if (forward) {
     if (split_products())
       hipLaunchKernelGGL((factored_forward_lanes<NT, P, false, true, true>), grid, block, 0, stream, a);
@@ -2778,7 +2818,7 @@ void launch_lanes_b16(bool forward, const FactArgs<float>& a, hipStream_t stream
 
 template <int NT, class P = RuntimeSlots>
 void launch_lanes_nt(bool forward, const FactArgs<float>& a, hipStream_t stream) {
-  const dim3 grid((unsigned)a.n_groups), block(64);
+  const dim3 grid(group_blocks(a)), block(64);
   const bool fused = a.trunk_w != nullptr;  // the trunk evaluated in the kernels: their own instantiation
   if constexpr (P::kStatic) {
     if (a.b16) return launch_lanes_b16<NT, P>(forward, a, stream);
@@ -3072,6 +3112,26 @@ GM_FACT_EXPORTS(double, f64)
 namespace gm {
 namespace {
 
+// Several heads in one launch (FactArgs::n_heads); one head by default.
+struct HeadStrides {
+  int64_t n = 1, h = 0, rows = 0, w = 0, g = 0;
+};
+
+int set_heads(FactArgs<float>& a, const HeadStrides& s) {
+  GM_REQUIRE(s.n >= 1 && s.n <= 1024, "between 1 and 1024 heads");
+  GM_REQUIRE(s.n == 1 || a.trunk_w == nullptr, "the fused trunk takes one head a launch");
+  GM_REQUIRE(s.n == 1 || s.h % 4 == 0, "the heads' stride must keep h 16-byte aligned");
+  GM_REQUIRE(s.n == 1 || a.n_slots == 0 || (s.rows % 2 == 0 && s.g % 2 == 0),
+             "the heads' strides must keep the rows and g 8-byte aligned");  // the lane-owned kernels' paired reads
+  GM_REQUIRE((a.n_groups + 7) / 8 * 8 * s.n < (int64_t(1) << 31), "too many groups and heads for one launch");
+  a.n_heads = (int)s.n;
+  a.h_hs = s.h;
+  a.rows_hs = s.rows;
+  a.w_hs = s.w;
+  a.g_hs = s.g;
+  return GM_OK;
+}
+
 // The grouped forward; b16: h_g and rows_g hold bfloat16 (compiled-in lane slots only).
 int forward_grouped(bool b16, const float* h_g, const float* const* z, const int64_t* node_stride,
                     const int64_t* t_stride, const int64_t* width, int64_t n_runs, const float* phase_g,
@@ -3079,7 +3139,8 @@ int forward_grouped(bool b16, const float* h_g, const float* const* z, const int
                     const int64_t* group_source, const int64_t* group_order, int64_t n_nodes, int64_t n_edges,
                     int64_t n_groups, int64_t K, int64_t wc, int64_t wr, int64_t pa, int64_t pt, int64_t n_blocks,
                     int64_t d_out, const float* trunk_w, const float* trunk_b, const float* trunk_centers,
-                    int64_t trunk_nb, double trunk_width, float* rows_g, void* stream) {
+                    int64_t trunk_nb, double trunk_width, float* rows_g, void* stream,
+                    const HeadStrides& heads = HeadStrides{}) {
   GM_REQUIRE(z && node_stride && t_stride && width, "the mix runs must be host arrays");
   GM_REQUIRE(!(b16 && trunk_w), "bfloat16 streams read the trunk features (no fused trunk)");
   const gm::Runs<float> runs{z, nullptr, node_stride, t_stride, width, n_runs};
@@ -3092,6 +3153,8 @@ int forward_grouped(bool b16, const float* h_g, const float* const* z, const int
   GM_REQUIRE(rows_g, "rows must be a device pointer");
   a.out = rows_g;
   a.group_order = group_order;
+  const int heads_status = set_heads(a, heads);
+  if (heads_status != GM_OK) return heads_status;
   GM_REQUIRE(zw_g == nullptr || gm::aligned(zw_g, 16), "zw_g must be a 16-byte aligned device pointer (or null)");
   a.zw_g = zw_g;
   a.b16 = b16;
@@ -3109,7 +3172,7 @@ int backward_grouped(bool b16, const float* g, int64_t g_ld, const int64_t* targ
                      int64_t n_edges, int64_t n_groups, int64_t K, int64_t wc, int64_t wr, int64_t pa, int64_t pt,
                      int64_t n_blocks, int64_t d_out, const float* trunk_w, const float* trunk_b,
                      const float* trunk_centers, int64_t trunk_nb, double trunk_width, int64_t accumulate, float* dh_g,
-                     float* dweights_g, void* stream) {
+                     float* dweights_g, void* stream, const HeadStrides& heads = HeadStrides{}) {
   GM_REQUIRE(z && dz && node_stride && t_stride && width, "the mix runs must be host arrays");
   GM_REQUIRE(!(b16 && trunk_w), "bfloat16 streams read the trunk features (no fused trunk)");
   GM_REQUIRE(g_ld >= d_out, "g_ld must be at least d_out");
@@ -3128,6 +3191,8 @@ int backward_grouped(bool b16, const float* g, int64_t g_ld, const int64_t* targ
   a.g = g;
   a.g_ld = g_ld;
   a.group_order = group_order;
+  const int heads_status = set_heads(a, heads);
+  if (heads_status != GM_OK) return heads_status;
   GM_REQUIRE(zw_g == nullptr || gm::aligned(zw_g, 16), "zw_g must be a 16-byte aligned device pointer (or null)");
   a.zw_g = zw_g;
   a.target_g = target_g;
@@ -3196,6 +3261,37 @@ extern "C" int gm_factored_backward_grouped_ld_bf16(
                               phase_g, rho_g, zw_g, desc, group_ptr, group_source, group_order, n_nodes, n_edges,
                               n_groups, K, wc, wr, pa, pt, n_blocks, d_out, nullptr, nullptr, nullptr, 0, 0.0,
                               accumulate, reinterpret_cast<float*>(dh_g), dweights_g, stream);
+}
+
+// Several heads' grouped kernels in one launch: head v reads and writes its
+// streams v times the head strides (elements) past the pointers given, and its
+// mixes at runs whose node stride steps over one head of a node's n_heads.
+extern "C" int gm_factored_forward_heads_f32(
+    const float* h_g, const float* const* z, const int64_t* node_stride, const int64_t* t_stride,
+    const int64_t* width, int64_t n_runs, const float* phase_g, const float* rho_g, const float* zw_g,
+    const int32_t* desc, const int64_t* group_ptr, const int64_t* group_source, const int64_t* group_order,
+    int64_t n_nodes, int64_t n_edges, int64_t n_groups, int64_t K, int64_t wc, int64_t wr, int64_t pa, int64_t pt,
+    int64_t n_blocks, int64_t d_out, int64_t n_heads, int64_t h_stride, int64_t rows_stride, float* rows_g,
+    void* stream) {
+  return gm::forward_grouped(false, h_g, z, node_stride, t_stride, width, n_runs, phase_g, rho_g, zw_g, desc,
+                             group_ptr, group_source, group_order, n_nodes, n_edges, n_groups, K, wc, wr, pa, pt,
+                             n_blocks, d_out, nullptr, nullptr, nullptr, 0, 0.0, rows_g, stream,
+                             gm::HeadStrides{n_heads, h_stride, rows_stride, 0, 0});
+}
+
+extern "C" int gm_factored_backward_heads_f32(
+    const float* g, int64_t g_ld, const int64_t* target_g, const float* weights_g, const float* rows_g,
+    const float* h_g, const float* const* z, float* const* dz, const int64_t* node_stride, const int64_t* t_stride,
+    const int64_t* width, int64_t n_runs, const float* phase_g, const float* rho_g, const float* zw_g,
+    const int32_t* desc, const int64_t* group_ptr, const int64_t* group_source, const int64_t* group_order,
+    int64_t n_nodes, int64_t n_edges, int64_t n_groups, int64_t K, int64_t wc, int64_t wr, int64_t pa, int64_t pt,
+    int64_t n_blocks, int64_t d_out, int64_t n_heads, int64_t g_stride, int64_t weights_stride, int64_t rows_stride,
+    int64_t h_stride, int64_t accumulate, float* dh_g, float* dweights_g, void* stream) {
+  return gm::backward_grouped(false, g, g_ld, target_g, weights_g, rows_g, h_g, z, dz, node_stride, t_stride, width,
+                              n_runs, phase_g, rho_g, zw_g, desc, group_ptr, group_source, group_order, n_nodes,
+                              n_edges, n_groups, K, wc, wr, pa, pt, n_blocks, d_out, nullptr, nullptr, nullptr, 0, 0.0,
+                              accumulate, dh_g, dweights_g, stream,
+                              gm::HeadStrides{n_heads, h_stride, rows_stride, weights_stride, g_stride});
 }
 
 extern "C" int gm_factored_backward_grouped_f32(

@@ -76,6 +76,8 @@ SIGNATURES_F32 = {
                                          + [_I] + [_P] * 3),
     "gm_factored_backward_grouped_ld_f32": (ctypes.c_int, [_P, _I] + [_P] * 9 + [_I] + [_P] * 7 + [_I] * 10
                                             + [_P] * 3 + [_I, _D] + [_I] + [_P] * 3),
+    "gm_factored_forward_heads_f32": (ctypes.c_int, [_P] * 5 + [_I] + [_P] * 7 + [_I] * 13 + [_P, _P]),
+    "gm_factored_backward_heads_f32": (ctypes.c_int, [_P, _I] + [_P] * 9 + [_I] + [_P] * 7 + [_I] * 16 + [_P] * 3),
     "gm_factored_aggregate_gather_f32": (ctypes.c_int, [_P] * 4 + [_I] * 3 + [_P, _P]),
     "gm_factored_lane_tables": (ctypes.c_int, [_P] + [_I] * 6 + [_P] * 3),
     "gm_factored_lanes_fixed": (ctypes.c_int, [_P] + [_I] * 6 + [_P]),
@@ -765,10 +767,15 @@ def _index_vector(t: Tensor, n: int | None, name: str, dtype: torch.dtype = torc
                          + (f" of {n} entries" if n is not None else ""))
 
 
-def _edge_stream(t: Tensor | None, n_edges: int, width: int, name: str) -> None:
-    """A per-edge stream in the grouping's order: contiguous (n_edges, width) (or (n_edges,) for width 1)."""
+def _edge_stream(t: Tensor | None, n_edges: int, width: int, name: str, heads: int | None = None) -> None:
+    """A per-edge stream in the grouping's order: contiguous (n_edges, width) (or (n_edges,) for width 1);
+    with ``heads`` one of these for each head, contiguous in itself, the heads further apart."""
     if t is None:
         return
+    if heads is not None:
+        if t.dim() != (2 if width == 1 else 3) or t.shape[0] != heads or (heads > 1 and t.stride(0) < n_edges * width):
+            raise ValueError(f"{name} must hold {heads} heads' ({n_edges}, {width}) streams one after the other")
+        t = t[0]
     shape = (n_edges,) if width == 1 else (n_edges, width)
     if tuple(t.shape) != shape or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous {shape} tensor")
@@ -818,8 +825,14 @@ def factored_forward_grouped(h_g: Tensor | None, runs: MixRuns, n_nodes: int, ph
     (into ``out`` (n_edges, d_out) when given).  With ``trunk`` the kernels
     evaluate h from ``rho_g`` and ``h_g`` may be None.  A bfloat16 ``h_g``
     gives bfloat16 rows (plans with compiled-in lane slots, :func:`lanes_fixed`;
-    float32 arithmetic)."""
+    float32 arithmetic).  A float32 ``h_g (H, n_edges, 16)`` runs H heads in
+    one launch into ``out (H, n_edges, d_out)`` (the heads of either may be
+    further apart), their mixes H to a node: the runs' node strides then step
+    over one head."""
     n_edges = rho_g.shape[0]
+    if h_g is not None and h_g.dim() == 3:
+        return _forward_heads(h_g, runs, n_nodes, phase_g, rho_g, zw_g, pa, pt, desc, group_ptr, group_source,
+                              group_order, K, wc, wr, d_out, out, trunk)
     if h_g is None and trunk is None:
         raise ValueError("h_g is required without a fused trunk")
     b16 = h_g is not None and h_g.dtype == torch.bfloat16
@@ -851,6 +864,65 @@ def factored_forward_grouped(h_g: Tensor | None, runs: MixRuns, n_nodes: int, ph
     return out
 
 
+def _forward_heads(h_g: Tensor, runs: MixRuns, n_nodes: int, phase_g: Tensor, rho_g: Tensor, zw_g: Tensor | None,
+                   pa: int, pt: int, desc: Tensor, group_ptr: Tensor, group_source: Tensor,
+                   group_order: Tensor | None, K: int, wc: int, wr: int, d_out: int, out: Tensor | None,
+                   trunk: FusedTrunk | None) -> Tensor:
+    n_edges, heads = rho_g.shape[0], h_g.shape[0]
+    _check(trunk is None and h_g.dtype == torch.float32, "several heads a launch take float32 trunk features")
+    if out is None:
+        out = torch.empty(heads, n_edges, d_out, dtype=torch.float32, device=rho_g.device)
+    _check(out.dtype == torch.float32, "out must be float32")
+    if n_edges == 0 or heads == 0:
+        return out
+    _grouping(group_ptr, group_source, group_order)
+    _edge_stream(h_g, n_edges, 16, "h_g", heads)
+    _edge_stream(out, n_edges, d_out, "out", heads)
+    _edge_stream(rho_g, n_edges, 1, "rho_g")
+    hd = host_desc32(desc)
+    _call("gm_factored_forward_heads_f32", _ptr(h_g), ctypes.cast(runs.z, ctypes.c_void_p),
+          ctypes.cast(runs.node_stride, ctypes.c_void_p), ctypes.cast(runs.t_stride, ctypes.c_void_p),
+          ctypes.cast(runs.width, ctypes.c_void_p), runs.n, _ptr(phase_g), _ptr(rho_g), _ptr(zw_g), hd.data_ptr(),
+          _ptr(group_ptr), _ptr(group_source), _ptr(group_order), n_nodes, n_edges, group_source.shape[0], K, wc,
+          wr, pa, pt, hd.shape[0], d_out, heads, h_g.stride(0), out.stride(0), _ptr(out), _stream(rho_g.device))
+    return out
+
+
+def _backward_heads(g: Tensor, target_g: Tensor, weights_g: Tensor, rows_g: Tensor, h_g: Tensor, runs: MixRuns,
+                    n_nodes: int, phase_g: Tensor, rho_g: Tensor, zw_g: Tensor | None, pa: int, pt: int, desc: Tensor,
+                    group_ptr: Tensor, group_source: Tensor, group_order: Tensor | None, K: int, wc: int, wr: int,
+                    dh_g: Tensor, dweights: Tensor | None, trunk: FusedTrunk | None, accumulate: bool) -> Tensor:
+    n_edges, heads, d_out = rho_g.shape[0], h_g.shape[0], g.shape[-1]
+    _check(trunk is None and all(t.dtype == torch.float32 for t in (g, weights_g, rows_g, h_g, dh_g)),
+           "several heads a launch take float32 streams")
+    if dweights is None:
+        dweights = torch.empty_like(weights_g)
+    if n_edges == 0 or heads == 0:
+        return dweights
+    _grouping(group_ptr, group_source, group_order)
+    _index_vector(target_g, n_edges, "target_g")
+    for t, width, name in ((weights_g, 1, "weights_g"), (rows_g, d_out, "rows_g"), (h_g, 16, "h_g"),
+                           (dh_g, 16, "dh_g"), (dweights, 1, "dweights")):
+        _edge_stream(t, n_edges, width, name, heads)
+    _check(heads == 1 or (dh_g.stride(0) == h_g.stride(0) and dweights.stride(0) == weights_g.stride(0)),
+           "dh and dweights must lie as h and the weights do")
+    _edge_stream(rho_g, n_edges, 1, "rho_g")
+    _check(g.dim() == 3 and g.shape[0] == heads, "g must be (heads, n_targets, d_out)")
+    # a head's gradient rows read in place (rows g.stride(1) floats apart) where the kernels' 8-byte reads allow
+    if g.stride(2) != 1 or g.stride(1) < d_out or g.stride(0) % 2 or (
+            g.stride(1) != d_out and (g.stride(1) % 2 or g.data_ptr() % 8)):
+        g = g.contiguous()
+    hd = host_desc32(desc)
+    _call("gm_factored_backward_heads_f32", _ptr(g), g.stride(1), _ptr(target_g), _ptr(weights_g), _ptr(rows_g),
+          _ptr(h_g), ctypes.cast(runs.z, ctypes.c_void_p), ctypes.cast(runs.dz, ctypes.c_void_p),
+          ctypes.cast(runs.node_stride, ctypes.c_void_p), ctypes.cast(runs.t_stride, ctypes.c_void_p),
+          ctypes.cast(runs.width, ctypes.c_void_p), runs.n, _ptr(phase_g), _ptr(rho_g), _ptr(zw_g), hd.data_ptr(),
+          _ptr(group_ptr), _ptr(group_source), _ptr(group_order), n_nodes, n_edges, group_source.shape[0], K,
+          wc, wr, pa, pt, hd.shape[0], d_out, heads, g.stride(0), weights_g.stride(0), rows_g.stride(0),
+          h_g.stride(0), int(accumulate), _ptr(dh_g), _ptr(dweights), _stream(rho_g.device))
+    return dweights
+
+
 def factored_backward_grouped(g: Tensor, target_g: Tensor, weights_g: Tensor, rows_g: Tensor, h_g: Tensor | None,
                               runs: MixRuns, n_nodes: int, phase_g: Tensor, rho_g: Tensor, zw_g: Tensor | None,
                               pa: int, pt: int, desc: Tensor, group_ptr: Tensor, group_source: Tensor,
@@ -865,9 +937,15 @@ def factored_backward_grouped(g: Tensor, target_g: Tensor, weights_g: Tensor, ro
     ``rho_g`` and ``h_g`` may be None.  ``accumulate``: dh and dweights are
     added to ``dh_g`` and ``dweights`` (which must then be given) instead of
     written.  With bfloat16 ``h_g`` the rows and ``dh_g`` are bfloat16 too
-    (float32 arithmetic)."""
+    (float32 arithmetic).  A float32 ``h_g (H, n_edges, 16)`` runs H heads in
+    one launch, every other per-edge stream and ``g (H, n_targets, d_out)``
+    with the heads leading (further apart where they are views), the mixes as
+    in :func:`factored_forward_grouped`."""
     if accumulate and dweights is None:
         raise ValueError("accumulate needs the dweights to add to")
+    if h_g is not None and h_g.dim() == 3:
+        return _backward_heads(g, target_g, weights_g, rows_g, h_g, runs, n_nodes, phase_g, rho_g, zw_g, pa, pt, desc,
+                               group_ptr, group_source, group_order, K, wc, wr, dh_g, dweights, trunk, accumulate)
     if h_g is None and trunk is None:
         raise ValueError("h_g is required without a fused trunk")
     if dweights is None:

@@ -908,10 +908,13 @@ class FactoredHeads(torch.autograd.Function):
         return (dh, dalpha, None, *dmixes)
 
 
-def _heads_runs(meta: dict, mixes: tuple[Tensor, ...], head: int, grads: list[Tensor] | None) -> _native.MixRuns:
+def _heads_runs(meta: dict, mixes: tuple[Tensor, ...], head: int, grads: list[Tensor] | None,
+                step: int | None = None) -> _native.MixRuns:
     """Head ``head``'s mix runs in packed-column order: every input
-    frequency's complex columns, then the real block's."""
-    K, H = meta["K"], meta["heads"]
+    frequency's complex columns, then the real block's.  With ``step`` the
+    runs of the heads ``head``, ``head + step``, ... of a launch: their node
+    strides step over ``step`` heads."""
+    K, H = meta["K"], meta["heads"] if step is None else step
     complex_runs, real_runs = [], []
     for (n, _blocks, cw, rw), mix in zip(meta["groups"], mixes, strict=True):
         C = cw + rw
@@ -993,6 +996,13 @@ def grouped_eligible(hp: HeadsPlan, h_dtype: torch.dtype, K: int) -> tuple[bool,
     return ok, pa, pt
 
 
+def _together(meta: dict, h_g: Tensor) -> bool:
+    """Whether a share of every head runs as one launch: float32 streams of
+    several heads in the default group order (the heads of a group then run
+    together, sharing its phases and targets in the caches)."""
+    return h_g.dtype == torch.float32 and h_g.shape[0] > 1 and meta["group_order"] is None
+
+
 class FactoredHeadsGrouped(torch.autograd.Function):
     """:class:`FactoredHeads` over the grouped streams: ``h_g (H, E, 16)`` in
     the grouping's order, ``alpha (E, H)`` in edge order, the mix arrays;
@@ -1007,7 +1017,15 @@ class FactoredHeadsGrouped(torch.autograd.Function):
         st: GroupedStreams = meta["streams"]
         shares = meta["heads"]
         rows = torch.empty(shares, E, meta["d_out"], dtype=h_g.dtype, device=h_g.device)
-        for v in range(shares):
+        together = _together(meta, h_g)
+        for share in range(split if together else 0):  # this share of every head in one launch
+            runs = _heads_runs(meta, mixes, share, None, split)
+            with torch.profiler.record_function("gm::kernel/pairs"):
+                _native.factored_forward_grouped(h_g, runs, meta["n_nodes"], st.phase_g, st.rho_g, st.zw_g, st.pa,
+                                                 st.pt, meta["desc"], meta["group_ptr"], meta["group_source"],
+                                                 meta["group_order"], meta["K"], meta["wc"], meta["wr"],
+                                                 meta["d_out"], out=rows[share::split])
+        for v in range(0 if together else shares):
             runs = _heads_runs(meta, mixes, v, None)
             with torch.profiler.record_function("gm::kernel/pairs"):
                 _native.factored_forward_grouped(h_g[v // split], runs, meta["n_nodes"], st.phase_g, st.rho_g,
@@ -1034,7 +1052,16 @@ class FactoredHeadsGrouped(torch.autograd.Function):
         alpha_gt = _native.gather_transpose(alpha, st.perm)  # (H, E) in the grouping's order
         dalpha_gt = torch.empty_like(alpha_gt)
         grad = grad.contiguous()
-        for v in range(shares):
+        together = _together(meta, h_g)
+        for share in range(split if together else 0):
+            runs = _heads_runs(meta, mixes, share, dmixes, split)
+            with torch.profiler.record_function("gm::kernel/pairs_backward"):
+                _native.factored_backward_grouped(
+                    grad.transpose(0, 1)[share::split], st.target_g, alpha_gt, rows[share::split], h_g, runs,
+                    meta["n_nodes"], st.phase_g, st.rho_g, st.zw_g, st.pa, st.pt, meta["desc"], meta["group_ptr"],
+                    meta["group_source"], meta["group_order"], meta["K"], meta["wc"], meta["wr"], dh_g,
+                    dweights=dalpha_gt, accumulate=share > 0)
+        for v in range(0 if together else shares):
             head, share = divmod(v, split)
             runs = _heads_runs(meta, mixes, v, dmixes)
             # a head's shares read the same trunk features and weights: the later shares add their gradients

@@ -552,6 +552,28 @@ int gm_factored_backward_grouped_ld_bf16(const float* g, int64_t g_ld, const int
                                          int64_t n_blocks, int64_t d_out, int64_t accumulate, uint16_t* dh_g,
                                          float* dweights_g, void* stream);
 
+/* Several heads of the grouped kernels in one launch: head v of n_heads reads
+ * and writes its streams v times the strides (in elements: h and dh, the rows,
+ * the weights and dweights, g) past the pointers given, and its mixes (and
+ * their gradients) at the runs' v-th step: the runs' node strides step over
+ * one head, a node holding n_heads of them.  Otherwise as the _grouped forms
+ * without the fused trunk, head by head. */
+int gm_factored_forward_heads_f32(
+    const float* h_g, const float* const* z, const int64_t* node_stride, const int64_t* t_stride,
+    const int64_t* width, int64_t n_runs, const float* phase_g, const float* rho_g, const float* zw_g,
+    const int32_t* desc, const int64_t* group_ptr, const int64_t* group_source, const int64_t* group_order,
+    int64_t n_nodes, int64_t n_edges, int64_t n_groups, int64_t K, int64_t wc, int64_t wr, int64_t pa, int64_t pt,
+    int64_t n_blocks, int64_t d_out, int64_t n_heads, int64_t h_stride, int64_t rows_stride, float* rows_g,
+    void* stream);
+int gm_factored_backward_heads_f32(
+    const float* g, int64_t g_ld, const int64_t* target_g, const float* weights_g, const float* rows_g,
+    const float* h_g, const float* const* z, float* const* dz, const int64_t* node_stride, const int64_t* t_stride,
+    const int64_t* width, int64_t n_runs, const float* phase_g, const float* rho_g, const float* zw_g,
+    const int32_t* desc, const int64_t* group_ptr, const int64_t* group_source, const int64_t* group_order,
+    int64_t n_nodes, int64_t n_edges, int64_t n_groups, int64_t K, int64_t wc, int64_t wr, int64_t pa, int64_t pt,
+    int64_t n_blocks, int64_t d_out, int64_t n_heads, int64_t g_stride, int64_t weights_stride, int64_t rows_stride,
+    int64_t h_stride, int64_t accumulate, float* dh_g, float* dweights_g, void* stream);
+
 /* gm_factored_aggregate with edge e's row at rows[inv[e]] (rows kept in the
  * grouping's order; inv is the grouping's inverse permutation). */
 int gm_factored_aggregate_gather_f32(const float* rows, const int64_t* inv, const float* weights,
