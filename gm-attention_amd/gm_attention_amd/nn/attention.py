@@ -251,7 +251,7 @@ class _LayerForms:
             for lins in maps:
                 forms += _stacked_matrix(lins, mhsa.field_type_in, [next(groups) for _ in lins])
             m, *bias = matrix_and_bias(proj, next(groups))
-            forms += [m.index_select(0, _heads_permutation(mhsa, m.device)), *bias]
+            forms += [_projection_rows(mhsa, layout, m), *bias]
             given = []
             for r in readouts:
                 it = iter(next(groups))
@@ -264,7 +264,8 @@ class _LayerForms:
         self.served = assembly.takes(params)
         if not self.served:
             return
-        forms = iter(assembly.assembled(mhsa, f"layer {layout.split} {trunk}", params, build))
+        name = f"layer {layout.split} {layout.padded} {trunk}"
+        forms = iter(assembly.assembled(mhsa, name, params, build))
 
         def pair(lin: SO2Linear) -> tuple[Tensor, Tensor | None]:
             return next(forms), next(forms) if lin.has_bias else None
@@ -272,6 +273,14 @@ class _LayerForms:
         self.query, self.key, self.projection = pair(heads[0].query), pair(heads[0].key), pair(proj)
         self.mixing = [next(forms) for _ in layout.hp.groups]
         self.trunk = list(forms)
+
+
+def _projection_rows(mhsa: SO2MHSA, layout: fused_factored.HeadsLayout, m: Tensor) -> Tensor:
+    """The output projection's matrix with its rows in the order of the layout's
+    rows ``(N, H split, d)`` side by side, zero where they hold a padded copy."""
+    perm = _heads_permutation(mhsa, torch.device("cpu")).tolist()
+    rows = [perm[c] if c >= 0 else m.shape[0] for c in layout.columns(mhsa.heads[0].value, mhsa.num_heads)]
+    return torch.cat([m, m.new_zeros(1, m.shape[1])]).index_select(0, torch.tensor(rows, device=m.device))
 
 
 def _stacked_matrix(linears: Sequence[SO2Linear], field_type_out: SO2FieldType,
@@ -332,7 +341,7 @@ def _attend_batched_flat(mhsa: SO2MHSA, x: SO2FeatureField, edges) -> Tensor | N
         return None
     compute = torch.float32 if x.dtype == torch.bfloat16 else x.dtype
     fused_trunk = radial.eligible(values, compute, x.device)
-    layout = fused_factored.heads_layout(values, compute)
+    layout = fused_factored.heads_layout(values, compute, None, (rows.shape[0], int(edges.n_edges)), rows.device)
     forms = _LayerForms(mhsa, values, layout, fused_trunk)
     proj = mhsa.output_projection
     with torch.profiler.record_function("gm::attention/attend"):
@@ -348,8 +357,9 @@ def _attend_batched_flat(mhsa: SO2MHSA, x: SO2FeatureField, edges) -> Tensor | N
                                                forms=forms.trunk if forms.served else None)
         else:
             h, trunk = torch.stack([k._trunk_hidden(edges.distances) for k in values]), None
+        # (N, H, d), or the layout's shares' rows, which the projection's rows follow
         out = fused_factored.forward_aggregated_heads(values, x, edges, alpha, h, groups, trunk,
-                                                      forms.mixing if forms.served else None)  # (N, H, d)
+                                                      (layout, forms.mixing) if forms.served else None)
     if forms.served:
         m, bias = forms.projection
     else:

@@ -22,6 +22,7 @@ the fused path, so ``"0"`` makes them raise rather than silently run torch.
 
 from __future__ import annotations
 
+import functools
 import os
 import weakref
 from collections import OrderedDict
@@ -625,6 +626,35 @@ class SubHead:
         return self.kernel._blocks()
 
 
+class PaddedHead:
+    """The value kernel of one head with every output frequency widened to the
+    same number of copies, the added copies' blocks zero: an uneven or small
+    head in ``shares`` equal shares of four copies a frequency, the shape of
+    the lane-owned kernels' compiled-in slots.  Stands in for the kernel where
+    only the plan is read."""
+
+    def __init__(self, kernel: Any, shares: int) -> None:
+        self.kernel = kernel
+        self.field_type_in = kernel.field_type_in
+        self.field_type_out = SO2FieldType({f: 4 * shares for f in kernel.field_type_out.frequencies})
+        self._pair_powers = kernel._pair_powers
+        self.complex_head, self.real_head = kernel.complex_head, kernel.real_head
+        self.radial_basis = kernel.radial_basis
+
+    def _blocks(self) -> list[tuple[int, int, str]]:
+        return self.kernel._blocks()
+
+
+def padded_unit(kernel: Any, shares: int) -> Any:
+    """One share of ``kernel`` padded to ``shares`` shares of four copies a frequency (cached)."""
+    key = ("_padded_head", shares)
+    head = kernel.__dict__.get(key)
+    if head is None:
+        head = PaddedHead(kernel, shares)
+        kernel.__dict__[key] = head
+    return sub_head(head, shares)
+
+
 def sub_head(kernel: Any, split: int) -> Any:
     """``kernel`` itself for ``split == 1``, else its :class:`SubHead` (cached)."""
     if split == 1:
@@ -637,28 +667,35 @@ def sub_head(kernel: Any, split: int) -> Any:
     return sub
 
 
-def share_columns(kernel: Any, split: int, heads: int, device: torch.device) -> Tensor:
+def _share_index(kernel: Any, part: SO2FieldType, split: int, heads: int) -> list[int]:
+    """For column ``h d + c`` of the heads' rows ``(N, H, d)`` (each head in the
+    per-head flat layout), its column in the rows ``(N, H split, part)`` of
+    shares of ``part``'s copies each (the last ones of a padded head unused)."""
+    out = kernel.field_type_out
+    full_s, part_s = out.slices(), part.slices()
+    index = []
+    for head in range(heads):
+        for f, m in out.items():
+            dim = 1 if f == 0 else 2
+            per = part.multiplicity(f)
+            for c in range(full_s[f].stop - full_s[f].start):
+                copy, re = divmod(c, dim)
+                share, local = divmod(copy, per)
+                index.append((head * split + share) * part.dimension + part_s[f].start + local * dim + re)
+    return index
+
+
+def share_columns(kernel: Any, split: int, heads: int, device: torch.device, unit: Any = None) -> Tensor:
     """For column ``h d + c`` of the heads' rows ``(N, H, d)`` (each head in
     the per-head flat layout), its column in the shares' rows
     ``(N, H split, d / split)`` -- the gather that puts the shares' outputs
-    back side by side."""
-    key = ("_share_columns", split, heads, str(device))
+    back side by side.  ``unit``: the share of a padded head."""
+    key = ("_share_columns", split, heads, str(device), unit is None)
     cols = kernel.__dict__.get(key)
     if cols is None:
-        out = kernel.field_type_out
-        part = SO2FieldType({f: m // split for f, m in out.items()})
-        full_s, part_s = out.slices(), part.slices()
-        d_part = part.dimension
-        index = []
-        for head in range(heads):
-            for f, m in out.items():
-                dim = 1 if f == 0 else 2
-                per = m // split
-                for c in range(full_s[f].stop - full_s[f].start):
-                    copy, re = divmod(c, dim)
-                    share, local = divmod(copy, per)
-                    index.append((head * split + share) * d_part + part_s[f].start + local * dim + re)
-        cols = torch.tensor(index, dtype=torch.int64, device=device)
+        part = (SO2FieldType({f: m // split for f, m in kernel.field_type_out.items()}) if unit is None
+                else unit.field_type_out)
+        cols = torch.tensor(_share_index(kernel, part, split, heads), dtype=torch.int64, device=device)
         kernel.__dict__[key] = cols
     return cols
 
@@ -666,14 +703,19 @@ def share_columns(kernel: Any, split: int, heads: int, device: torch.device) -> 
 def _heads_mixing_from(kernels: list[Any], hp: HeadsPlan, params: list[list[Tensor | None]],
                        split: int = 1) -> list[Tensor]:
     """``heads_mixing`` from stand-in readout parameters (one list per head);
-    with ``split > 1`` the columns run over the heads' shares (head-major)."""
+    with ``split > 1`` the columns run over the heads' shares (head-major), the
+    copies a padded plan adds zero."""
     from gm_attention_amd.nn.node_products import mixing_matrix
 
     mats = []
     for n, blocks, _cw, _rw in hp.groups:
         per_share = []
         for k, pk in zip(kernels, params, strict=True):
-            weights = {b.block: k._block_weights(b.block, pk) for b in blocks}  # (b_m, a_n, K) of the full head
+            weights = {}  # (b_m, a_n, K) of the full head, padded to the shares' copies
+            for b in blocks:
+                w = k._block_weights(b.block, pk)
+                added = split * b.b_m - w.shape[0]
+                weights[b.block] = torch.cat([w, w.new_zeros(added, *w.shape[1:])]) if added > 0 else w
             for share in range(split):
                 pieces = []
                 for b in blocks:
@@ -703,7 +745,7 @@ def _mixing_maps(kernels: list[Any], hp: HeadsPlan, split: int = 1) -> dict:
     only moves and negates.  :class:`_SignedGather` keeps its gradient plan in
     the same dictionary."""
     shapes = tuple(tuple(None if p is None else tuple(p.shape) for p in k.readout_parameters()) for k in kernels)
-    key = (tuple(id(k) for k in kernels), shapes, split)
+    key = (tuple(id(k) for k in kernels), shapes, split, hp.plan.d_out)
     hit = _MIXING_MAPS.get(key)
     if hit is not None:
         return hit
@@ -798,7 +840,7 @@ def heads_mixing(kernels: list[Any], hp: HeadsPlan, split: int = 1) -> list[Tens
             return _heads_mixing_from(kernels, hp, [[None if p is None else next(it) for p in r] for r in readouts],
                                       split)
 
-        return assembly.assembled(kernels[0], f"mixing {len(kernels)} {split}", params, build)
+        return assembly.assembled(kernels[0], f"mixing {len(kernels)} {split} {hp.plan.d_out}", params, build)
     plan = _mixing_maps(kernels, hp, split)
     flat = torch.cat([p.reshape(-1) for k in kernels for p in k.readout_parameters() if p is not None])
     return list(_SignedGather.apply(flat, plan))
@@ -829,27 +871,93 @@ def heads_mixes(x: SO2FeatureField, hp: HeadsPlan, mats: list[Tensor]) -> list[T
 @dataclass(frozen=True)
 class HeadsLayout:
     """How :func:`forward_aggregated_heads` runs a layer's heads: the plan of one
-    share (``split`` shares a head; 1 and ``grouped`` False for the kernels
-    that are not grouped), the phase orders of the grouped streams."""
+    share (``unit``; ``split`` shares a head, 1 and ``grouped`` False for the
+    kernels that are not grouped; ``padded``: of the padded head), the phase
+    orders of the grouped streams."""
 
     hp: HeadsPlan
+    unit: Any
     split: int
     grouped: bool
+    padded: bool
     pa: int
     pt: int
 
+    def columns(self, kernel: Any, heads: int) -> list[int]:
+        """For every column of the rows ``(N, H split, d)`` side by side, the
+        column ``h d + c`` of the heads' rows it holds, or -1 (a padded copy)."""
+        index = _share_index(kernel, self.unit.field_type_out, self.split, heads)
+        columns = [-1] * (heads * self.split * self.hp.plan.d_out)
+        for column, at in enumerate(index):
+            columns[at] = column
+        return columns
 
-def heads_layout(kernels: list[Any], dtype: torch.dtype, K: int | None = None) -> HeadsLayout:
-    """The layout of the heads' value kernels for trunk features of ``dtype`` (K - 1 of them)."""
+
+#: Device memory the padded shares' mixes, mix gradients and rows may take (a share of the device's):
+#: an uneven layer that fits without padding still fits.
+PADDED_SHARE = 0.25
+
+
+@functools.cache
+def _device_memory(index: int) -> int:
+    return torch.cuda.get_device_properties(index).total_memory
+
+
+def _padded_shares(kernel: Any, split: int, K: int, heads: int, size: tuple[int, int] | None,
+                   device: torch.device) -> int:
+    """Into how many padded shares of four copies a frequency each head goes, or
+    0 where its own plan (``split`` shares) is the better one.
+
+    The estimates are microseconds of one forward and backward launch of 6
+    heads over 0.75 M edges (45x91, B = 3): compiled-in slots 250 + 89 a
+    16-column tile (3 tiles 517, 7 tiles 872), runtime slots 400 a tile (5:
+    1,800, 8: 3,535), the generic kernels 650 a tile (3: 1,950, 4: 2,290, 7:
+    4,640).  ``size`` is (nodes, edges): the padding's memory is bounded."""
+    env = (os.environ.get("GM_FACTORED_LANES", "1"), os.environ.get("GM_FACTORED_STATIC", "1"))
+    key = ("_padded_shares", split, K, env)
+    held = kernel.__dict__.get(key)
+    if held is None:
+        held = (0, 0, 0)
+        out = kernel.field_type_out
+        shares = -(-max(out.multiplicities) // 4)
+        unit = padded_unit(kernel, shares)
+        hp = heads_plan(unit)
+        ok, pa, pt = grouped_eligible(hp, torch.float32, K)
+        own = sub_head(kernel, max(split, 1))
+        own_hp = heads_plan(own)
+        own_ok, own_pa, own_pt = grouped_eligible(own_hp, torch.float32, K)
+        if ok and _lanes_fixed(unit, hp, pa, pt) and not (own_ok and _lanes_fixed(own, own_hp, own_pa, own_pt)):
+            tiles = lambda p: -(-(2 * p.wc + p.wr) // 16)  # noqa: E731
+            lanes = own_ok and _lanes_apply(own, own_hp, own_pa, own_pt)
+            if shares * (250 + 89 * tiles(hp.plan)) < max(split, 1) * (400 if lanes else 650) * tiles(own_hp.plan):
+                held = (shares, hp.plan.d_out, 2 * hp.plan.wc + hp.plan.wr)
+        kernel.__dict__[key] = held
+    shares, d_out, C = held
+    if not shares or size is None or device.type != "cuda":
+        return 0
+    nodes, edges = size
+    taken = 4 * heads * shares * (edges * d_out + 2 * nodes * K * C)
+    return shares if taken <= PADDED_SHARE * _device_memory(device.index or 0) else 0
+
+
+def heads_layout(kernels: list[Any], dtype: torch.dtype, K: int | None = None, size: tuple[int, int] | None = None,
+                 device: torch.device | None = None) -> HeadsLayout:
+    """The layout of the heads' value kernels for trunk features of ``dtype`` (K
+    - 1 of them); with ``size`` (nodes, edges) heads that the compiled-in lane
+    slots do not serve as they are may be padded to a shape they do
+    (:func:`_padded_shares`)."""
     if K is None:
         first = kernels[0]
         K = (first.complex_head if first.complex_head is not None else first.real_head).in_features + 1
     split = head_split(kernels[0], K) if dtype == torch.float32 else 0
-    hp = heads_plan(sub_head(kernels[0], max(split, 1)))
+    shares = (_padded_shares(kernels[0], split, K, len(kernels), size, device)
+              if dtype == torch.float32 and size is not None and device is not None else 0)
+    unit = padded_unit(kernels[0], shares) if shares else sub_head(kernels[0], max(split, 1))
+    hp = heads_plan(unit)
     ok, pa, pt = grouped_eligible(hp, dtype, K)
-    if ok and split:
-        return HeadsLayout(hp, split, True, pa, pt)
-    return HeadsLayout(heads_plan(kernels[0]), 1, False, pa, pt)
+    if ok and (shares or split):
+        return HeadsLayout(hp, unit, shares or split, True, shares > 0, pa, pt)
+    return HeadsLayout(heads_plan(kernels[0]), kernels[0], 1, False, False, pa, pt)
 
 
 def mixing_forms(kernels: list[Any], layout: HeadsLayout, params: list[list[Tensor | None]]) -> list[Tensor]:
@@ -1199,10 +1307,10 @@ def head_split(kernel: Any, K: int) -> int:
 
 def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any, alpha: Tensor, h: Tensor | None,
                              groups: tuple[Tensor, Tensor, Tensor], trunk=None,
-                             mats: list[Tensor] | None = None) -> Tensor:
-    """Every head's ``forward_factored_aggregated`` at once: ``(N, H, d_out)``
-    (``mats``: the heads' mixing matrices for their :func:`heads_layout`, formed
-    here when not given).
+                             forms: tuple[HeadsLayout, list[Tensor]] | None = None) -> Tensor:
+    """Every head's ``forward_factored_aggregated`` at once: ``(N, H, d_out)``.
+    With ``forms``, the heads' :func:`heads_layout` and their mixing matrices
+    for it, the layout's own rows ``(N, H split, d)`` (:meth:`HeadsLayout.columns`).
 
     ``h`` is every head's trunk features in edge order; alternatively
     ``trunk(rho, dtype)`` computes them from ``rho = d / cutoff`` in whatever
@@ -1214,20 +1322,21 @@ def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any,
     K = (h.shape[2] if h is not None else kernels[0].complex_head.in_features) + 1
     # bfloat16 rows: the node mixes read them as they are, everything after runs in float32
     dtype = h.dtype if h is not None else (torch.float32 if x.dtype == torch.bfloat16 else x.dtype)
-    layout = heads_layout(kernels, dtype, K)
-    hp, split, pa, pt = layout.hp, layout.split, layout.pa, layout.pt
-    if mats is None:
-        mats = heads_mixing(kernels, hp, split)
+    if forms is None:
+        layout = heads_layout(kernels, dtype, K, (x.batch_shape[0], int(edges.n_edges)), x.device)
+        mats = heads_mixing(kernels, layout.hp, layout.split)
+    else:
+        layout, mats = forms
+    hp, unit, split, pa, pt = layout.hp, layout.unit, layout.split, layout.pa, layout.pt
     mixes = heads_mixes(x, hp, mats)
     if layout.grouped:
         p = hp.plan
-        unit = sub_head(kernels[0], split)
         order, group_ptr, group_source = groups
         st = grouped_streams(edges, order, kernels[0].radial_basis.cutoff, pa, pt, dtype)
         fused = (FUSED_TRUNK and split == 1 and len(kernels) <= 8 and trunk is not None
-                 and _lanes_apply(kernels[0], hp, pa, pt))
-        b16 = (BF16_STREAMS and not fused and trunk is not None and x.dtype == torch.bfloat16
-               and _lanes_fixed(kernels[0], hp, pa, pt))
+                 and not layout.padded and _lanes_apply(kernels[0], hp, pa, pt))
+        b16 = (BF16_STREAMS and not fused and not layout.padded and trunk is not None
+               and x.dtype == torch.bfloat16 and _lanes_fixed(kernels[0], hp, pa, pt))
         h_g = None if fused else (trunk(st.rho_g, torch.bfloat16 if b16 else None) if trunk is not None
                                   else h.index_select(1, st.perm))
         if st.group_order is None and os.environ.get("GM_FACTORED_LPT", "0") == "1":
@@ -1248,10 +1357,10 @@ def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any,
             meta.update(centers=centers, centers_t=rb.centers.contiguous(), width=float(rb.width))
             return FactoredHeadsTrunk.apply(w, b, alpha.to(dtype).contiguous(), meta, *mixes)
         out = FactoredHeadsGrouped.apply(h_g.contiguous(), alpha.to(dtype).contiguous(), meta, *mixes)
-        if split == 1:
+        if forms is not None or (split == 1 and not layout.padded):
             return out
         n = out.shape[0]
-        cols = share_columns(kernels[0], split, len(kernels), out.device)
+        cols = share_columns(kernels[0], split, len(kernels), out.device, unit if layout.padded else None)
         return out.reshape(n, -1).index_select(1, cols).reshape(n, len(kernels), -1)
     if h is None:
         h = trunk((edges.distances / kernels[0].radial_basis.cutoff).to(dtype).contiguous())
