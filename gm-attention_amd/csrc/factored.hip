@@ -2990,8 +2990,10 @@ int prepare_grouped(FactArgs<float>& a, const float* h, const Runs<float>& runs,
                     int64_t pt, int64_t n_blocks, int64_t d_out, const TrunkParams& trunk) {
   GM_REQUIRE(pa >= 1 && pt >= 1 && pa + pt <= kPhaseRow / 2, "the grouped phase rows hold at most 8 pairs");
   const bool fused = trunk.w != nullptr;
-  // under the fused trunk h is never read: rho_g stands in for prepare's pointer check
-  const int status = prepare(a, fused ? rho_g : h, runs, phase_g, phase_g, rho_g, desc, group_ptr /* order unused */,
+  // under the fused trunk h is never read, nor are the phase rows by the compiled-in slots (need_phases):
+  // rho_g stands in for prepare's pointer checks
+  const float* phases = phase_g != nullptr ? phase_g : rho_g;
+  const int status = prepare(a, fused ? rho_g : h, runs, phases, phases, rho_g, desc, group_ptr /* order unused */,
                              group_ptr, group_source, n_nodes, n_edges, n_groups, K, wc, wr, pa > pt ? pa : pt,
                              n_blocks, d_out);
   if (status != GM_OK) return status;
@@ -3014,7 +3016,7 @@ int prepare_grouped(FactArgs<float>& a, const float* h, const Runs<float>& runs,
     const Block& d = a.desc[b];
     GM_REQUIRE(std::abs(d.ang) < pa && std::abs(d.tr) < pt, "a block's harmonic order exceeds the grouped phase rows");
   }
-  if (n_edges > 0) GM_REQUIRE((fused || (h && aligned(h, 16))) && phase_g && aligned(phase_g, 16) && rho_g,
+  if (n_edges > 0) GM_REQUIRE((fused || (h && aligned(h, 16))) && aligned(phase_g, 16) && rho_g,
                               "h and the phase rows must be 16-byte aligned device pointers");
   a.phase_g = phase_g;
   a.rho_g = rho_g;
@@ -3112,6 +3114,14 @@ GM_FACT_EXPORTS(double, f64)
 namespace gm {
 namespace {
 
+// The phase rows may be null where the compiled-in slots serve the call (they
+// read the zw rows); every other kernel reads them.
+int need_phases(const FactArgs<float>& a) {
+  GM_REQUIRE(a.phase_g != nullptr || fixed_slots(a),
+             "this plan's kernels read the phase rows: phase_g must be a device pointer");
+  return GM_OK;
+}
+
 // Several heads in one launch (FactArgs::n_heads); one head by default.
 struct HeadStrides {
   int64_t n = 1, h = 0, rows = 0, w = 0, g = 0;
@@ -3157,6 +3167,8 @@ int forward_grouped(bool b16, const float* h_g, const float* const* z, const int
   if (heads_status != GM_OK) return heads_status;
   GM_REQUIRE(zw_g == nullptr || gm::aligned(zw_g, 16), "zw_g must be a 16-byte aligned device pointer (or null)");
   a.zw_g = zw_g;
+  const int phases_status = need_phases(a);
+  if (phases_status != GM_OK) return phases_status;
   a.b16 = b16;
   if (b16) GM_REQUIRE(fixed_slots(a), "bfloat16 streams take plans with compiled-in lane slots (gm_factored_lanes_fixed)");
   gm::launch_grouped(true, a, (hipStream_t)stream);
@@ -3202,6 +3214,8 @@ int backward_grouped(bool b16, const float* g, int64_t g_ld, const int64_t* targ
   a.dweights = dweights_g;
   a.accumulate = accumulate != 0;
   GM_REQUIRE(!(a.accumulate && trunk_w), "the fused trunk's backward writes dh_g and dweights_g (no accumulate)");
+  const int phases_status = need_phases(a);
+  if (phases_status != GM_OK) return phases_status;
   a.b16 = b16;
   if (b16) GM_REQUIRE(fixed_slots(a), "bfloat16 streams take plans with compiled-in lane slots (gm_factored_lanes_fixed)");
   gm::launch_grouped(false, a, (hipStream_t)stream);

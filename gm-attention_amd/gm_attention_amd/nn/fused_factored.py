@@ -1045,51 +1045,75 @@ class GroupedStreams:
     """An edge set's per-edge streams in the order of its source grouping:
     ``perm`` (= the grouping's order), its inverse ``inv``, ``rho_g``, the
     phase rows ``phase_g (E, 8, 2)`` (angular orders ``0..pa-1`` then
-    transport orders ``0..pt-1``) and ``target_g``."""
+    transport orders ``0..pt-1``; None for plans whose kernels read only
+    ``zw_g``) and ``target_g``."""
 
     perm: Tensor
     inv: Tensor
     rho_g: Tensor
-    phase_g: Tensor
+    phase_g: Tensor | None
     target_g: Tensor
     pa: int
     pt: int
     zw_g: Tensor | None = None  # (E, 4): r e^{i phi}, e^{i gamma} (order-1 phases) in grouping order
     group_order: Tensor | None = None
 
+    def bytes(self) -> int:
+        """Device memory of the streams (``perm`` is the grouping's own)."""
+        held = (self.inv, self.rho_g, self.phase_g, self.target_g, self.zw_g)
+        return sum(t.numel() * t.element_size() for t in held if t is not None)
+
 
 _STREAMS: OrderedDict[tuple, tuple[Any, GroupedStreams]] = OrderedDict()
+#: Streams kept whatever they take; beyond these many, the least recently used
+#: go once they all take more than this share of the device's memory.  (A model
+#: of two stages has six edge sets with streams: with three hierarchies in turn
+#: a bound of eight sets alone rebuilt them on every pass, 80 of 243 ms.)
+STREAMS_KEPT, STREAMS_SHARE = 8, 0.125
 
 
-def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, dtype: torch.dtype) -> GroupedStreams:
-    """The grouped streams of ``edges`` under ``order``, cached while the edge set lives."""
+def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, dtype: torch.dtype,
+                    phases: bool = True) -> GroupedStreams:
+    """The grouped streams of ``edges`` under ``order`` (with the phase rows
+    only where ``phases``), cached while the edge set lives."""
     key = (id(edges.edge_index), edges.edge_index.data_ptr(), int(edges.n_edges), order.data_ptr(), float(cutoff), pa,
-           pt, dtype)
+           pt, dtype, phases)
     hit = _STREAMS.get(key)
     if hit is not None and hit[0]() is edges.edge_index:
+        try:
+            _STREAMS.move_to_end(key)
+        except KeyError:  # dropped by another thread meanwhile
+            pass
         return hit[1]
     with torch.profiler.record_function("gm::kernel/group_streams"):
         perm = order
         inv = torch.empty_like(perm)
         inv[perm] = torch.arange(perm.shape[0], device=perm.device)
         rho_g = (edges.distances.index_select(0, perm) / cutoff).to(dtype).contiguous()
-        ang = torch.view_as_real(edges.angular_phases[:, :pa].index_select(0, perm))
-        tra = torch.view_as_real(edges.transport_phases[:, :pt].index_select(0, perm))
-        phase_g = torch.zeros(perm.shape[0], 8, 2, dtype=dtype, device=perm.device)
-        phase_g[:, :pa] = ang.to(dtype)
-        phase_g[:, pa:pa + pt] = tra.to(dtype)
+        phase_g = None
+        if phases:
+            ang = torch.view_as_real(edges.angular_phases[:, :pa].index_select(0, perm))
+            tra = torch.view_as_real(edges.transport_phases[:, :pt].index_select(0, perm))
+            phase_g = torch.zeros(perm.shape[0], 8, 2, dtype=dtype, device=perm.device)
+            phase_g[:, :pa] = ang.to(dtype)
+            phase_g[:, pa:pa + pt] = tra.to(dtype)
         # r e^{i phi} and e^{i gamma}: every block factor is a product of their powers
         r64 = edges.distances.index_select(0, perm).double() / cutoff
         a1 = edges.angular_phases[:, 1].index_select(0, perm).to(torch.complex128) * r64
         t1 = edges.transport_phases[:, 1].index_select(0, perm).to(torch.complex128)
         zw_g = torch.stack([a1.real, a1.imag, t1.real, t1.imag], dim=1).to(dtype).contiguous()
-        streams = GroupedStreams(perm, inv, rho_g, phase_g.contiguous(),
-                                 edges.target_index.index_select(0, perm).contiguous(), pa, pt, zw_g)
-    for stale in [k for k, (ref, _) in _STREAMS.items() if ref() is None]:
-        del _STREAMS[stale]
+        streams = GroupedStreams(perm, inv, rho_g, phase_g, edges.target_index.index_select(0, perm).contiguous(), pa,
+                                 pt, zw_g)
+    for stale in [k for k, (ref, _) in list(_STREAMS.items()) if ref() is None]:
+        _STREAMS.pop(stale, None)
     _STREAMS[key] = (weakref.ref(edges.edge_index), streams)
-    while len(_STREAMS) > 8:
-        _STREAMS.popitem(last=False)
+    held = [s for _, s in list(_STREAMS.values()) if s.inv.device == perm.device]
+    taken = sum(s.bytes() for s in held)
+    most = STREAMS_SHARE * _device_memory(perm.device.index or 0) if perm.is_cuda else 0.0
+    while len(_STREAMS) > STREAMS_KEPT and taken > most:
+        _, (_, dropped) = _STREAMS.popitem(last=False)
+        if dropped.inv.device == perm.device:
+            taken -= dropped.bytes()
     return streams
 
 
@@ -1332,11 +1356,12 @@ def forward_aggregated_heads(kernels: list[Any], x: SO2FeatureField, edges: Any,
     if layout.grouped:
         p = hp.plan
         order, group_ptr, group_source = groups
-        st = grouped_streams(edges, order, kernels[0].radial_basis.cutoff, pa, pt, dtype)
+        fixed = _lanes_fixed(unit, hp, pa, pt)
+        st = grouped_streams(edges, order, kernels[0].radial_basis.cutoff, pa, pt, dtype, not fixed)
         fused = (FUSED_TRUNK and split == 1 and len(kernels) <= 8 and trunk is not None
                  and not layout.padded and _lanes_apply(kernels[0], hp, pa, pt))
         b16 = (BF16_STREAMS and not fused and not layout.padded and trunk is not None
-               and x.dtype == torch.bfloat16 and _lanes_fixed(kernels[0], hp, pa, pt))
+               and x.dtype == torch.bfloat16 and fixed)
         h_g = None if fused else (trunk(st.rho_g, torch.bfloat16 if b16 else None) if trunk is not None
                                   else h.index_select(1, st.perm))
         if st.group_order is None and os.environ.get("GM_FACTORED_LPT", "0") == "1":

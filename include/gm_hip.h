@@ -485,7 +485,10 @@ int gm_factored_backward_seg_f64(const double* g, const int64_t* target, const d
  * may be NULL (the reference's separate trunk, nn/kernels.py:191-231,
  * 605-607, then never writes h).  Plans that take the generic grouped kernels
  * are rejected under it (gm_factored_lane_tables reports which).  dh_g is
- * still written by the backward. * accumulate != 0: dh_g and dweights_g are added to (the shares of one head's
+ * still written by the backward.
+ * phase_g may be NULL where compiled-in lane slots serve the plan
+ * (gm_factored_lanes_fixed) and zw_g is given: those kernels read only zw_g.
+ * accumulate != 0: dh_g and dweights_g are added to (the shares of one head's
  * output copies, run one launch each, read the same trunk features and weights)
  * instead of written.
  */
