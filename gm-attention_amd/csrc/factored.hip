@@ -335,7 +335,7 @@ struct AggHeadsArgs {
 
 constexpr int kAggStep = 4;  // edges a step: 55 VGPRs, eight waves a SIMD (eight a step: five waves, 10.4 vs 9.0 ms at NS)
 
-// One wave per target, lane l owning the 16-byte pieces l, l + 64, ...,
+// One wave per target (or four, below), lane l owning the 16-byte pieces l, l + 64, ...,
 // l + 64 (P - 1) of the target's H d_out outputs (piece o: row head o / q4,
 // columns 4 (o % q4) ..).  The rows are read in the CSR's edge order, so the
 // sums are each head's sums in that order.  The target is wave-uniform, so the
@@ -346,12 +346,26 @@ constexpr int kAggStep = 4;  // edges a step: 55 VGPRs, eight waves a SIMD (eigh
 
 // B16: the rows are bfloat16 (four to an 8-byte piece, widened exactly), the
 // sums float32.
-template <int P, bool B16 = false>
+//
+// WPT: waves a target.  One, or a workgroup's four, each summing a quarter of the
+// target's edges (whole steps), the quarters added in order through LDS.  Small
+// launches are bound by their longest rows -- a polar target's edges are one
+// wave's serial chain of loads -- and take four: 32x64, B = 1, four heads 99 ->
+// 31 us; 64x128, B = 1, eight heads 322 -> 128; 181x360, B = 1 1573 -> 1108.  Once
+// the launch fills the chip for many rows' time the bytes bound it (4.4-5.0 TB/s)
+// and the split only adds its start and its sum: 131,072 targets of 40 pieces
+// 2.10 ms with one wave, 2.16 with four (B = 4 of 128x256), 2.15 and 2.35 (B = 1
+// of 256x512); 65,536 of 80 pieces 2.12 and 2.27.  The line between lies between
+// 65,536 and 131,072 targets of 40 pieces.
+constexpr int64_t kAggWidePieces = int64_t(7) << 19;
+template <int P, bool B16 = false, int WPT = 1>
 __global__ __launch_bounds__(256) void aggregate_heads_vec_kernel(AggHeadsArgs a) {
-  const int64_t i = xcd_balanced_block(blockIdx.x, gridDim.x, a.row_ptr, a.n_targets, kWavesPerBlock) * kWavesPerBlock +
-                    __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int kPerBlock = kWavesPerBlock / WPT;  // targets a workgroup
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t i = xcd_balanced_block(blockIdx.x, gridDim.x, a.row_ptr, a.n_targets, kPerBlock) * kPerBlock +
+                    (WPT == 1 ? wv : 0);
   const int lane = threadIdx.x & 63;
-  if (i >= a.n_targets) return;
+  if (i >= a.n_targets) return;  // with WPT > 1 the whole workgroup
   const int q4 = a.d_out / 4, W4 = a.H * q4, Ha = a.H / a.split;
   bool live[P];
   int ha[P];
@@ -373,7 +387,12 @@ __global__ __launch_bounds__(256) void aggregate_heads_vec_kernel(AggHeadsArgs a
       return *reinterpret_cast<const floatx4*>(a.rows + base[p] + row * a.d_out);
     }
   };
-  const int64_t e0 = a.row_ptr[i], e1 = a.row_ptr[i + 1];
+  int64_t e0 = a.row_ptr[i], e1 = a.row_ptr[i + 1];
+  if constexpr (WPT > 1) {
+    const int64_t part = (e1 - e0 + WPT * kAggStep - 1) / (WPT * kAggStep) * kAggStep;
+    e0 = e0 + wv * part < e1 ? e0 + wv * part : e1;
+    e1 = e0 + part < e1 ? e0 + part : e1;
+  }
   floatx4 s[P];
 #pragma unroll
   for (int p = 0; p < P; ++p) s[p] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -420,6 +439,18 @@ __global__ __launch_bounds__(256) void aggregate_heads_vec_kernel(AggHeadsArgs a
     for (int u = 0; u < kAggStep; ++u)
 #pragma unroll
       for (int p = 0; p < P; ++p) s[p] += w[u][p] * v[u][p];
+  }
+  if constexpr (WPT > 1) {
+    __shared__ floatx4 parts[WPT - 1][P][kWave];
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+      if (wv > 0) parts[wv - 1][p][lane] = s[p];
+    __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int w = 0; w < WPT - 1; ++w)
+#pragma unroll
+      for (int p = 0; p < P; ++p) s[p] += parts[w][p][lane];
   }
   float* o = a.out + i * (int64_t)a.H * a.d_out;
 #pragma unroll
@@ -3386,6 +3417,26 @@ extern "C" int gm_factored_lanes_fixed(const int32_t* desc, int64_t n_blocks, in
 namespace gm {
 namespace {
 
+template <int P, bool B16>
+void launch_aggregate_vec(const AggHeadsArgs& a, int64_t pieces, hipStream_t stream) {
+  if (a.n_targets <= kAggWidePieces / pieces)
+    hipLaunchKernelGGL((aggregate_heads_vec_kernel<P, B16, kWavesPerBlock>), dim3((unsigned)a.n_targets), dim3(256), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((aggregate_heads_vec_kernel<P, B16>), dim3((unsigned)blocks_for(a.n_targets)), dim3(256), 0,
+                       stream, a);
+}
+
+template <bool B16>
+void launch_aggregate(const AggHeadsArgs& a, int64_t pieces, hipStream_t stream) {
+  switch ((pieces + kWave - 1) / kWave) {
+    case 1: launch_aggregate_vec<1, B16>(a, pieces, stream); break;
+    case 2: launch_aggregate_vec<2, B16>(a, pieces, stream); break;
+    case 3: launch_aggregate_vec<3, B16>(a, pieces, stream); break;
+    default: launch_aggregate_vec<4, B16>(a, pieces, stream); break;
+  }
+}
+
 // rows float32, or bfloat16 (b16: the 16-byte-piece kernels only, as 8-byte pieces)
 int aggregate_heads(bool b16, const float* rows, const int64_t* inv, const float* alpha, const int64_t* row_ptr,
                     int64_t n_targets, int64_t n_edges, int64_t H, int64_t d_out, int64_t split, float* out,
@@ -3398,31 +3449,17 @@ int aggregate_heads(bool b16, const float* rows, const int64_t* inv, const float
   GM_REQUIRE(row_ptr && out && (n_edges == 0 || (rows && inv && alpha)),
              "rows, inv, alpha, row_ptr and out must be device pointers");
   const gm::AggHeadsArgs a{rows, alpha, inv, row_ptr, out, n_targets, n_edges, (int)H, (int)d_out, (int)split};
-  const dim3 grid((unsigned)gm::blocks_for(n_targets)), block(256);
   const int64_t pieces = d_out % 4 == 0 ? H * d_out / 4 : 0;
   const bool vec = pieces > 0 && pieces <= 64 * 4 && gm::aligned(rows, b16 ? 8 : 16) && gm::aligned(out, 16);
   if (b16) {
     GM_REQUIRE(vec, "bfloat16 rows take d_out a multiple of 4, H d_out <= 1024, 8-byte aligned rows and 16-byte aligned out");
-    if (pieces <= 64)
-      hipLaunchKernelGGL((gm::aggregate_heads_vec_kernel<1, true>), grid, block, 0, (hipStream_t)stream, a);
-    else if (pieces <= 128)
-      hipLaunchKernelGGL((gm::aggregate_heads_vec_kernel<2, true>), grid, block, 0, (hipStream_t)stream, a);
-    else if (pieces <= 192)
-      hipLaunchKernelGGL((gm::aggregate_heads_vec_kernel<3, true>), grid, block, 0, (hipStream_t)stream, a);
-    else
-      hipLaunchKernelGGL((gm::aggregate_heads_vec_kernel<4, true>), grid, block, 0, (hipStream_t)stream, a);
-    return gm::check_launch("factored_aggregate_heads");
+    launch_aggregate<true>(a, pieces, (hipStream_t)stream);
+  } else if (vec) {
+    launch_aggregate<false>(a, pieces, (hipStream_t)stream);
+  } else {
+    hipLaunchKernelGGL(gm::aggregate_heads_kernel, dim3((unsigned)gm::blocks_for(n_targets)), dim3(256), 0,
+                       (hipStream_t)stream, a);
   }
-  if (vec && pieces <= 64)
-    hipLaunchKernelGGL(gm::aggregate_heads_vec_kernel<1>, grid, block, 0, (hipStream_t)stream, a);
-  else if (vec && pieces <= 128)
-    hipLaunchKernelGGL(gm::aggregate_heads_vec_kernel<2>, grid, block, 0, (hipStream_t)stream, a);
-  else if (vec && pieces <= 192)
-    hipLaunchKernelGGL(gm::aggregate_heads_vec_kernel<3>, grid, block, 0, (hipStream_t)stream, a);
-  else if (vec)
-    hipLaunchKernelGGL(gm::aggregate_heads_vec_kernel<4>, grid, block, 0, (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(gm::aggregate_heads_kernel, grid, block, 0, (hipStream_t)stream, a);
   return gm::check_launch("factored_aggregate_heads");
 }
 
