@@ -20,9 +20,10 @@
 // works on edge c of a 16-edge tile and computes trunk features 4q..4q+3 of
 // it; the coefficient product D_m = R_m (w H~) over k-steps s = 0..4 (k =
 // 4q + s, then the bias row) leaves the lane rows 4q..4q+3 of tile m for its
-// edge: four scalar copies or one complex copy, whose message it forms at
-// once.  Forward: one wave per target node, lanes accumulate their edge
-// column's messages, a 16-lane butterfly per target.  Backward: persistent
+// edge: four scalar copies or one complex copy (the backward).  Forward: one wave
+// per target node and the product the other way round, H~^T R^T: the lane holds
+// one copy's coefficients for edges 4q..4q+3 of the tile and sums their
+// messages, two shuffles per target.  Backward: persistent
 // waves over SOURCE nodes (the transposed CSR): per edge tile the same
 // coefficients, then dC (the coefficients' gradient) and dv in registers,
 // dh~ = R^T dC on MFMA (D layout = the lane's own trunk features), and
@@ -227,116 +228,225 @@ __device__ __forceinline__ bool tile_live(const RadialConvArgs& a, int m) {
   return m < kRNS ? m < a.ns : m - kRNS < a.nc;
 }
 
-// Coefficient tile m's source values for the lane: a scalar tile's four, a
-// complex tile's pair in x and y (zeros for a dead tile or absent copies).
-__device__ __forceinline__ float4 tile_x(const RadialConvArgs& a, int m, int q, const float* vj) {
-  if (m < kRNS) {
-    const int col = 16 * m + 4 * q;
-    if (m < a.ns && col < a.a0) return *reinterpret_cast<const float4*>(vj + col);
-  } else if (m - kRNS < a.nc) {
-    const float2 x = ld2(vj + a.tile_col[m - kRNS] + 2 * q);
-    return make_float4(x.x, x.y, 0.f, 0.f);
-  }
-  return make_float4(0.f, 0.f, 0.f, 0.f);
+// ---- forward
+//
+// Edges are the product's rows: D[edge 4q + r][column c] with the copies of
+// sixteen columns, a tile a component (Ar, Ai, Br, Bi) for complex copies.  Lane
+// (q, c) then holds copy c's coefficients for edges 4q .. 4q + 3, so
+//   * its rows' loads are contiguous over the lanes: a load covers four rows'
+//     128 (complex) or 64 bytes.  With the coefficients as rows, lane (q, c) read
+//     8 bytes of edge c's row: neighbouring lanes in different rows, 64 separate
+//     pieces a load, and the vector cache's lookups bound the walk (2, 3 and 4
+//     waves a SIMD and 25% less arithmetic all took the same time);
+//   * its sums over edges are sums in the lane: ten accumulators instead of forty.
+// The edges' factors come from the wave's LDS.  256x512, B = 4, 32 + 32 + 32
+// copies: 10.4 -> 7.6 ms; 91x181, B = 1, 64 + 64 + 64 copies (two walks): 1.21 ->
+// 0.46.  What is left is latency: three waves a SIMD (166 VGPRs, three workgroups
+// of four by LDS) 7.6 ms, two 9.1, four 13.0 (spills).
+constexpr int kFGroups = kRNC / 4;       // groups of sixteen complex copies
+
+struct EdgeFactors {                     // of a wave's sixteen edges
+  float4 f[2][16];                       // per frequency: w tau, p conj(w tau)
+  int64_t row[16];                       // element offset of the source's row
+  float w[16];
+};
+
+// The edge lane (q, c) describes: edge c of the tile at frequency 1 + (q & 1).
+struct RawEdge {
+  int64_t node;
+  float w, r;
+  float2 t, p;
+};
+
+__device__ __forceinline__ RawEdge raw_edge(const RadialConvArgs& a, int64_t e, bool live, int n) {
+  RawEdge v;
+  v.node = a.source[e];
+  v.w = live ? a.weights[e] : 0.f;
+  v.r = a.rho[e];
+  v.t = ld2(a.transport + e * a.orders * 2 + 2 * n);
+  v.p = ld2(a.angular + e * a.orders * 2 + 4 * n);
+  return v;
+}
+
+// Row `row` of slot `slot`'s product tile: scalar slot m: tile m's row; complex
+// slot 4 g + p: component p of copy `row` of group g, row 4 (row % 4) + p of tile
+// 4 g + row / 4.  Returns its index over all tiles' rows, -1 for a dead tile.
+__device__ __forceinline__ int slot_row(const RadialConvArgs& a, int slot, int row) {
+  if (slot < kRNS) return slot < a.ns ? 16 * slot + row : -1;
+  const int g = (slot - kRNS) / 4, p = (slot - kRNS) % 4, m = 4 * g + row / 4;
+  return m < a.nc ? 16 * (kRNS + m) + 4 * (row % 4) + p : -1;
 }
 
 template <int NB, bool SPLIT>
-__global__ __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(SPLIT ? 4 : 1))) void
+__global__ __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(3))) void
 conv_radial_forward_kernel(RadialConvArgs a) {
-  __shared__ float rf_s[SPLIT ? 1 : kRNT * 4 * 64];
-  __shared__ __attribute__((aligned(16))) SplitTile rs_s[SPLIT ? kRNT * kWave : 1];
-  __shared__ __attribute__((aligned(16))) float bias_s[kRNT * 16];
+  // lane l of slot m: features 4 (l / 16) .. + 3 of the slot's row l % 16
+  __shared__ __attribute__((aligned(16))) float4 rf_s[SPLIT ? 1 : kRNT * kWave];
+  __shared__ __attribute__((aligned(16))) u32x4 rs_s[SPLIT ? kRNT * 2 * kWave : 1];
+  __shared__ __attribute__((aligned(16))) float4 bias_s[kRNT * 16];  // four of the same: the product starts from it
   __shared__ float w1s[16 * kRMaxBasis + 16];
-  if constexpr (SPLIT) {
-    load_split(a, rs_s);
-    load_tables(a, nullptr, nullptr, bias_s, w1s, NB);
-  } else {
-    load_tables(a, rf_s, nullptr, bias_s, w1s, NB);
+  __shared__ EdgeFactors ef_s[kRWaves];
+  for (int i = threadIdx.x; i < kRNT * kWave; i += kRThreads) {
+    const int m = i / kWave, l = i % kWave, row = slot_row(a, m, l & 15);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row >= 0) {
+      const float* r = a.rf + (row / 16 * 4) * kWave + (l & 48) + row % 16;
+      v = make_float4(r[0], r[kWave], r[2 * kWave], r[3 * kWave]);
+    }
+    if constexpr (SPLIT) {
+      const SplitA sa = split_a(v.x, v.y, v.z, v.w);
+      rs_s[2 * kWave * m + l] = sa.hm;
+      rs_s[2 * kWave * m + kWave + l] = sa.hl;
+    } else {
+      rf_s[i] = v;
+    }
+    if (l < 16) {
+      const float b = row >= 0 ? a.rbias[row] : 0.f;
+      bias_s[16 * m + l] = make_float4(b, b, b, b);
+    }
   }
+  for (int i = threadIdx.x; i < 16 * kRMaxBasis; i += kRThreads) {
+    const int t = i / kRMaxBasis, k = i % kRMaxBasis;
+    w1s[i] = k < NB ? a.w1[t * NB + k] : 0.f;
+  }
+  if (threadIdx.x < 16) w1s[16 * kRMaxBasis + threadIdx.x] = a.b1 ? a.b1[threadIdx.x] : 0.f;
   __syncthreads();
-  const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
-  const int64_t i = xcd_block(blockIdx.x, gridDim.x) * kRWaves + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4, wave = threadIdx.x >> 6;
+  const int64_t i = xcd_balanced_block(blockIdx.x, gridDim.x, a.row_ptr, a.n_nodes, kRWaves) * kRWaves + wave;
   if (i >= a.n_nodes) return;
-  float accs[kRNS][4], accc[kRNC][2];
+  EdgeFactors& ef = ef_s[wave];
+  // the lane's copy of each group: its column (a dead copy reads column 0, and is not stored) and frequency
+  int col[kFGroups], freq[kFGroups];
+  bool live_copy[kFGroups];
 #pragma unroll
-  for (int m = 0; m < kRNS; ++m) accs[m][0] = accs[m][1] = accs[m][2] = accs[m][3] = 0.f;
+  for (int g = 0; g < kFGroups; ++g) {
+    col[g] = freq[g] = 0;
+    live_copy[g] = 4 * g + (c >> 2) < a.nc;
 #pragma unroll
-  for (int m = 0; m < kRNC; ++m) accc[m][0] = accc[m][1] = 0.f;
+    for (int k = 0; k < 4; ++k)
+      if ((c >> 2) == k && live_copy[g]) {
+        col[g] = a.tile_col[4 * g + k] + 2 * (c & 3);
+        freq[g] = a.tile_n[4 * g + k] - 1;
+      }
+  }
+  const int groups = (a.nc + 3) >> 2;
+  float accs[kRNS], accc[kFGroups][2];
+#pragma unroll
+  for (int m = 0; m < kRNS; ++m) accs[m] = 0.f;
+#pragma unroll
+  for (int g = 0; g < kFGroups; ++g) accc[g][0] = accc[g][1] = 0.f;
   const int64_t e0 = a.row_ptr[i], e1 = a.row_ptr[i + 1];
   // the next tile's edge rows and sources are requested while this tile computes
-  EdgeView nxt;
-  if (e0 < e1) {
-    const int64_t e = e0 + c < e1 ? e0 + c : e0;
-    nxt = edge_view(a, e, a.source[e], e0 + c < e1);
-  }
+  const int n = 1 + (q & 1);
+  RawEdge nxt{};
+  if (e0 < e1) nxt = raw_edge(a, e0 + c < e1 ? e0 + c : e0, e0 + c < e1, n);
   for (int64_t base = e0; base < e1; base += 16) {
-    const EdgeView ev = with_radius(nxt);
+    const float r = nxt.r;
+    const float r2 = r * r, rn = n == 1 ? r2 : r2 * r2;
+    const float2 t = make_float2(nxt.w * nxt.t.x, nxt.w * nxt.t.y), p = make_float2(rn * nxt.p.x, rn * nxt.p.y);
+    wave_sync();  // the previous tile's reads are done
+    if (q < 2) ef.f[q][c] = make_float4(t.x, t.y, p.x * t.x + p.y * t.y, p.y * t.x - p.x * t.y);
+    if (q == 2) ef.row[c] = nxt.node * a.D;
+    if (q == 3) ef.w[c] = nxt.w;
+    wave_sync();
     if (base + 16 < e1) {
       const bool live = base + 16 + c < e1;
-      const int64_t e = live ? base + 16 + c : e0;
-      nxt = edge_view(a, e, a.source[e], live);
+      nxt = raw_edge(a, live ? base + 16 + c : e0, live, n);
+    }
+    const float* vr[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) vr[k] = a.v + ef.row[4 * q + k];
+    // a group's rows are requested ahead of the group before it, the scalars' ahead of the last
+    float2 x[4], xn[4];
+    float xs[kRNS][4];
+    auto scalars = [&]() {
+      if (a.ns == 0) return;
+#pragma unroll
+      for (int m = 0; m < kRNS; ++m)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xs[m][k] = vr[k][16 * m + c < a.a0 ? 16 * m + c : 0];
+    };
+    if (groups > 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) xn[k] = ld2(vr[k] + col[0]);
+    } else {
+      scalars();
     }
     float bas[NB], pre[4], h[4];
-    trunk_of<NB>(a, w1s, ev.r, q, bas, pre, h);
-    float bv[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) bv[u] = ev.w * h[u];
+    trunk_of<NB>(a, w1s, r, q, bas, pre, h);
     SplitB hb{};
-    if constexpr (SPLIT) hb = split_b(bv[0], bv[1], bv[2], bv[3]);
-    const float* vj = a.v + ev.node * a.D;
-#pragma unroll
-    for (int m = 0; m < kRNS; ++m) {
-      const float4 x = tile_x(a, m, q, vj);
-      if (m < a.ns) {
-      const floatx4 d = coefficients_of<SPLIT>(rf_s, rs_s, bias_s, m, lane, q, ev.w, bv, hb);
-      const int col = 16 * m + 4 * q;
-      if (col < a.a0) {
-        accs[m][0] = fmaf(d[0], x.x, accs[m][0]);
-        accs[m][1] = fmaf(d[1], x.y, accs[m][1]);
-        accs[m][2] = fmaf(d[2], x.z, accs[m][2]);
-        accs[m][3] = fmaf(d[3], x.w, accs[m][3]);
+    if constexpr (SPLIT) hb = split_b(h[0], h[1], h[2], h[3]);
+    // edges 4q .. 4q + 3 of slot m's row c
+    auto product = [&](int m) {
+      floatx4 d = *reinterpret_cast<const floatx4*>(&bias_s[16 * m + c]);
+      if constexpr (SPLIT) {
+        const u32x4 hm = rs_s[2 * kWave * m + lane], hl = rs_s[2 * kWave * m + kWave + lane];
+        d = mfma_bf16(hb.lh, hl, d);
+        d = mfma_bf16(hb.mm, hm, d);
+        return mfma_bf16(hb.hh, hm, d);
+      } else {
+        const float4 rv = rf_s[kWave * m + lane];
+        d = mfma16(h[0], rv.x, d);
+        d = mfma16(h[1], rv.y, d);
+        d = mfma16(h[2], rv.z, d);
+        return mfma16(h[3], rv.w, d);
       }
+    };
+    // m = A z + B u with z = (w tau) x and u = w p conj(tau x) = (p conj(w tau)) conj(x)
+#pragma unroll
+    for (int g = 0; g < kFGroups; ++g) {
+      if (g < groups) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = xn[k];
+        if (g + 1 < kFGroups && g + 1 < groups) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) xn[k] = ld2(vr[k] + col[g + 1 < kFGroups ? g + 1 : 0]);
+        } else {
+          scalars();
+        }
+        floatx4 d[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[k] = product(kRNS + 4 * g + k);
+        float mr = 0.f, mi = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float4 f = ef.f[freq[g]][4 * q + k];
+          const float zr = f.x * x[k].x - f.y * x[k].y, zi = f.x * x[k].y + f.y * x[k].x;
+          const float ur = f.z * x[k].x + f.w * x[k].y, ui = f.w * x[k].x - f.z * x[k].y;
+          mr += d[0][k] * zr - d[1][k] * zi + d[2][k] * ur - d[3][k] * ui;
+          mi += d[0][k] * zi + d[1][k] * zr + d[2][k] * ui + d[3][k] * ur;
+        }
+        accc[g][0] += mr;
+        accc[g][1] += mi;
       }
     }
+    if (a.ns > 0) {
+      const float4 w = *reinterpret_cast<const float4*>(&ef.w[4 * q]);
 #pragma unroll
-    for (int m = 0; m < kRNC; ++m) {
-      const float4 x = tile_x(a, kRNS + m, q, vj);
-      if (m < a.nc) {
-      const floatx4 d = coefficients_of<SPLIT>(rf_s, rs_s, bias_s, kRNS + m, lane, q, ev.w, bv, hb);
-      const bool one = a.tile_n[m] == 1;
-      const float tc = one ? ev.t1.x : ev.t2.x, ts = one ? ev.t1.y : ev.t2.y;
-      const float pr = one ? ev.p1.x : ev.p2.x, pi = one ? ev.p1.y : ev.p2.y;
-      const float zr = tc * x.x - ts * x.y, zi = tc * x.y + ts * x.x;
-      const float bzr = d[2] * zr + d[3] * zi, bzi = d[3] * zr - d[2] * zi;  // B conj(z)
-      accc[m][0] += (d[0] * zr - d[1] * zi) + (pr * bzr - pi * bzi);
-      accc[m][1] += (d[0] * zi + d[1] * zr) + (pr * bzi + pi * bzr);
-      }
+      for (int m = 0; m < kRNS; ++m)
+        if (m < a.ns) {
+          const floatx4 d = product(m);
+          accs[m] += d[0] * (w.x * xs[m][0]) + d[1] * (w.y * xs[m][1]) + d[2] * (w.z * xs[m][2]) +
+                     d[3] * (w.w * xs[m][3]);
+        }
     }
   }
-  // sum each copy over the 16 edge lanes of its row, then lane c = 0 stores
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) {
-#pragma unroll
-    for (int m = 0; m < kRNS; ++m)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) accs[m][u] += __shfl_xor(accs[m][u], off, kWave);
-#pragma unroll
-    for (int m = 0; m < kRNC; ++m) {
-      accc[m][0] += __shfl_xor(accc[m][0], off, kWave);
-      accc[m][1] += __shfl_xor(accc[m][1], off, kWave);
-    }
-  }
-  if (c != 0) return;
+  // sum each copy over the four lane rows' edges, then lane row 0 stores
+  auto rows = [](float v) {
+    v += __shfl_xor(v, 16, kWave);
+    return v + __shfl_xor(v, 32, kWave);
+  };
   float* oi = a.out + i * a.D;
 #pragma unroll
   for (int m = 0; m < kRNS; ++m) {
-    const int col = 16 * m + 4 * q;
-    if (m < a.ns && col < a.a0)
-      *reinterpret_cast<float4*>(oi + col) = make_float4(accs[m][0], accs[m][1], accs[m][2], accs[m][3]);
+    const float v = rows(accs[m]);
+    if (q == 0 && 16 * m + c < a.a0) oi[16 * m + c] = v;
   }
 #pragma unroll
-  for (int m = 0; m < kRNC; ++m)
-    if (m < a.nc) *reinterpret_cast<float2*>(oi + a.tile_col[m] + 2 * q) = make_float2(accc[m][0], accc[m][1]);
+  for (int g = 0; g < kFGroups; ++g) {
+    const float2 v = make_float2(rows(accc[g][0]), rows(accc[g][1]));
+    if (q == 0 && live_copy[g]) *reinterpret_cast<float2*>(oi + col[g]) = v;
+  }
 }
 
 // A coefficient tile's source values and target gradient pieces for the lane
@@ -701,9 +811,6 @@ int64_t launch_backward_groups(const RadialConvArgs& a, float* partial, int64_t 
   return rows * groups;
 }
 
-// The forward's split form is held to four waves a SIMD (its registers would
-// otherwise allow three): 12.3 ms (fp32) -> 12.8 (split, three waves) -> 11.2 ms
-// (split, four waves) at 256x512, B = 4.
 template <int NB>
 void launch_forward(const RadialConvArgs& a, dim3 grid, hipStream_t s) {
   if (split_products())
