@@ -1285,19 +1285,21 @@ int check_shapes(int64_t N, int64_t w, int64_t C) {
 
 int width_class(int64_t w) { return w <= 16 ? 16 : (w <= 32 ? 32 : (w <= 64 ? 64 : 128)); }
 
-// Whether vectors of w reals take the 32-deep kernels.
-bool deep(int64_t w) { return split_products() && w > 16; }
+// Whether vectors of w reals take the split kernels (`split`) in their 32-deep
+// form.  Float vectors take the split kernels unless GM_SPLIT_PRODUCTS=0;
+// bfloat16 ones (and float ones with bfloat16 mix gradients) have no others.
+bool deep(int64_t w, bool split) { return split && w > 16; }
 
-// Column tile of the weight gradient's workgroups: 64 columns for vectors up to
-// 64 reals; above, 32 for the split kernel and 128 for the fp32 one.
-int64_t weight_tile(int64_t w) {
-  if (deep(w)) return 64 * (w <= 64 ? DeepJT<64> : DeepJT<128>);
+// Column tile of the weight gradient's workgroups: of the 32-deep kernels; of
+// the others 64 columns for vectors up to 64 reals, above 128.
+int64_t weight_tile(int64_t w, bool split) {
+  if (deep(w, split)) return 64 * (w <= 64 ? DeepJT<64> : DeepJT<128>);
   return w <= 64 ? 64 : 128;
 }
 
-// Partial matrices a workgroup row writes: four (one a wave) but for the fp32
-// kernel of vectors above 64 reals (one).
-int64_t weight_partials_per_split(int64_t w) { return w <= 64 && !deep(w) ? 4 : 1; }
+// Partial matrices a workgroup row writes: four (one a wave) but for the
+// 32-deep kernels and the fp32 kernel of vectors above 64 reals (one).
+int64_t weight_partials_per_split(int64_t w, bool split) { return w <= 64 && !deep(w, split) ? 4 : 1; }
 
 // Row groups g of a grid of nx x g workgroups whose rows each workgroup loops
 // over in equal shares: about `want` workgroups in whole rounds of the
@@ -1313,10 +1315,9 @@ int64_t round_groups(int64_t nx, int64_t want, int64_t slots) {
   return (r * slots) / nx;
 }
 
-// The weight gradient's kernel for vectors of w reals (float vectors; the
-// bfloat16 form shares its workspace, so its grid follows this one).
-const void* dweight_kernel(int64_t w) {
-  const bool sp = split_products();
+// The weight gradient's kernel for vectors of w reals (for bfloat16 vectors
+// its float form's occupancy stands in).
+const void* dweight_kernel(int64_t w, bool sp) {
   switch (width_class(w)) {
     case 16: return sp ? (const void*)node_mix_dweight_split<16> : (const void*)node_mix_dweight_k_kernel<16>;
     case 32: return sp ? (const void*)node_mix_dweight_deep<32> : (const void*)node_mix_dweight_k_kernel<32>;
@@ -1332,13 +1333,13 @@ const void* dweight_kernel(int64_t w) {
 constexpr int64_t kMaxChainRows = 4096;
 
 // The weight gradient's row splits: about 1024 workgroups in whole rounds, whole 64-row chunks per split.
-void weight_splits(int64_t N, int64_t w, int64_t C, int64_t max_splits, int64_t& splits, int64_t& rps) {
-  const int64_t tile = weight_tile(w);
+void weight_splits(int64_t N, int64_t w, int64_t C, bool split, int64_t max_splits, int64_t& splits, int64_t& rps) {
+  const int64_t tile = weight_tile(w, split);
   const int64_t nx = (C + tile - 1) / tile > 0 ? (C + tile - 1) / tile : 1;
   const int64_t chunks = (N + 63) / 64;
   int64_t want = 1024;
-  if (deep(w)) want = std::max(want, nx * ((N + kMaxChainRows - 1) / kMaxChainRows));
-  int64_t s = round_groups(nx, want, resident_blocks(dweight_kernel(w), kThreads));
+  if (deep(w, split)) want = std::max(want, nx * ((N + kMaxChainRows - 1) / kMaxChainRows));
+  int64_t s = round_groups(nx, want, resident_blocks(dweight_kernel(w, split), kThreads));
   if (s > chunks) s = chunks;
   if (s > max_splits) s = max_splits;
   if (s < 1) s = 1;
@@ -1396,11 +1397,11 @@ int launch_dinput(const float* dmix, const float* M, int64_t N, int64_t w, int64
 
 int launch_dweight(const float* v, int64_t ldv, const float* dmix, int64_t N, int64_t w, int64_t C, int64_t splits,
                    int64_t rps, float* partial, float* dM, hipStream_t stream) {
-  const int64_t tile = weight_tile(w), nx = (C + tile - 1) / tile;
+  const bool sp = split_products();
+  const int64_t tile = weight_tile(w, sp), nx = (C + tile - 1) / tile;
   if (N > 0 && nx > 0) {
     const dim3 grid((unsigned)nx, (unsigned)splits), block(kThreads);
     const int vec = aligned(v, 16) && ldv % 4 == 0, vec_p = aligned(partial, 16);
-    const bool sp = split_products();
     switch (width_class(w)) {
       case 16:
         if (sp) hipLaunchKernelGGL(node_mix_dweight_split<16>, grid, block, 0, stream, v, ldv, dmix, N, (int)w, C, rps, partial, vec);
@@ -1424,7 +1425,7 @@ int launch_dweight(const float* v, int64_t ldv, const float* dmix, int64_t N, in
   }
   const int64_t n = w * C;
   if (n > 0) {
-    const int64_t parts = (N > 0 && C > 0) ? splits * weight_partials_per_split(w) : (int64_t)0;
+    const int64_t parts = (N > 0 && C > 0) ? splits * weight_partials_per_split(w, sp) : (int64_t)0;
     return launch_reduce(partial, n, parts, dM, stream);
   }
   return GM_OK;
@@ -1523,7 +1524,7 @@ int backward_input(const float* dmix, const float* M, int64_t N, int64_t w, int6
   GM_REQUIRE(C == 0 || (dmix && M), "dmix and M must be device pointers");
   GM_REQUIRE(C % 4 == 0 && aligned(dmix, 16) && aligned(M, 16),
              "dmix and M must be 16-byte aligned with C a multiple of 4");
-  if (deep(w)) {
+  if (deep(w, split_products())) {
     int64_t splits = 1, per_split = 0;
     if (partial != nullptr) {
       input_splits(N, w, C, splits, per_split);
@@ -1555,7 +1556,7 @@ extern "C" int gm_node_mix_backward_input_f32(const float* dmix, const float* M,
 }
 
 extern "C" int64_t gm_node_mix_input_partials(int64_t N, int64_t w, int64_t C) {
-  if (N <= 0 || w < 1 || w > 128 || C <= 0 || !gm::deep(w)) return 0;
+  if (N <= 0 || w < 1 || w > 128 || C <= 0 || !gm::deep(w, gm::split_products())) return 0;
   int64_t splits = 1, per_split = 0;
   gm::input_splits(N, w, C, splits, per_split);
   return splits > 1 ? splits * N * w : 0;
@@ -1567,9 +1568,14 @@ extern "C" int gm_node_mix_backward_input_split_f32(const float* dmix, const flo
 }
 
 extern "C" int64_t gm_node_mix_weight_partials(int64_t N, int64_t w, int64_t C) {
-  int64_t splits = 1, rps = 64;
-  gm::weight_splits(N, w, C, 1 << 20, splits, rps);
-  return splits * gm::weight_partials_per_split(w) * w * C;
+  // one workspace for float and bfloat16 vectors: the larger of what their kernels write
+  int64_t most = 0;
+  for (const bool split : {gm::split_products(), true}) {
+    int64_t splits = 1, rps = 64;
+    gm::weight_splits(N, w, C, split, 1 << 20, splits, rps);
+    most = std::max(most, splits * gm::weight_partials_per_split(w, split) * w * C);
+  }
+  return most;
 }
 
 extern "C" int gm_node_mix_backward_weight_f32(const float* v, int64_t ldv, const float* dmix, int64_t N, int64_t w,
@@ -1581,7 +1587,7 @@ extern "C" int gm_node_mix_backward_weight_f32(const float* v, int64_t ldv, cons
   GM_REQUIRE(N == 0 || (v && dmix && ldv >= w), "v (ldv >= w) and dmix must be device pointers");
   GM_REQUIRE(C % 4 == 0 && (N == 0 || gm::aligned(dmix, 16)), "dmix must be 16-byte aligned with C a multiple of 4");
   int64_t splits = 1, rps = 64;
-  gm::weight_splits(N, w, C, 1 << 20, splits, rps);
+  gm::weight_splits(N, w, C, gm::split_products(), 1 << 20, splits, rps);
   return gm::launch_dweight(v, ldv, dmix, N, w, C, splits, rps, partial, dM, (hipStream_t)stream);
 }
 
@@ -1593,7 +1599,7 @@ extern "C" int gm_node_mix_backward_weight_noalloc_f32(const float* v, int64_t l
   GM_REQUIRE(dM, "dM must be a device pointer");
   GM_REQUIRE(N == 0 || (v && dmix && ldv >= w), "v (ldv >= w) and dmix must be device pointers");
   GM_REQUIRE(C % 4 == 0 && (N == 0 || gm::aligned(dmix, 16)), "dmix must be 16-byte aligned with C a multiple of 4");
-  const int64_t per_split = gm::weight_partials_per_split(w) * w * C;
+  const int64_t per_split = gm::weight_partials_per_split(w, gm::split_products()) * w * C;
   const int64_t needed = (w <= 64 || gm::split_products() ? 4 : 1) * w * C;
   GM_REQUIRE(needed <= gm::kScratchFloats,
              "w * C is too large for the no-allocation weight gradient: its partials need " +
@@ -1618,7 +1624,7 @@ extern "C" int gm_node_mix_backward_weight_noalloc_f32(const float* v, int64_t l
   }
   // as many row splits as the scratch holds (every partial is written in full: nothing to clear)
   int64_t splits = 1, rps = 64;
-  gm::weight_splits(N, w, C, gm::kScratchFloats / per_split, splits, rps);
+  gm::weight_splits(N, w, C, gm::split_products(), gm::kScratchFloats / per_split, splits, rps);
   rc = gm::launch_dweight(v, ldv, dmix, N, w, C, splits, rps, partial, dM, s);
   if (rc != GM_OK || !ordered) return rc;
   err = hipEventRecord(gm::scratch_done[device], s);
@@ -1668,8 +1674,8 @@ template <typename V, typename DM>
 int split_dweight(const V* v, int64_t ldv, const DM* dmix, int64_t N, int64_t w, int64_t C, float* partial, float* dM,
                   hipStream_t s) {
   int64_t splits = 1, rps = 64;
-  weight_splits(N, w, C, 1 << 20, splits, rps);
-  const int64_t tile = weight_tile(w), nx = (C + tile - 1) / tile;
+  weight_splits(N, w, C, true, 1 << 20, splits, rps);
+  const int64_t tile = weight_tile(w, true), nx = (C + tile - 1) / tile;
   if (N > 0 && nx > 0) {
     const dim3 grid((unsigned)nx, (unsigned)splits), block(kThreads);
     const int vec = aligned(v, sizeof(V) == 2 ? 8 : 16) && ldv % 4 == 0, vec_p = aligned(partial, 16);
@@ -1685,7 +1691,7 @@ int split_dweight(const V* v, int64_t ldv, const DM* dmix, int64_t N, int64_t w,
     const int rc = check_launch("node_mix_backward_weight");
     if (rc != GM_OK) return rc;
   }
-  const int64_t parts = (N > 0 && C > 0) ? splits * weight_partials_per_split(w) : (int64_t)0;
+  const int64_t parts = (N > 0 && C > 0) ? splits * weight_partials_per_split(w, true) : (int64_t)0;
   return launch_reduce(partial, w * C, parts, dM, s);
 }
 
