@@ -17,6 +17,7 @@ several devices or not contiguous -- go through the construction itself.
 from __future__ import annotations
 
 import itertools
+import threading
 from collections.abc import Callable, Sequence
 from typing import Any
 
@@ -28,6 +29,8 @@ from gm_attention_amd import _native
 MAX_SOURCES = 256  # tensors a launch reads
 MAX_USES = 16  # uses of one parameter entry the gradient's padded table holds
 _ALIGN = 64  # entries a form starts at a multiple of (256 bytes: whole cache lines)
+_OFFSET = (1 << 39) - 1  # of a code: its entry's offset in the tensor
+_LOCK = threading.RLock()  # plans and their tables are found by one thread at a time
 
 
 def _starts(sizes: Sequence[int], align: int) -> list[int]:
@@ -35,9 +38,17 @@ def _starts(sizes: Sequence[int], align: int) -> list[int]:
     return list(itertools.accumulate((-(-n // align) * align for n in sizes), initial=0))
 
 
+def _complete(device: torch.device) -> None:
+    """Waits for what this stream writes: the kernels follow a plan's tables
+    unchecked, and other streams and threads use them without an event of this
+    one's, so they are complete before anything else can see them."""
+    if device.type == "cuda":
+        torch.cuda.current_stream(device).synchronize()
+
+
 class Plan:
     """Where every entry of a construction's forms comes from, found on the
-    parameters' device."""
+    parameters' device and complete on return."""
 
     def __init__(self, shapes: tuple[torch.Size, ...], build: Callable[[list[Tensor]], list[Tensor]],
                  device: torch.device) -> None:
@@ -53,11 +64,11 @@ class Plan:
         for a, m in zip(self.out_starts, forms):
             flat[a:a + m.numel()] = m.reshape(-1)
         position = flat.abs().long() - 1  # -1: zero
-        self._used = (position, flat < 0)
         self.codes = torch.where(position < 0, -1, self._code(self.in_starts, position, flat < 0)).reshape(1, -1)
         counts = torch.bincount(position.clamp_min(-1) + 1, minlength=2)[1:]
         self.most = int(counts.max())  # uses of one parameter entry
         self.back: Tensor | None = None
+        _complete(device)
 
     @staticmethod
     def _code(starts: list[int], position: Tensor, negative: Tensor) -> Tensor:
@@ -70,23 +81,33 @@ class Plan:
     def gradient_codes(self) -> Tensor:
         """``(uses, parameter entries)``: entry p's j-th use among the forms' entries."""
         if self.back is None:
-            position, negative = self._used
-            used = torch.nonzero(position >= 0).squeeze(1)
-            at, order = torch.sort(position[used], stable=True)
-            used = used[order]
-            rank = torch.arange(at.numel(), device=at.device) - torch.searchsorted(at, at)
-            table = torch.full((max(self.most, 1), self.in_starts[-1]), -1, dtype=torch.int64, device=at.device)
-            table[rank, at] = self._code(self.out_starts, used, negative[used])
-            self.back = table
-            self._used = None
+            with _LOCK:
+                if self.back is None:
+                    codes = self.codes[0]
+                    used = torch.nonzero(codes >= 0).squeeze(1)
+                    codes = codes[used]
+                    starts = torch.tensor(self.in_starts, dtype=torch.int64, device=codes.device)
+                    at, order = torch.sort(starts[codes >> 40] + ((codes >> 1) & _OFFSET), stable=True)
+                    rank = torch.arange(at.numel(), device=at.device) - torch.searchsorted(at, at)
+                    table = torch.full((max(self.most, 1), self.in_starts[-1]), -1, dtype=torch.int64,
+                                       device=at.device)
+                    table[rank, at] = self._code(self.out_starts, used[order], (codes[order] & 1) == 1)
+                    _complete(table.device)
+                    self.back = table
         return self.back
+
+
+def _gather(tensors: Sequence[Tensor | None], codes: Tensor) -> Tensor:
+    """``signed_gather`` on the current stream, which the table's memory then outlives."""
+    codes.record_stream(torch.cuda.current_stream(codes.device))
+    return _native.signed_gather(tensors, codes)
 
 
 class _Assemble(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, plan: Plan, *params: Tensor) -> tuple:
         ctx.plan = plan
-        out = _native.signed_gather(params, plan.codes)
+        out = _gather(params, plan.codes)
         return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.out_starts, plan.form_shapes))
 
     @staticmethod
@@ -94,7 +115,7 @@ class _Assemble(torch.autograd.Function):
     def backward(ctx: Any, *grads: Tensor | None) -> tuple:
         plan = ctx.plan
         held = [None if g is None else g.to(torch.float32).contiguous() for g in grads]
-        flat = _native.signed_gather(held, plan.gradient_codes())
+        flat = _gather(held, plan.gradient_codes())
         return (None, *(flat[a:a + s.numel()].view(s) if need else None
                         for a, s, need in zip(plan.in_starts, plan.shapes, ctx.needs_input_grad[1:])))
 
@@ -119,8 +140,13 @@ def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[
     key = ("_assembly", name, str(params[0].device))
     plan = owner.__dict__.get(key)
     if plan is None or plan.shapes != shapes:
-        plan = Plan(shapes, build, params[0].device)
-        owner.__dict__[key] = plan
+        with _LOCK:
+            plan = owner.__dict__.get(key)
+            if plan is None or plan.shapes != shapes:
+                plan = Plan(shapes, build, params[0].device)
+                owner.__dict__[key] = plan
     if plan.most > MAX_USES:
         return build(list(params))
+    if torch.is_grad_enabled() and any(p.requires_grad for p in params):
+        plan.gradient_codes()  # found here: the backward runs on a thread and perhaps a stream of its own
     return list(_Assemble.apply(plan, *params))

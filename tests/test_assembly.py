@@ -3,6 +3,9 @@ transposed gather against the construction itself and its autograd gradient,
 by evaluating the codes in torch on the CPU, and the HIP launch on the GPU
 (moves and sign changes: bit for bit; gradients: the uses of an entry added)."""
 
+import threading
+import time
+
 import pytest
 import torch
 
@@ -65,6 +68,82 @@ def test_parameters_the_kernel_does_not_take_go_through_the_construction():
     got = assembly.assembled(Owner(), "x", params, _build)  # CPU
     for g, w in zip(got, _build(params)):
         assert torch.equal(g, w) and g.grad_fn is not None
+
+
+class _Owner:
+    pass
+
+
+@pytest.fixture
+def on_cpu(monkeypatch):
+    """Assembly on the CPU: the launch replaced by its definition."""
+    monkeypatch.setattr(assembly, "takes", lambda params: True)
+    monkeypatch.setattr(assembly, "_gather", lambda sources, codes: _gather(sources, codes).float())
+
+
+def test_the_gradients_table_is_there_before_any_backward(on_cpu, monkeypatch):
+    """A backward runs on a thread, and perhaps a stream, of its own: it finds its table complete."""
+    owner, params, plans = _Owner(), [p.requires_grad_(True) for p in _params()], []
+    find = assembly.Plan.__init__
+    monkeypatch.setattr(assembly.Plan, "__init__", lambda self, *a: (find(self, *a), plans.append(self))[0])
+    with torch.no_grad():
+        assembly.assembled(owner, "x", params, _build)
+    assert plans[0].back is None  # inference needs none
+    got = assembly.assembled(owner, "x", params, _build)
+    assert len(plans) == 1 and plans[0].back is not None
+    up = [torch.randn_like(g) for g in got]
+    want = torch.autograd.grad(_build(params), params, up, allow_unused=True)
+    for g, w in zip(torch.autograd.grad(got, params, up), want):
+        assert torch.allclose(g, torch.zeros_like(g) if w is None else w, rtol=0, atol=1e-6)
+
+
+def test_threads_finding_one_table_agree(monkeypatch):
+    plan = assembly.Plan(tuple(p.shape for p in _params()), _build, torch.device("cpu"))
+    want = assembly.Plan(plan.shapes, _build, torch.device("cpu")).gradient_codes()
+    code = assembly.Plan._code
+
+    def slowly(*args):
+        time.sleep(0.05)
+        return code(*args)
+
+    monkeypatch.setattr(assembly.Plan, "_code", staticmethod(slowly))
+    start, got = threading.Barrier(8), []
+
+    def find():
+        start.wait()
+        time.sleep(0.01 * len(got))
+        got.append(plan.gradient_codes())
+
+    threads = [threading.Thread(target=find) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 8 and all(g is got[0] for g in got) and torch.equal(got[0], want)
+
+
+@pytest.mark.gpu
+def test_tables_found_behind_a_busy_stream_are_complete_for_another(cuda):
+    owner, params = _Owner(), [p.requires_grad_(True) for p in _params(cuda)]
+    want = _build(params)
+    up = [torch.randn_like(w) for w in want]
+    ref = torch.autograd.grad(want, params, up, allow_unused=True)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(100_000_000)  # some tens of milliseconds ahead of the tables
+        assembly.Plan(tuple(p.shape for p in params), _build, cuda)
+        assert first.query()
+        torch.cuda._sleep(100_000_000)
+        got = assembly.assembled(owner, "x", params, _build)
+    with torch.cuda.stream(second):  # while `first` may still gather its forms
+        again = assembly.assembled(owner, "x", params, _build)
+        grads = torch.autograd.grad(again, params, up)
+    torch.cuda.synchronize()
+    for a, b, w in zip(got, again, want):
+        assert torch.equal(a, w) and torch.equal(b, w)
+    for g, r in zip(grads, ref):
+        assert torch.allclose(g, torch.zeros_like(g) if r is None else r, rtol=0, atol=1e-6)
 
 
 @pytest.mark.gpu
