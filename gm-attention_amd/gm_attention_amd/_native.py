@@ -705,7 +705,8 @@ def _column_view(v: Tensor) -> tuple[int, int]:
 
 def signed_gather(sources: Any, codes: Tensor) -> Tensor:
     """``(n,)`` sums of the entries ``codes (uses, n)`` names among ``sources``
-    (float32, contiguous, None for zeros; ``gm_signed_gather_f32``)."""
+    (float32, contiguous, on the codes' device, None for zeros; ``gm_signed_gather_f32``)."""
+    _require_device(codes)
     uses, n = codes.shape
     out = torch.empty(n, dtype=torch.float32, device=codes.device)
     pointers = (_P * len(sources))(*[_ptr(t) for t in sources])

@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import itertools
 import threading
+import weakref
 from collections.abc import Callable, Sequence
 from typing import Any
 
@@ -31,6 +32,10 @@ MAX_USES = 16  # uses of one parameter entry the gradient's padded table holds
 _ALIGN = 64  # entries a form starts at a multiple of (256 bytes: whole cache lines)
 _OFFSET = (1 << 39) - 1  # of a code: its entry's offset in the tensor
 _LOCK = threading.RLock()  # plans and their tables are found by one thread at a time
+#: Plans by the module whose parameters they assemble, then by name, device and
+#: shapes: beside the modules, so that these copy, pickle and list as if there
+#: were none, and gone with them.
+_PLANS: weakref.WeakKeyDictionary[Any, dict[tuple, Plan]] = weakref.WeakKeyDictionary()
 
 
 def _starts(sizes: Sequence[int], align: int) -> list[int]:
@@ -131,20 +136,19 @@ def takes(params: Sequence[Tensor]) -> bool:
 
 def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[list[Tensor]], list[Tensor]]) -> list:
     """``build(params)``, a list of forms whose every entry is an entry of
-    ``params``, negated or not, or zero.  The plan is kept on ``owner`` under
-    ``name`` (which also names whatever else ``build`` depends on) for the
-    parameters' shapes and device."""
+    ``params``, negated or not, or zero.  The plan is kept for ``owner`` under
+    ``name`` (which also names whatever else ``build`` depends on) and the
+    parameters' device and shapes."""
     if not takes(params):
         return build(list(params))
-    shapes = tuple(p.shape for p in params)
-    key = ("_assembly", name, str(params[0].device))
-    plan = owner.__dict__.get(key)
-    if plan is None or plan.shapes != shapes:
+    key = (name, params[0].device, tuple(p.shape for p in params))
+    plan = _PLANS.get(owner, {}).get(key)
+    if plan is None:
         with _LOCK:
-            plan = owner.__dict__.get(key)
-            if plan is None or plan.shapes != shapes:
-                plan = Plan(shapes, build, params[0].device)
-                owner.__dict__[key] = plan
+            plans = _PLANS.setdefault(owner, {})
+            plan = plans.get(key)
+            if plan is None:
+                plan = plans[key] = Plan(key[2], build, key[1])
     if plan.most > MAX_USES:
         return build(list(params))
     if torch.is_grad_enabled() and any(p.requires_grad for p in params):

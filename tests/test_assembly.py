@@ -3,8 +3,13 @@ transposed gather against the construction itself and its autograd gradient,
 by evaluating the codes in torch on the CPU, and the HIP launch on the GPU
 (moves and sign changes: bit for bit; gradients: the uses of an entry added)."""
 
+import copy
+import gc
+import inspect
+import pickle
 import threading
 import time
+import weakref
 
 import pytest
 import torch
@@ -120,6 +125,36 @@ def test_threads_finding_one_table_agree(monkeypatch):
     for t in threads:
         t.join()
     assert len(got) == 8 and all(g is got[0] for g in got) and torch.equal(got[0], want)
+
+
+def test_modules_with_plans_list_copy_and_pickle_without_them(on_cpu):
+    from gm_attention_amd.nn.normalization import SO2LayerNorm
+
+    field = SO2FieldType({0: 4, 1: 3})
+    plain, norm = SO2LayerNorm(field), SO2LayerNorm(field)
+    want = norm.gamma_flat(torch.float32)
+    assert set(norm.__dict__) == set(plain.__dict__)
+    assert len(assembly._PLANS[norm]) == 1
+    assert dir(norm) == dir(plain) and len(inspect.getmembers(norm)) == len(inspect.getmembers(plain))
+    assert len(pickle.dumps(norm)) == len(pickle.dumps(plain))
+    for copied in (copy.deepcopy, lambda m: pickle.loads(pickle.dumps(m))):
+        other = copied(norm)
+        assert other not in assembly._PLANS
+        assert torch.equal(other.gamma_flat(torch.float32), want)
+        plan = weakref.ref(next(iter(assembly._PLANS[other].values())))
+        del other
+        gc.collect()
+        assert plan() is None  # gone with its module
+
+
+def test_shapes_and_devices_have_plans_of_their_own(on_cpu):
+    owner = _Owner()
+    params = _params()
+    wider = [p.repeat(2, *([1] * (p.dim() - 1))) if i == 2 else p for i, p in enumerate(params)]
+    for ps in (params, wider, params):
+        for g, w in zip(assembly.assembled(owner, "x", ps, _build), _build(ps)):
+            assert torch.equal(g, w)
+    assert len(assembly._PLANS[owner]) == 2
 
 
 @pytest.mark.gpu
