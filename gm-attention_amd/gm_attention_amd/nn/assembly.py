@@ -11,7 +11,8 @@ parameter entry's uses added in a fixed order.  The numbers are the
 construction's own, bit for bit (moves and sign changes only).
 
 Parameters the kernel does not take -- CPU tensors, other types, parameters on
-several devices or not contiguous -- go through the construction itself.
+several devices or not contiguous -- go through the construction itself, as do
+parameters without a plan on a stream under capture.
 """
 
 from __future__ import annotations
@@ -143,6 +144,9 @@ def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[
         return build(list(params))
     key = (name, params[0].device, tuple(p.shape for p in params))
     plan = _PLANS.get(owner, {}).get(key)
+    graded = torch.is_grad_enabled() and any(p.requires_grad for p in params)
+    if (plan is None or (graded and plan.back is None)) and torch.cuda.is_current_stream_capturing():
+        return build(list(params))  # finding a plan waits on the host: a captured stream takes the construction
     if plan is None:
         with _LOCK:
             plans = _PLANS.setdefault(owner, {})
@@ -151,6 +155,6 @@ def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[
                 plan = plans[key] = Plan(key[2], build, key[1])
     if plan.most > MAX_USES:
         return build(list(params))
-    if torch.is_grad_enabled() and any(p.requires_grad for p in params):
+    if graded:
         plan.gradient_codes()  # found here: the backward runs on a thread and perhaps a stream of its own
     return list(_Assemble.apply(plan, *params))

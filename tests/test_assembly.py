@@ -84,6 +84,7 @@ def on_cpu(monkeypatch):
     """Assembly on the CPU: the launch replaced by its definition."""
     monkeypatch.setattr(assembly, "takes", lambda params: True)
     monkeypatch.setattr(assembly, "_gather", lambda sources, codes: _gather(sources, codes).float())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
 
 
 def test_the_gradients_table_is_there_before_any_backward(on_cpu, monkeypatch):
@@ -155,6 +156,63 @@ def test_shapes_and_devices_have_plans_of_their_own(on_cpu):
         for g, w in zip(assembly.assembled(owner, "x", ps, _build), _build(ps)):
             assert torch.equal(g, w)
     assert len(assembly._PLANS[owner]) == 2
+
+
+def test_a_captured_stream_without_a_plan_takes_the_construction(on_cpu, monkeypatch):
+    owner, params = _Owner(), [p.requires_grad_(True) for p in _params()]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    for g, w in zip(assembly.assembled(owner, "x", params, _build), _build(params)):
+        assert torch.equal(g, w)
+    assert owner not in assembly._PLANS
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    with torch.no_grad():
+        assembly.assembled(owner, "x", params, _build)
+    plan = next(iter(assembly._PLANS[owner].values()))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assembly.assembled(owner, "x", params, _build)
+    assert plan.back is None  # no gradient table is found under capture either
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("train", [False, True])
+def test_first_calls_of_norm_gate_and_linear_under_capture(train, cuda):
+    """Modules that have run nothing yet, captured forward (and backward): replays
+    between eager work equal the eager results, bit for bit forward."""
+    from gm_attention_amd.nn.linear import SO2Linear, flat_forward
+    from gm_attention_amd.nn.nonlinearities import SO2ScalarGatedNonlinearity
+    from gm_attention_amd.nn.normalization import SO2LayerNorm
+
+    field = SO2FieldType({0: 8, 1: 4, 2: 4})
+    torch.manual_seed(0)
+    made = dict(dtype=torch.float32, device=cuda)
+    norm, gate, lin = SO2LayerNorm(field, **made), SO2ScalarGatedNonlinearity(field, **made), SO2Linear(field, field, **made)
+    params = [p for m in (norm, gate, lin) for p in m.parameters()]
+    x = torch.randn(50, field.dimension, device=cuda, requires_grad=train)
+    up = torch.randn(50, field.dimension, device=cuda)
+
+    def step(norm, gate, lin, params):
+        with torch.set_grad_enabled(train):
+            out = flat_forward(lin, gate.forward_flat(norm.forward_flat(x)))
+        return (out.detach(), *torch.autograd.grad(out, [x, *params], up)) if train else (out,)
+
+    # the libraries' handles come up on another set of modules
+    others = [copy.deepcopy(m) for m in (norm, gate, lin)]
+    with torch.cuda.stream(torch.cuda.Stream()):
+        want = step(*others, [p for m in others for p in m.parameters()])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(norm, gate, lin, params)
+    for value in (x.detach().clone(), torch.randn_like(x), torch.randn_like(x)):
+        with torch.no_grad():
+            x.copy_(value)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = step(*others, [p for m in others for p in m.parameters()])
+        assert torch.equal(got[0], want[0])
+        for g, w in zip(got[1:], want[1:], strict=True):
+            assert torch.allclose(g, w, rtol=1e-5, atol=1e-5)
+        torch.cuda.synchronize()
 
 
 @pytest.mark.gpu
