@@ -10,9 +10,11 @@ where every entry comes from, and from then on fills every form with one
 parameter entry's uses added in a fixed order.  The numbers are the
 construction's own, bit for bit (moves and sign changes only).
 
-Parameters the kernel does not take -- CPU tensors, other types, parameters on
-several devices or not contiguous -- go through the construction itself, as do
-parameters without a plan on a stream under capture.
+Parameters the kernel does not take -- CPU tensors, other types and subclasses,
+parameters on several devices or another than the current one, or not
+contiguous -- go through the construction itself, as do parameters without a
+plan on a stream under capture, and all of them under functorch transforms,
+forward-mode derivatives, tracing and compiling.
 """
 
 from __future__ import annotations
@@ -24,13 +26,15 @@ from collections.abc import Callable, Sequence
 from typing import Any
 
 import torch
-from torch import Tensor
+from torch import Tensor, nn
+from torch.autograd import forward_ad
 
 from gm_attention_amd import _native
 
 MAX_SOURCES = 256  # tensors a launch reads
 MAX_USES = 16  # uses of one parameter entry the gradient's padded table holds
 _ALIGN = 64  # entries a form starts at a multiple of (256 bytes: whole cache lines)
+_PLAIN = (Tensor, nn.Parameter)  # subclasses may hold their numbers elsewhere
 _OFFSET = (1 << 39) - 1  # of a code: its entry's offset in the tensor
 _LOCK = threading.RLock()  # plans and their tables are found by one thread at a time
 #: Plans by the module whose parameters they assemble, then by name, device and
@@ -110,20 +114,50 @@ def _gather(tensors: Sequence[Tensor | None], codes: Tensor) -> Tensor:
 
 
 class _Assemble(torch.autograd.Function):
+    """The forms from the parameters; its gradient is :class:`_Transposed`, and that one's is this one."""
+
     @staticmethod
-    def forward(ctx: Any, plan: Plan, *params: Tensor) -> tuple:
+    def forward(ctx: Any, plan: Plan, *params: Tensor | None) -> tuple:
         ctx.plan = plan
+        ctx.set_materialize_grads(False)
         out = _gather(params, plan.codes)
         return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.out_starts, plan.form_shapes))
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx: Any, *grads: Tensor | None) -> tuple:
-        plan = ctx.plan
-        held = [None if g is None else g.to(torch.float32).contiguous() for g in grads]
-        flat = _gather(held, plan.gradient_codes())
-        return (None, *(flat[a:a + s.numel()].view(s) if need else None
-                        for a, s, need in zip(plan.in_starts, plan.shapes, ctx.needs_input_grad[1:])))
+        if all(g is None for g in grads):
+            return (None,) * len(ctx.needs_input_grad)
+        out = _Transposed.apply(ctx.plan, *grads)
+        return (None, *(g if need else None for g, need in zip(out, ctx.needs_input_grad[1:])))
+
+
+class _Transposed(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx: Any, plan: Plan, *grads: Tensor | None) -> tuple:
+        ctx.plan = plan
+        ctx.set_materialize_grads(False)
+        out = _gather(_held(grads), plan.gradient_codes())
+        return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.in_starts, plan.shapes))
+
+    @staticmethod
+    def backward(ctx: Any, *grads: Tensor | None) -> tuple:
+        if all(g is None for g in grads):
+            return (None,) * len(ctx.needs_input_grad)
+        out = _Assemble.apply(ctx.plan, *_held(grads))
+        return (None, *(g if need else None for g, need in zip(out, ctx.needs_input_grad[1:])))
+
+
+def _held(tensors: Sequence[Tensor | None]) -> list[Tensor | None]:
+    """The tensors as the kernel reads them."""
+    return [None if t is None else t.to(torch.float32).resolve_neg().contiguous() for t in tensors]
+
+
+def _transformed() -> bool:
+    """Whether something follows torch's own operations here that an autograd
+    function with a launch of its own in it would hide from it: a functorch
+    transform, forward-mode derivatives, tracing or compiling."""
+    return (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0 or torch.jit.is_tracing()
+            or torch.compiler.is_compiling())
 
 
 def takes(params: Sequence[Tensor]) -> bool:
@@ -131,16 +165,19 @@ def takes(params: Sequence[Tensor]) -> bool:
     if not 0 < len(params) <= MAX_SOURCES:
         return False
     device = params[0].device
-    return device.type == "cuda" and all(p.dtype == torch.float32 and p.device == device and p.is_contiguous()
-                                         for p in params)
+    return (device.type == "cuda" and device.index == torch.cuda.current_device() and not _transformed()
+            and all(p.dtype == torch.float32 and p.device == device and p.is_contiguous() and not p.is_neg()
+                    and type(p) in _PLAIN for p in params))
 
 
-def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[list[Tensor]], list[Tensor]]) -> list:
+def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[list[Tensor]], list[Tensor]],
+              taken: bool | None = None) -> list:
     """``build(params)``, a list of forms whose every entry is an entry of
     ``params``, negated or not, or zero.  The plan is kept for ``owner`` under
     ``name`` (which also names whatever else ``build`` depends on) and the
-    parameters' device and shapes."""
-    if not takes(params):
+    parameters' device and shapes.  ``taken``: :func:`takes` of ``params`` where
+    the caller has it."""
+    if not (takes(params) if taken is None else taken):
         return build(list(params))
     key = (name, params[0].device, tuple(p.shape for p in params))
     plan = _PLANS.get(owner, {}).get(key)

@@ -265,7 +265,7 @@ class _LayerForms:
         if not self.served:
             return
         name = f"layer {layout.split} {layout.padded} {trunk}"
-        forms = iter(assembly.assembled(mhsa, name, params, build))
+        forms = iter(assembly.assembled(mhsa, name, params, build, taken=True))
 
         def pair(lin: SO2Linear) -> tuple[Tensor, Tensor | None]:
             return next(forms), next(forms) if lin.has_bias else None

@@ -840,7 +840,7 @@ def heads_mixing(kernels: list[Any], hp: HeadsPlan, split: int = 1) -> list[Tens
             return _heads_mixing_from(kernels, hp, [[None if p is None else next(it) for p in r] for r in readouts],
                                       split)
 
-        return assembly.assembled(kernels[0], f"mixing {len(kernels)} {split} {hp.plan.d_out}", params, build)
+        return assembly.assembled(kernels[0], f"mixing {len(kernels)} {split} {hp.plan.d_out}", params, build, taken=True)
     plan = _mixing_maps(kernels, hp, split)
     flat = torch.cat([p.reshape(-1) for k in kernels for p in k.readout_parameters() if p is not None])
     return list(_SignedGather.apply(flat, plan))

@@ -158,6 +158,76 @@ def test_shapes_and_devices_have_plans_of_their_own(on_cpu):
     assert len(assembly._PLANS[owner]) == 2
 
 
+def test_second_derivatives_are_the_constructions(on_cpu):
+    owner, params = _Owner(), [p.requires_grad_(True) for p in _params()]
+    torch.manual_seed(2)
+    probes = [torch.randn_like(w) for w in _build(params)]
+    probes[3] = None  # a form nothing reads
+
+    def twice(forms):
+        loss = sum((f ** 3 * p).sum() for f, p in zip(forms, probes) if p is not None)
+        first = torch.autograd.grad(loss, params, create_graph=True, allow_unused=True)
+        first = [torch.zeros_like(p) if g is None else g for g, p in zip(first, params)]
+        second = torch.autograd.grad(sum((g ** 2).sum() for g in first), params, allow_unused=True)
+        return [*first, *(torch.zeros_like(p) if g is None else g for g, p in zip(second, params))]
+
+    for g, w in zip(twice(assembly.assembled(owner, "x", params, _build)), twice(_build(params)), strict=True):
+        assert torch.allclose(g, w, rtol=1e-5, atol=1e-5)
+
+
+def test_transforms_are_followed_through_the_construction(monkeypatch):
+    from torch.autograd import forward_ad
+
+    seen = []
+    look = lambda x: seen.append(assembly._transformed()) or 2 * x  # noqa: E731
+    one = torch.ones(2)
+    look(one)
+    torch.func.grad(lambda x: look(x).sum())(one)
+    torch.vmap(look)(one)
+    torch.func.jvp(look, (one,), (one,))
+    with forward_ad.dual_level():
+        look(one)
+    before = len(seen)
+    torch.jit.trace(look, one, check_trace=False)
+    assert seen[:before] == [False, True, True, True, True] and all(seen[before:]) and len(seen) > before
+
+
+@pytest.mark.gpu
+def test_transforms_and_second_derivatives_of_norms_gains_on_the_gpu(cuda):
+    from torch.autograd import forward_ad
+
+    from gm_attention_amd.nn.normalization import SO2LayerNorm
+
+    norm = SO2LayerNorm(SO2FieldType({0: 5, 2: 3}), dtype=torch.float32, device=cuda)
+    gains = {f"gamma.{f}": torch.randn_like(p) for f, p in norm.gamma.items()}
+
+    def flat(g):
+        return torch.func.functional_call(_Gains(norm), {f"norm.{k}": v for k, v in g.items()}, ())
+
+    want = torch.cat([gains["gamma.0"], gains["gamma.2"].repeat_interleave(2)])
+    assert torch.equal(flat(gains), want)
+    grads = torch.func.grad(lambda g: (flat(g) ** 2).sum())(gains)
+    assert torch.allclose(grads["gamma.0"], 2 * gains["gamma.0"]) and torch.allclose(grads["gamma.2"], 4 * gains["gamma.2"])
+    many = torch.vmap(flat)({k: torch.stack([v, 2 * v]) for k, v in gains.items()})
+    assert torch.equal(many, torch.stack([want, 2 * want]))
+    with forward_ad.dual_level():
+        out = flat({k: forward_ad.make_dual(v, torch.ones_like(v)) for k, v in gains.items()})
+        assert torch.equal(forward_ad.unpack_dual(out).tangent, torch.ones_like(want))
+    leaves = [g.clone().requires_grad_(True) for g in gains.values()]
+    first = torch.autograd.grad((flat(dict(zip(gains, leaves))) ** 3).sum(), leaves, create_graph=True)
+    second = torch.autograd.grad(sum(g.sum() for g in first), leaves)
+    assert torch.allclose(second[0], 6 * leaves[0]) and torch.allclose(second[1], 12 * leaves[1])
+
+
+class _Gains(torch.nn.Module):
+    def __init__(self, norm):
+        super().__init__()
+        self.norm = norm
+
+    def forward(self):
+        return self.norm.gamma_flat(torch.float32)
+
+
 def test_a_captured_stream_without_a_plan_takes_the_construction(on_cpu, monkeypatch):
     owner, params = _Owner(), [p.requires_grad_(True) for p in _params()]
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
