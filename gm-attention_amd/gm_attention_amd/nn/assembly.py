@@ -36,7 +36,7 @@ MAX_USES = 16  # uses of one parameter entry the gradient's padded table holds
 _ALIGN = 64  # entries a form starts at a multiple of (256 bytes: whole cache lines)
 _PLAIN = (Tensor, nn.Parameter)  # subclasses may hold their numbers elsewhere
 _OFFSET = (1 << 39) - 1  # of a code: its entry's offset in the tensor
-_LOCK = threading.RLock()  # plans and their tables are found by one thread at a time
+LOCK = threading.RLock()  # plans and their tables are found by one thread at a time
 #: Plans by the module whose parameters they assemble, then by name, device and
 #: shapes: beside the modules, so that these copy, pickle and list as if there
 #: were none, and gone with them.
@@ -48,7 +48,7 @@ def _starts(sizes: Sequence[int], align: int) -> list[int]:
     return list(itertools.accumulate((-(-n // align) * align for n in sizes), initial=0))
 
 
-def _complete(device: torch.device) -> None:
+def complete(device: torch.device) -> None:
     """Waits for what this stream writes: the kernels follow a plan's tables
     unchecked, and other streams and threads use them without an event of this
     one's, so they are complete before anything else can see them."""
@@ -78,7 +78,7 @@ class Plan:
         counts = torch.bincount(position.clamp_min(-1) + 1, minlength=2)[1:]
         self.most = int(counts.max())  # uses of one parameter entry
         self.back: Tensor | None = None
-        _complete(device)
+        complete(device)
 
     @staticmethod
     def _code(starts: list[int], position: Tensor, negative: Tensor) -> Tensor:
@@ -91,7 +91,7 @@ class Plan:
     def gradient_codes(self) -> Tensor:
         """``(uses, parameter entries)``: entry p's j-th use among the forms' entries."""
         if self.back is None:
-            with _LOCK:
+            with LOCK:
                 if self.back is None:
                     codes = self.codes[0]
                     used = torch.nonzero(codes >= 0).squeeze(1)
@@ -102,7 +102,7 @@ class Plan:
                     table = torch.full((max(self.most, 1), self.in_starts[-1]), -1, dtype=torch.int64,
                                        device=at.device)
                     table[rank, at] = self._code(self.out_starts, used[order], (codes[order] & 1) == 1)
-                    _complete(table.device)
+                    complete(table.device)
                     self.back = table
         return self.back
 
@@ -185,7 +185,7 @@ def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[
     if (plan is None or (graded and plan.back is None)) and torch.cuda.is_current_stream_capturing():
         return build(list(params))  # finding a plan waits on the host: a captured stream takes the construction
     if plan is None:
-        with _LOCK:
+        with LOCK:
             plans = _PLANS.setdefault(owner, {})
             plan = plans.get(key)
             if plan is None:

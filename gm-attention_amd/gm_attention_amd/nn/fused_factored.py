@@ -783,6 +783,26 @@ class _SignedGather(torch.autograd.Function):
     kMaxUses = 16
 
     @staticmethod
+    def _gradient_plan(maps: list[tuple[Tensor, Tensor]], n: int) -> dict:
+        """Complete on return: other threads and streams use it once it is in the plan."""
+        index = torch.cat([i.reshape(-1) for i, _ in maps])
+        order = torch.argsort(index, stable=True)
+        counts = torch.bincount(index, minlength=n)
+        offsets = torch.cat([counts.new_zeros(1), torch.cumsum(counts, 0)])
+        found = dict(sign=torch.cat([s.reshape(-1) for _, s in maps]), order=order, offsets=offsets)
+        uses = int(counts.max()) if counts.numel() else 0
+        if uses <= _SignedGather.kMaxUses:
+            # column j: each parameter's j-th use (its position), or the appended zero
+            total = index.numel()
+            srt = index.index_select(0, order)
+            rank = torch.arange(total, device=index.device) - offsets.index_select(0, srt)
+            cols = torch.full((max(uses, 1), n), total, dtype=torch.int64, device=index.device)
+            cols[rank, srt] = order
+            found["cols"] = cols
+        assembly.complete(index.device)
+        return found
+
+    @staticmethod
     def forward(ctx: Any, flat: Tensor, plan: dict, *maps: tuple) -> tuple:
         ctx.plan = plan
         ctx.shapes = [index.shape for index, _ in plan["maps"]]
@@ -795,20 +815,9 @@ class _SignedGather(torch.autograd.Function):
     def backward(ctx: Any, *grads: Tensor) -> tuple:
         plan = ctx.plan
         if "order" not in plan:
-            index = torch.cat([i.reshape(-1) for i, _ in plan["maps"]])
-            plan["sign"] = torch.cat([s.reshape(-1) for _, s in plan["maps"]])
-            plan["order"] = torch.argsort(index, stable=True)
-            counts = torch.bincount(index, minlength=ctx.n)
-            plan["offsets"] = torch.cat([counts.new_zeros(1), torch.cumsum(counts, 0)])
-            uses = int(counts.max()) if counts.numel() else 0
-            if uses <= _SignedGather.kMaxUses:
-                # column j: each parameter's j-th use (its position), or the appended zero
-                total = index.numel()
-                srt = index.index_select(0, plan["order"])
-                rank = torch.arange(total, device=index.device) - plan["offsets"].index_select(0, srt)
-                cols = torch.full((max(uses, 1), ctx.n), total, dtype=torch.int64, device=index.device)
-                cols[rank, srt] = plan["order"]
-                plan["cols"] = cols
+            with assembly.LOCK:
+                if "order" not in plan:
+                    plan.update(_SignedGather._gradient_plan(plan["maps"], ctx.n))
         g = torch.cat([(gi if gi is not None else torch.zeros(sh, dtype=plan["sign"].dtype, device=plan["sign"].device))
                        .reshape(-1) for gi, sh in zip(grads, ctx.shapes, strict=True)])
         vals = g * plan["sign"].to(g.dtype)

@@ -3,6 +3,9 @@ its values and its parameter gradient equal those of plain indexing
 (``flat[index] * sign`` under autograd) on maps with repeated parameters,
 negated and zero entries; no GPU needed."""
 
+import threading
+import time
+
 import torch
 
 from gm_attention_amd.nn import fused_factored
@@ -70,3 +73,30 @@ def test_signed_gather_many_uses_takes_the_segment_sum():
     got_grad, = torch.autograd.grad(got, flat, up)
     assert "cols" not in plan
     assert torch.allclose(got_grad, want_grad, rtol=0, atol=1e-12)
+
+
+def test_threads_backwards_on_one_plan_agree(monkeypatch):
+    """A plan's gradient tables are seen whole or not at all."""
+    n = 31
+    maps = _maps(n, [(4, 10), (2, 9)], seed=2)
+    plan, got = dict(maps=maps), []
+    bincount = torch.bincount
+    monkeypatch.setattr(torch, "bincount", lambda *a, **k: (time.sleep(0.05), bincount(*a, **k))[1])
+    start = threading.Barrier(4)
+
+    def step(i):
+        flat = torch.randn(n, dtype=torch.float64, requires_grad=True)
+        a, b = fused_factored._SignedGather.apply(flat, plan)
+        start.wait()
+        time.sleep(0.01 * i)
+        got.append(torch.autograd.grad(a.sum() + b.sum(), flat)[0])
+
+    threads = [threading.Thread(target=step, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    want = torch.zeros(n, dtype=torch.float64)
+    for i, s in maps:
+        want.index_add_(0, i.reshape(-1), s.reshape(-1))
+    assert len(got) == 4 and all(torch.allclose(g, want, rtol=0, atol=1e-12) for g in got)
