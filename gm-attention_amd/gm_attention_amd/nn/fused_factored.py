@@ -1067,18 +1067,46 @@ class GroupedStreams:
     zw_g: Tensor | None = None  # (E, 4): r e^{i phi}, e^{i gamma} (order-1 phases) in grouping order
     group_order: Tensor | None = None
 
-    def bytes(self) -> int:
-        """Device memory of the streams (``perm`` is the grouping's own)."""
+    def bytes(self, phases: bool = False) -> int:
+        """Device memory of the streams (``perm`` is the grouping's own); ``phases``: with the phase rows they lack."""
         held = (self.inv, self.rho_g, self.phase_g, self.target_g, self.zw_g)
-        return sum(t.numel() * t.element_size() for t in held if t is not None)
+        taken = sum(t.numel() * t.element_size() for t in held if t is not None)
+        return taken + (16 * self.rho_g.numel() * self.rho_g.element_size() if phases and self.phase_g is None else 0)
 
 
 _STREAMS: OrderedDict[tuple, tuple[Any, GroupedStreams]] = OrderedDict()
-#: Streams kept whatever they take; beyond these many, the least recently used
-#: go once they all take more than this share of the device's memory.  (A model
-#: of two stages has six edge sets with streams: with three hierarchies in turn
-#: a bound of eight sets alone rebuilt them on every pass, 80 of 243 ms.)
-STREAMS_KEPT, STREAMS_SHARE = 8, 0.125
+#: Streams kept whatever they take: the last ones used.  Older ones stay while a
+#: device's streams take no more together than these would with phase rows, or
+#: than this share of the device's memory (2.2 GB of 288).  A model of two
+#: stages reads the streams of six edge sets: with three hierarchies in turn
+#: (128x256, B = 8: 0.9 GB) eight sets alone are rebuilt on every pass, 80 of
+#: 243 ms.
+STREAMS_KEPT, STREAMS_SHARE = 8, 1 / 128
+
+
+def release_streams() -> None:
+    """Gives back every edge set's streams (:func:`grouped_streams`); a later call on a set makes its own again."""
+    with assembly.LOCK:
+        _STREAMS.clear()
+
+
+def _trim_streams() -> None:
+    """Drops the streams of edge sets that are gone, then the least recently
+    used ones beyond what their own device's bound allows."""
+    for key in [k for k, (owner, _) in _STREAMS.items() if owner() is None]:
+        del _STREAMS[key]
+    entries = [(key, s, s.inv.device) for key, (_, s) in _STREAMS.items()]
+    allowed: dict[torch.device, float] = {}
+    held: dict[torch.device, int] = {}
+    for i, (_, s, device) in enumerate(entries):
+        held[device] = held.get(device, 0) + s.bytes()
+        if i >= len(entries) - STREAMS_KEPT:
+            allowed[device] = allowed.get(device, 0) + s.bytes(phases=True)
+    for key, s, device in entries[:-STREAMS_KEPT]:
+        share = STREAMS_SHARE * _device_memory(device.index or 0) if device.type == "cuda" else 0.0
+        if held[device] > max(allowed.get(device, 0), share):
+            del _STREAMS[key]
+            held[device] -= s.bytes()
 
 
 def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, dtype: torch.dtype,
@@ -1089,10 +1117,9 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
            pt, dtype, phases)
     hit = _STREAMS.get(key)
     if hit is not None and hit[0]() is edges.edge_index:
-        try:
-            _STREAMS.move_to_end(key)
-        except KeyError:  # dropped by another thread meanwhile
-            pass
+        with assembly.LOCK:
+            if key in _STREAMS:  # not dropped by another thread meanwhile
+                _STREAMS.move_to_end(key)
         return hit[1]
     with torch.profiler.record_function("gm::kernel/group_streams"):
         perm = order
@@ -1113,16 +1140,10 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
         zw_g = torch.stack([a1.real, a1.imag, t1.real, t1.imag], dim=1).to(dtype).contiguous()
         streams = GroupedStreams(perm, inv, rho_g, phase_g, edges.target_index.index_select(0, perm).contiguous(), pa,
                                  pt, zw_g)
-    for stale in [k for k, (ref, _) in list(_STREAMS.items()) if ref() is None]:
-        _STREAMS.pop(stale, None)
-    _STREAMS[key] = (weakref.ref(edges.edge_index), streams)
-    held = [s for _, s in list(_STREAMS.values()) if s.inv.device == perm.device]
-    taken = sum(s.bytes() for s in held)
-    most = STREAMS_SHARE * _device_memory(perm.device.index or 0) if perm.is_cuda else 0.0
-    while len(_STREAMS) > STREAMS_KEPT and taken > most:
-        _, (_, dropped) = _STREAMS.popitem(last=False)
-        if dropped.inv.device == perm.device:
-            taken -= dropped.bytes()
+    with assembly.LOCK:
+        _STREAMS[key] = (weakref.ref(edges.edge_index), streams)
+        _STREAMS.move_to_end(key)
+        _trim_streams()
     return streams
 
 

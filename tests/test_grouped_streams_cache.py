@@ -1,0 +1,76 @@
+"""The kept grouped streams (fused_factored.grouped_streams): what stays, what
+goes and what a device's bound counts; on the CPU, where the share of the
+device's memory is none."""
+
+import pytest
+import torch
+
+import problems
+from gm_attention_amd.nn import fused_factored
+
+
+@pytest.fixture(autouse=True)
+def empty(monkeypatch):
+    monkeypatch.setattr(fused_factored, "_STREAMS", type(fused_factored._STREAMS)())
+
+
+def _edges(n, nlat=6):
+    one = problems.discretization(nlat, 2 * nlat).edge_geometry.to("cpu", torch.float32)
+    return [one.tile(2 + i % 3, n_sources=2 * nlat * nlat) for i in range(n)]
+
+
+def _streams(edges, phases=False):
+    order = fused_factored.groups_for(edges, edges.source_index)[0]
+    return fused_factored.grouped_streams(edges, order, 0.5, 5, 3, torch.float32, phases)
+
+
+def _kept():
+    return [s for _, s in fused_factored._STREAMS.values()]
+
+
+def test_no_more_is_kept_than_eight_sets_with_phase_rows_take():
+    sets = _edges(40)
+    for e in sets:
+        s = _streams(e)
+        assert s.phase_g is None and s.bytes(phases=True) == s.bytes() + 64 * e.n_edges
+        kept = _kept()
+        assert kept[-1] is s
+        assert sum(k.bytes() for k in kept) <= sum(k.bytes(phases=True) for k in kept[-8:])
+    assert fused_factored.STREAMS_SHARE <= 1 / 128  # beyond that: of the device's memory
+    assert len(_kept()) > 16  # 36 bytes an edge against 100
+    assert _streams(sets[-1]) is _kept()[-1] and _streams(sets[-8]) is _kept()[-1]  # used again: the last to go
+    fused_factored.release_streams()
+    assert not _kept()
+
+
+def test_sets_with_phase_rows_are_the_last_eight():
+    sets = _edges(12)
+    made = [_streams(e, phases=True) for e in sets]
+    assert all(a is b for a, b in zip(_kept(), made[-8:], strict=False)) and len(_kept()) <= 9
+
+
+def test_streams_go_with_their_edge_set():
+    sets = _edges(3)
+    for e in sets:
+        _streams(e)
+    assert len(_kept()) == 3
+    del sets[0], e
+    _streams(sets[0], phases=True)
+    assert len(_kept()) == 3  # two sets, one of them with and without phase rows
+
+
+def test_one_devices_bound_drops_nothing_of_another():
+    class Elsewhere:
+        """Streams of another device that fit its bound, as far as the bound looks at them."""
+
+        inv = torch.empty(0, device="meta")
+
+        def bytes(self, phases=False):
+            return 0
+
+    owner = torch.zeros(1)
+    fused_factored._STREAMS["other"] = (lambda: owner, Elsewhere())
+    sets = _edges(40)
+    for e in sets:
+        _streams(e)
+    assert len(_kept()) < len(sets) and next(iter(fused_factored._STREAMS)) == "other"
