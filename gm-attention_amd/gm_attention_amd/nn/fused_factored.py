@@ -160,7 +160,9 @@ def source_groups(source_index: Tensor, key: tuple | None = None,
             held, groups = hit
             same = (owner is None) if held is None else (held() is not None and held() is owner)
             if same and groups[0].device == source_index.device:
-                _GROUPS.move_to_end(key)
+                with assembly.LOCK:
+                    if key in _GROUPS:  # not dropped by another thread meanwhile
+                        _GROUPS.move_to_end(key)
                 return groups
     order = torch.argsort(source_index, stable=True)
     group_source, counts = torch.unique_consecutive(source_index[order], return_counts=True)
@@ -168,9 +170,11 @@ def source_groups(source_index: Tensor, key: tuple | None = None,
     group_ptr[1:] = torch.cumsum(counts, dim=0)
     result = (order.contiguous(), group_ptr.contiguous(), group_source.contiguous())
     if key is not None:
-        _GROUPS[key] = (None if owner is None else weakref.ref(owner), result)
-        while len(_GROUPS) > GROUP_CACHE_SIZE:
-            _GROUPS.popitem(last=False)
+        assembly.complete(source_index.device)  # the kernels follow them unchecked, on whatever stream finds them
+        with assembly.LOCK:
+            _GROUPS[key] = (None if owner is None else weakref.ref(owner), result)
+            while len(_GROUPS) > GROUP_CACHE_SIZE:
+                _GROUPS.popitem(last=False)
     return result
 
 
@@ -1066,6 +1070,14 @@ class GroupedStreams:
     pt: int
     zw_g: Tensor | None = None  # (E, 4): r e^{i phi}, e^{i gamma} (order-1 phases) in grouping order
     group_order: Tensor | None = None
+    made_on: int = 0  # the stream they were made on: their memory returns to it
+
+    def outlive(self, stream: Any) -> None:
+        """Keeps their memory for what ``stream`` has queued, should they be dropped meanwhile."""
+        if stream.cuda_stream != self.made_on:
+            for t in (self.perm, self.inv, self.rho_g, self.phase_g, self.target_g, self.zw_g):
+                if t is not None:
+                    t.record_stream(stream)
 
     def bytes(self, phases: bool = False) -> int:
         """Device memory of the streams (``perm`` is the grouping's own); ``phases``: with the phase rows they lack."""
@@ -1112,7 +1124,8 @@ def _trim_streams() -> None:
 def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, dtype: torch.dtype,
                     phases: bool = True) -> GroupedStreams:
     """The grouped streams of ``edges`` under ``order`` (with the phase rows
-    only where ``phases``), cached while the edge set lives."""
+    only where ``phases``), complete on return and cached while the edge set
+    lives."""
     key = (id(edges.edge_index), edges.edge_index.data_ptr(), int(edges.n_edges), order.data_ptr(), float(cutoff), pa,
            pt, dtype, phases)
     hit = _STREAMS.get(key)
@@ -1120,6 +1133,8 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
         with assembly.LOCK:
             if key in _STREAMS:  # not dropped by another thread meanwhile
                 _STREAMS.move_to_end(key)
+        if order.is_cuda:
+            hit[1].outlive(torch.cuda.current_stream(order.device))
         return hit[1]
     with torch.profiler.record_function("gm::kernel/group_streams"):
         perm = order
@@ -1140,6 +1155,11 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
         zw_g = torch.stack([a1.real, a1.imag, t1.real, t1.imag], dim=1).to(dtype).contiguous()
         streams = GroupedStreams(perm, inv, rho_g, phase_g, edges.target_index.index_select(0, perm).contiguous(), pa,
                                  pt, zw_g)
+    if perm.is_cuda and torch.cuda.is_current_stream_capturing():
+        return streams  # the graph's own: no numbers in them before its replay, and no waiting for them here
+    if perm.is_cuda:
+        streams.made_on = torch.cuda.current_stream(perm.device).cuda_stream
+    assembly.complete(perm.device)  # the kernels follow them unchecked, on whatever stream finds them
     with assembly.LOCK:
         _STREAMS[key] = (weakref.ref(edges.edge_index), streams)
         _STREAMS.move_to_end(key)

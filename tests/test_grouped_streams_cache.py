@@ -74,3 +74,30 @@ def test_one_devices_bound_drops_nothing_of_another():
     for e in sets:
         _streams(e)
     assert len(_kept()) < len(sets) and next(iter(fused_factored._STREAMS)) == "other"
+
+
+def test_groups_and_streams_are_complete_before_they_are_kept(monkeypatch):
+    """Another stream or thread that finds them waits for nothing."""
+    kept = []
+    monkeypatch.setattr(fused_factored, "_GROUPS", type(fused_factored._GROUPS)())
+    monkeypatch.setattr(fused_factored.assembly, "complete",
+                        lambda device: kept.append((len(fused_factored._GROUPS), len(fused_factored._STREAMS))))
+    edges, = _edges(1)
+    _streams(edges)
+    assert kept == [(0, 0), (1, 0)] and len(fused_factored._GROUPS) == len(fused_factored._STREAMS) == 1
+    _streams(edges)
+    assert len(kept) == 2
+
+
+@pytest.mark.gpu
+def test_streams_found_behind_a_busy_stream_are_complete(cuda):
+    edges = problems.discretization(9, 18).edge_geometry.to(cuda, torch.float32)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(50_000_000)
+        got = _streams(edges, phases=True)
+        assert stream.query()
+    assert got.made_on == stream.cuda_stream and _streams(edges, phases=True) is got  # on the default stream
+    order = torch.argsort(edges.source_index, stable=True)
+    assert torch.equal(got.perm, order) and torch.equal(got.target_g, edges.target_index[order])
