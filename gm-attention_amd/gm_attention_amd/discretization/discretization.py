@@ -35,9 +35,10 @@ class SphericalDiscretization:
         self.frames = frames.contiguous()
         self.edge_geometry = edge_geometry
         self.coverage_radius = float(coverage_radius)
-        # kept where the builder computed them: at 256x512 they are 126 MB, and their copy to the host was 25 of the
-        # 36 ms that from_grid took on a GPU grid
+        # one sample's, kept where the builder computed them (8 of a coverage edge's 232 bytes): at 256x512 they are
+        # 126 MB, and their copy to the host was 25 of the 36 ms that from_grid took on a GPU grid
         self._exact_distances = None if exact_distances is None else exact_distances.detach().to(torch.float64)
+        self._exact_copies = 1  # samples whose edges follow each other, all with these distances
         self._radius_cache: dict[float, EdgeGeometry] = {self._key(coverage_radius): edge_geometry}
 
     @staticmethod
@@ -78,6 +79,7 @@ class SphericalDiscretization:
         if key not in self._radius_cache:
             if self._exact_distances is not None:
                 mask = (self._exact_distances <= radius + EXACT_SLACK).to(self.edge_geometry.distances.device)
+                mask = mask.repeat(self._exact_copies)
             else:
                 mask = within_cutoff(self.edge_geometry.distances, radius)
             self._radius_cache[key] = self.edge_geometry.select(mask)
@@ -94,8 +96,9 @@ class SphericalDiscretization:
         union = SphericalDiscretization(
             self.grid.tile(count), self.frames.repeat(count, 1, 1),
             self.edge_geometry.tile(count, n_sources=self.n_nodes), self.coverage_radius,
-            None if self._exact_distances is None else self._exact_distances.repeat(count),
+            self._exact_distances,
         )
+        union._exact_copies = self._exact_copies * count
         coverage = self._key(self.coverage_radius)
         for key, edges in self._radius_cache.items():
             if key != coverage:
@@ -104,10 +107,11 @@ class SphericalDiscretization:
 
     def to(self, device=None, dtype=None) -> SphericalDiscretization:
         exact = self._exact_distances
-        if exact is not None and device is not None and torch.device(device).type == "cpu":
-            exact = exact.cpu()  # nothing of a discretization on the host stays on a GPU
+        if exact is not None and device is not None and exact.device.type != "cpu":
+            exact = exact.to(device)  # with the tables, to the host or another GPU; on the host they stay
         moved = SphericalDiscretization(self.grid.to(device, dtype), self.frames.to(device=device, dtype=dtype),
                                         self.edge_geometry.to(device, dtype), self.coverage_radius, exact)
+        moved._exact_copies = self._exact_copies
         coverage = self._key(self.coverage_radius)
         for key, edges in self._radius_cache.items():
             if key != coverage:

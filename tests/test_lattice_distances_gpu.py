@@ -8,9 +8,38 @@ import torch
 from gm_attention_amd.discretization.discretization import SphericalDiscretization
 from gm_attention_amd.discretization.grid import build_equiangular_grid
 
-pytestmark = pytest.mark.gpu
 
 
+def test_samples_share_their_distances_and_follow_a_move():
+    one = SphericalDiscretization.from_grid(build_equiangular_grid(9, 16), 0.9)
+    two = one.tile(2)
+    six = two.to("cpu", torch.float32).tile(3)
+    assert two._exact_distances.data_ptr() == one._exact_distances.data_ptr() and six._exact_distances.numel() == one.n_edges
+    for union, count in ((two, 2), (six, 6)):
+        want = one.edges_within(0.5).tile(count, n_sources=one.n_nodes)
+        got = union.edges_within(0.5)
+        assert torch.equal(got.edge_index, want.edge_index) and torch.equal(got.row_ptr, want.row_ptr)
+
+    class OnAnotherGpu:
+        device = torch.device("cuda:0")
+        moved_to = None
+
+        def detach(self):
+            return self
+
+        def to(self, where):
+            if isinstance(where, str):
+                self.moved_to = where
+            return self
+
+    one._exact_distances = held = OnAnotherGpu()
+    one.to(dtype=torch.float32)
+    assert held.moved_to is None
+    one.to("cpu")
+    assert held.moved_to == "cpu"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nlat,nlon", [(16, 32), (19, 36)])
 def test_radius_subsets_are_the_same_wherever_the_distances_live(nlat, nlon, cuda):
     """Whole shells (radii on the lattice's own spacing) chosen on the GPU, on the
