@@ -906,9 +906,12 @@ class HeadsLayout:
         return columns
 
 
-#: Device memory the padded shares' mixes, mix gradients and rows may take (a share of the device's):
-#: an uneven layer that fits without padding still fits.
-PADDED_SHARE = 0.25
+#: Device memory that padding a layer's heads may add to what the layer keeps for
+#: its backward (the shares' rows and mixes, less those of the heads' own plan),
+#: as a share of the device's: 4.5 GB of 288, so a model of eight such layers
+#: grows by at most an eighth of the device.  Sizes decide it and not the memory
+#: that is free, which a recomputed forward would find changed.
+PADDED_SHARE = 1 / 64
 
 
 @functools.cache
@@ -925,12 +928,13 @@ def _padded_shares(kernel: Any, split: int, K: int, heads: int, size: tuple[int,
     heads over 0.75 M edges (45x91, B = 3): compiled-in slots 250 + 89 a
     16-column tile (3 tiles 517, 7 tiles 872), runtime slots 400 a tile (5:
     1,800, 8: 3,535), the generic kernels 650 a tile (3: 1,950, 4: 2,290, 7:
-    4,640).  ``size`` is (nodes, edges): the padding's memory is bounded."""
+    4,640).  ``size`` is (nodes, edges): what the padding adds to the layer's
+    memory is bounded (:data:`PADDED_SHARE`)."""
     env = (os.environ.get("GM_FACTORED_LANES", "1"), os.environ.get("GM_FACTORED_STATIC", "1"))
     key = ("_padded_shares", split, K, env)
     held = kernel.__dict__.get(key)
     if held is None:
-        held = (0, 0, 0)
+        held = (0, 0, 0)  # the shares, and the reals a head's rows (an edge) and mixes (a node) grow by
         out = kernel.field_type_out
         shares = -(-max(out.multiplicities) // 4)
         unit = padded_unit(kernel, shares)
@@ -943,14 +947,17 @@ def _padded_shares(kernel: Any, split: int, K: int, heads: int, size: tuple[int,
             tiles = lambda p: -(-(2 * p.wc + p.wr) // 16)  # noqa: E731
             lanes = own_ok and _lanes_apply(own, own_hp, own_pa, own_pt)
             if shares * (250 + 89 * tiles(hp.plan)) < max(split, 1) * (400 if lanes else 650) * tiles(own_hp.plan):
-                held = (shares, hp.plan.d_out, 2 * hp.plan.wc + hp.plan.wr)
+                grown = [shares * mine - max(split, 1) * theirs for mine, theirs in
+                         ((hp.plan.d_out, own_hp.plan.d_out),
+                          (K * (2 * hp.plan.wc + hp.plan.wr), K * (2 * own_hp.plan.wc + own_hp.plan.wr)))]
+                held = (shares, *grown)
         kernel.__dict__[key] = held
-    shares, d_out, C = held
+    shares, row, mix = held
     if not shares or size is None or device.type != "cuda":
         return 0
     nodes, edges = size
-    taken = 4 * heads * shares * (edges * d_out + 2 * nodes * K * C)
-    return shares if taken <= PADDED_SHARE * _device_memory(device.index or 0) else 0
+    added = 4 * heads * (edges * row + nodes * mix)
+    return shares if added <= PADDED_SHARE * _device_memory(device.index or 0) else 0
 
 
 def heads_layout(kernels: list[Any], dtype: torch.dtype, K: int | None = None, size: tuple[int, int] | None = None,

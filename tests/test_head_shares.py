@@ -128,3 +128,29 @@ def test_depthwise_channel_groups_partition_the_copies(field, groups):
     cols, rows = torch.cat(cols), torch.cat(rows)
     assert torch.equal(cols.sort().values, torch.arange(ft.dimension))
     assert torch.equal(rows.sort().values, torch.arange(n_rows))
+
+
+@pytest.mark.parametrize("field,heads,shares", [({0: 24, 1: 12, 2: 6}, 6, 1), ({0: 10, 1: 6, 2: 2}, 2, 2)])
+def test_padding_adds_at_most_its_share_of_the_memory(field, heads, shares, monkeypatch):
+    """What padding adds to a layer's kept rows and mixes decides it: just below
+    the share it is taken, just above it is not, and a layer many times the
+    small grids' size stays on its own plan."""
+    memory = 288 * 10 ** 9
+    monkeypatch.setattr(fused_factored, "_device_memory", lambda index: memory)
+    kernel = SO2MHSA(SO2FieldType(field), heads, cutoff=0.3, batched=True, dtype=torch.float32).heads[0].value
+    split = fused_factored.head_split(kernel, 17)
+
+    def plan(nodes, edges):
+        return fused_factored._padded_shares(kernel, split, 17, heads, (nodes, edges), torch.device("cuda", 0))
+
+    padded = fused_factored.heads_plan(fused_factored.padded_unit(kernel, shares)).plan
+    own = fused_factored.heads_plan(fused_factored.sub_head(kernel, max(split, 1))).plan
+    more = [heads * (shares * p - max(split, 1) * q) for p, q in
+            ((padded.d_out, own.d_out), (2 * padded.wc + padded.wr, 2 * own.wc + own.wr))]
+    assert all(m > 0 for m in more)
+    bound = memory * fused_factored.PADDED_SHARE
+    assert bound <= memory / 64
+    nodes = int(bound / (4 * (60 * more[0] + 17 * more[1])))
+    assert plan(nodes, 60 * nodes) == shares and plan(nodes + 100, 60 * (nodes + 100)) == 0
+    assert plan(12285, 750_000) == shares  # 45x91, three samples
+    assert plan(524_288, 63_000_000) == 0  # 256x512, four

@@ -14,7 +14,8 @@ def test_samples_share_their_distances_and_follow_a_move():
     one = SphericalDiscretization.from_grid(build_equiangular_grid(9, 16), 0.9)
     two = one.tile(2)
     six = two.to("cpu", torch.float32).tile(3)
-    assert two._exact_distances.data_ptr() == one._exact_distances.data_ptr() and six._exact_distances.numel() == one.n_edges
+    assert two._exact_distances.data_ptr() == one._exact_distances.data_ptr()
+    assert six._exact_distances.numel() == one.n_edges
     for union, count in ((two, 2), (six, 6)):
         want = one.edges_within(0.5).tile(count, n_sources=one.n_nodes)
         got = union.edges_within(0.5)
