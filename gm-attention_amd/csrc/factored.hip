@@ -350,20 +350,28 @@ constexpr int kAggStep = 4;  // edges a step: 55 VGPRs, eight waves a SIMD (eigh
 // WPT: waves a target.  One, or a workgroup's four, each summing a quarter of the
 // target's edges (whole steps), the quarters added in order through LDS.  Small
 // launches are bound by their longest rows -- a polar target's edges are one
-// wave's serial chain of loads -- and take four: 32x64, B = 1, four heads 99 ->
-// 31 us; 64x128, B = 1, eight heads 322 -> 128; 181x360, B = 1 1573 -> 1108.  Once
-// the launch fills the chip for many rows' time the bytes bound it (4.4-5.0 TB/s)
-// and the split only adds its start and its sum: 131,072 targets of 40 pieces
-// 2.10 ms with one wave, 2.16 with four (B = 4 of 128x256), 2.15 and 2.35 (B = 1
-// of 256x512); 65,536 of 80 pieces 2.12 and 2.27.  The line between lies between
-// 65,536 and 131,072 targets of 40 pieces.
-constexpr int64_t kAggWidePieces = int64_t(7) << 19;
+// wave's serial chain of loads -- and take four, one wave -> four at 8, 40 and 80
+// pieces a target: 32x64, B = 1 83 -> 19, 106 -> 35, 193 -> 60 us; 64x128, B = 5 423
+// -> 337, 677 -> 557, 1474 -> 1334; 181x360, B = 1 1150 -> 641, 1683 -> 1068, 3694 ->
+// 2520.  Once the launch fills the chip for many rows' time the bytes bound it
+// (4.4-5.0 TB/s) and the split only adds its start and its sum: 98,304 targets
+// (64x128, B = 12) 814 -> 831, 1420 -> 1339, 2950 -> 3150; 115,200 (240x480, B = 1)
+// 1040 -> 1111, 1959 -> 2111, 4200 -> 4560; 524,288 (256x512, B = 4) 4778 -> 5560,
+// 7802 -> 8417.  The line falls with the pieces (the bytes) from 40 up and not
+// below, where the rows' chains are as long: 91,750 targets of up to 40 pieces,
+// 45,875 of 80.  It cannot see the rows: many samples of a grid with short ones
+// lose (16x32, B = 128: 391 -> 465, 681 -> 782).
+//
+// Four waves a target take the spread order whatever the ranges' balance: with
+// contiguous ranges 64x128, B = 6 takes 480, 796 and 1784 us (one wave 426, 720 and
+// 1583), spread 435, 719 and 1587; B = 5 and 10 gain 6-8% too.
+constexpr int64_t kAggWidePieces = int64_t(7) << 19, kAggFewPieces = 40;
 template <int P, bool B16 = false, int WPT = 1>
 __global__ __launch_bounds__(256) void aggregate_heads_vec_kernel(AggHeadsArgs a) {
   constexpr int kPerBlock = kWavesPerBlock / WPT;  // targets a workgroup
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t i = xcd_balanced_block(blockIdx.x, gridDim.x, a.row_ptr, a.n_targets, kPerBlock) * kPerBlock +
-                    (WPT == 1 ? wv : 0);
+  const int64_t i = WPT == 1 ? xcd_balanced_block(blockIdx.x, gridDim.x, a.row_ptr, a.n_targets, kPerBlock) * kPerBlock + wv
+                             : xcd_spread_block(blockIdx.x, gridDim.x);
   const int lane = threadIdx.x & 63;
   if (i >= a.n_targets) return;  // with WPT > 1 the whole workgroup
   const int q4 = a.d_out / 4, W4 = a.H * q4, Ha = a.H / a.split;
@@ -3419,7 +3427,7 @@ namespace {
 
 template <int P, bool B16>
 void launch_aggregate_vec(const AggHeadsArgs& a, int64_t pieces, hipStream_t stream) {
-  if (a.n_targets <= kAggWidePieces / pieces)
+  if (a.n_targets <= kAggWidePieces / (pieces > kAggFewPieces ? pieces : kAggFewPieces))
     hipLaunchKernelGGL((aggregate_heads_vec_kernel<P, B16, kWavesPerBlock>), dim3((unsigned)a.n_targets), dim3(256), 0,
                        stream, a);
   else

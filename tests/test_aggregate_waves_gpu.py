@@ -8,12 +8,13 @@ from gm_attention_amd import _native
 
 pytestmark = pytest.mark.gpu
 
-LINE = 7 << 19  # targets x 16-byte output pieces up to which a target takes four waves
+LINE = 7 << 19  # targets x 16-byte output pieces (40 or more) up to which a target takes four waves
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,d_out,n", [(1, 4, 1), (8, 20, 9), (6, 20, 700), (16, 20, 333), (48, 16, 65),
-                                       (16, 64, LINE // 256), (16, 64, LINE // 256 + 1)])
+                                       (16, 64, LINE // 256), (16, 64, LINE // 256 + 1),
+                                       (1, 32, LINE // 40), (1, 32, LINE // 40 + 1)])
 def test_aggregate_on_both_sides_of_the_line(H, d_out, n, dtype, cuda):
     """Degrees of no edge, fewer than a wave's step, quarters that end early and
     rows of thousands, against float64 sums: n products added in any order are
