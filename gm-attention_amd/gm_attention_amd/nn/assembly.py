@@ -56,6 +56,11 @@ def complete(device: torch.device) -> None:
         torch.cuda.current_stream(device).synchronize()
 
 
+def stream_handle(device: torch.device) -> int:
+    """The device's current stream, without the object ``torch.cuda.current_stream`` makes (a microsecond)."""
+    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
+
+
 class Plan:
     """Where every entry of a construction's forms comes from, found on the
     parameters' device and complete on return."""
@@ -77,7 +82,9 @@ class Plan:
         self.codes = torch.where(position < 0, -1, self._code(self.in_starts, position, flat < 0)).reshape(1, -1)
         counts = torch.bincount(position.clamp_min(-1) + 1, minlength=2)[1:]
         self.most = int(counts.max())  # uses of one parameter entry
+        self.made_on = stream_handle(device)
         self.back: Tensor | None = None
+        self.back_made_on = 0
         complete(device)
 
     @staticmethod
@@ -103,13 +110,15 @@ class Plan:
                                        device=at.device)
                     table[rank, at] = self._code(self.out_starts, used[order], (codes[order] & 1) == 1)
                     complete(table.device)
+                    self.back_made_on = stream_handle(table.device)
                     self.back = table
         return self.back
 
 
-def _gather(tensors: Sequence[Tensor | None], codes: Tensor) -> Tensor:
-    """``signed_gather`` on the current stream, which the table's memory then outlives."""
-    codes.record_stream(torch.cuda.current_stream(codes.device))
+def _gather(tensors: Sequence[Tensor | None], codes: Tensor, made_on: int) -> Tensor:
+    """``signed_gather`` on the current stream; a table made on another one outlives what this has queued."""
+    if stream_handle(codes.device) != made_on:
+        codes.record_stream(torch.cuda.current_stream(codes.device))
     return _native.signed_gather(tensors, codes)
 
 
@@ -120,7 +129,7 @@ class _Assemble(torch.autograd.Function):
     def forward(ctx: Any, plan: Plan, *params: Tensor | None) -> tuple:
         ctx.plan = plan
         ctx.set_materialize_grads(False)
-        out = _gather(params, plan.codes)
+        out = _gather(params, plan.codes, plan.made_on)
         return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.out_starts, plan.form_shapes))
 
     @staticmethod
@@ -136,7 +145,7 @@ class _Transposed(torch.autograd.Function):
     def forward(ctx: Any, plan: Plan, *grads: Tensor | None) -> tuple:
         ctx.plan = plan
         ctx.set_materialize_grads(False)
-        out = _gather(_held(grads), plan.gradient_codes())
+        out = _gather(_held(grads), plan.gradient_codes(), plan.back_made_on)
         return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.in_starts, plan.shapes))
 
     @staticmethod
@@ -165,9 +174,13 @@ def takes(params: Sequence[Tensor]) -> bool:
     if not 0 < len(params) <= MAX_SOURCES:
         return False
     device = params[0].device
-    return (device.type == "cuda" and device.index == torch.cuda.current_device() and not _transformed()
-            and all(p.dtype == torch.float32 and p.device == device and p.is_contiguous() and not p.is_neg()
-                    and type(p) in _PLAIN for p in params))
+    if device.type != "cuda" or device.index != torch.cuda.current_device() or _transformed():
+        return False
+    for p in params:  # a loop of cheap tests: small layers have sixty parameters and half a millisecond
+        if (p.dtype is not torch.float32 or p.get_device() != device.index or not p.is_contiguous() or p.is_neg()
+                or type(p) not in _PLAIN):
+            return False
+    return True
 
 
 def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[list[Tensor]], list[Tensor]],

@@ -1079,9 +1079,10 @@ class GroupedStreams:
     group_order: Tensor | None = None
     made_on: int = 0  # the stream they were made on: their memory returns to it
 
-    def outlive(self, stream: Any) -> None:
-        """Keeps their memory for what ``stream`` has queued, should they be dropped meanwhile."""
-        if stream.cuda_stream != self.made_on:
+    def outlive_queue(self) -> None:
+        """Keeps their memory for what the current stream has queued, should they be dropped meanwhile."""
+        if assembly.stream_handle(self.perm.device) != self.made_on:
+            stream = torch.cuda.current_stream(self.perm.device)
             for t in (self.perm, self.inv, self.rho_g, self.phase_g, self.target_g, self.zw_g):
                 if t is not None:
                     t.record_stream(stream)
@@ -1140,8 +1141,7 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
         with assembly.LOCK:
             if key in _STREAMS:  # not dropped by another thread meanwhile
                 _STREAMS.move_to_end(key)
-        if order.is_cuda:
-            hit[1].outlive(torch.cuda.current_stream(order.device))
+        hit[1].outlive_queue()
         return hit[1]
     with torch.profiler.record_function("gm::kernel/group_streams"):
         perm = order
@@ -1164,8 +1164,7 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
                                  pt, zw_g)
     if perm.is_cuda and torch.cuda.is_current_stream_capturing():
         return streams  # the graph's own: no numbers in them before its replay, and no waiting for them here
-    if perm.is_cuda:
-        streams.made_on = torch.cuda.current_stream(perm.device).cuda_stream
+    streams.made_on = assembly.stream_handle(perm.device)
     assembly.complete(perm.device)  # the kernels follow them unchecked, on whatever stream finds them
     with assembly.LOCK:
         _STREAMS[key] = (weakref.ref(edges.edge_index), streams)

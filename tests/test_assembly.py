@@ -83,7 +83,7 @@ class _Owner:
 def on_cpu(monkeypatch):
     """Assembly on the CPU: the launch replaced by its definition."""
     monkeypatch.setattr(assembly, "takes", lambda params: True)
-    monkeypatch.setattr(assembly, "_gather", lambda sources, codes: _gather(sources, codes).float())
+    monkeypatch.setattr(assembly, "_gather", lambda sources, codes, made_on: _gather(sources, codes).float())
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
 
 
