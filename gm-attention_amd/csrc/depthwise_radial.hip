@@ -243,7 +243,16 @@ __device__ __forceinline__ bool tile_live(const RadialConvArgs& a, int m) {
 // copies: 10.4 -> 7.6 ms; 91x181, B = 1, 64 + 64 + 64 copies (two walks): 1.21 ->
 // 0.46.  What is left is latency: three waves a SIMD (166 VGPRs, three workgroups
 // of four by LDS) 7.6 ms, two 9.1, four 13.0 (spills).
-constexpr int kFGroups = kRNC / 4;       // groups of sixteen complex copies
+//
+// G: groups of sixteen complex copies the kernel holds registers and tables for,
+// one (up to four tiles), two (eight) or all.  A group takes its four products
+// whatever it holds of its sixteen copies, so narrow fields need the waves: in the
+// kernel of four groups fields of up to sixteen copies took 3.7 ms at 256x512, B =
+// 4 (16 + 8 + 4; 3.3 with the coefficients as rows); one group's takes 126 VGPRs,
+// four waves a SIMD, 2.9 ms (five, spilling: 5.1).  Two: 160 VGPRs, three waves, 16
+// + 16 + 16 4.8 -> 4.5 (four, spilling: 6.6).  Against the coefficients as rows only
+// fields of four complex copies at that size stay behind (16 + 4: 2.62 -> 2.83).
+constexpr int kFGroups = kRNC / 4;
 
 struct EdgeFactors {                     // of a wave's sixteen edges
   float4 f[2][16];                       // per frequency: w tau, p conj(w tau)
@@ -277,16 +286,17 @@ __device__ __forceinline__ int slot_row(const RadialConvArgs& a, int slot, int r
   return m < a.nc ? 16 * (kRNS + m) + 4 * (row % 4) + p : -1;
 }
 
-template <int NB, bool SPLIT>
-__global__ __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(3))) void
+template <int NB, bool SPLIT, int G>
+__global__ __launch_bounds__(kRThreads) __attribute__((amdgpu_waves_per_eu(G == 1 ? 4 : 3))) void
 conv_radial_forward_kernel(RadialConvArgs a) {
+  constexpr int kSlots = kRNS + 4 * G;
   // lane l of slot m: features 4 (l / 16) .. + 3 of the slot's row l % 16
-  __shared__ __attribute__((aligned(16))) float4 rf_s[SPLIT ? 1 : kRNT * kWave];
-  __shared__ __attribute__((aligned(16))) u32x4 rs_s[SPLIT ? kRNT * 2 * kWave : 1];
-  __shared__ __attribute__((aligned(16))) float4 bias_s[kRNT * 16];  // four of the same: the product starts from it
+  __shared__ __attribute__((aligned(16))) float4 rf_s[SPLIT ? 1 : kSlots * kWave];
+  __shared__ __attribute__((aligned(16))) u32x4 rs_s[SPLIT ? kSlots * 2 * kWave : 1];
+  __shared__ __attribute__((aligned(16))) float4 bias_s[kSlots * 16];  // four of the same: the product starts from it
   __shared__ float w1s[16 * kRMaxBasis + 16];
   __shared__ EdgeFactors ef_s[kRWaves];
-  for (int i = threadIdx.x; i < kRNT * kWave; i += kRThreads) {
+  for (int i = threadIdx.x; i < kSlots * kWave; i += kRThreads) {
     const int m = i / kWave, l = i % kWave, row = slot_row(a, m, l & 15);
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (row >= 0) {
@@ -316,10 +326,10 @@ conv_radial_forward_kernel(RadialConvArgs a) {
   if (i >= a.n_nodes) return;
   EdgeFactors& ef = ef_s[wave];
   // the lane's copy of each group: its column (a dead copy reads column 0, and is not stored) and frequency
-  int col[kFGroups], freq[kFGroups];
-  bool live_copy[kFGroups];
+  int col[G], freq[G];
+  bool live_copy[G];
 #pragma unroll
-  for (int g = 0; g < kFGroups; ++g) {
+  for (int g = 0; g < G; ++g) {
     col[g] = freq[g] = 0;
     live_copy[g] = 4 * g + (c >> 2) < a.nc;
 #pragma unroll
@@ -330,11 +340,11 @@ conv_radial_forward_kernel(RadialConvArgs a) {
       }
   }
   const int groups = (a.nc + 3) >> 2;
-  float accs[kRNS], accc[kFGroups][2];
+  float accs[kRNS], accc[G][2];
 #pragma unroll
   for (int m = 0; m < kRNS; ++m) accs[m] = 0.f;
 #pragma unroll
-  for (int g = 0; g < kFGroups; ++g) accc[g][0] = accc[g][1] = 0.f;
+  for (int g = 0; g < G; ++g) accc[g][0] = accc[g][1] = 0.f;
   const int64_t e0 = a.row_ptr[i], e1 = a.row_ptr[i + 1];
   // the next tile's edge rows and sources are requested while this tile computes
   const int n = 1 + (q & 1);
@@ -394,13 +404,13 @@ conv_radial_forward_kernel(RadialConvArgs a) {
     };
     // m = A z + B u with z = (w tau) x and u = w p conj(tau x) = (p conj(w tau)) conj(x)
 #pragma unroll
-    for (int g = 0; g < kFGroups; ++g) {
+    for (int g = 0; g < G; ++g) {
       if (g < groups) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) x[k] = xn[k];
-        if (g + 1 < kFGroups && g + 1 < groups) {
+        if (g + 1 < G && g + 1 < groups) {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) xn[k] = ld2(vr[k] + col[g + 1 < kFGroups ? g + 1 : 0]);
+          for (int k = 0; k < 4; ++k) xn[k] = ld2(vr[k] + col[g + 1 < G ? g + 1 : 0]);
         } else {
           scalars();
         }
@@ -443,7 +453,7 @@ conv_radial_forward_kernel(RadialConvArgs a) {
     if (q == 0 && 16 * m + c < a.a0) oi[16 * m + c] = v;
   }
 #pragma unroll
-  for (int g = 0; g < kFGroups; ++g) {
+  for (int g = 0; g < G; ++g) {
     const float2 v = make_float2(rows(accc[g][0]), rows(accc[g][1]));
     if (q == 0 && live_copy[g]) *reinterpret_cast<float2*>(oi + col[g]) = v;
   }
@@ -811,12 +821,22 @@ int64_t launch_backward_groups(const RadialConvArgs& a, float* partial, int64_t 
   return rows * groups;
 }
 
-template <int NB>
+template <int NB, int G>
 void launch_forward(const RadialConvArgs& a, dim3 grid, hipStream_t s) {
   if (split_products())
-    hipLaunchKernelGGL((conv_radial_forward_kernel<NB, true>), grid, dim3(kRThreads), 0, s, a);
+    hipLaunchKernelGGL((conv_radial_forward_kernel<NB, true, G>), grid, dim3(kRThreads), 0, s, a);
   else
-    hipLaunchKernelGGL((conv_radial_forward_kernel<NB, false>), grid, dim3(kRThreads), 0, s, a);
+    hipLaunchKernelGGL((conv_radial_forward_kernel<NB, false, G>), grid, dim3(kRThreads), 0, s, a);
+}
+
+template <int NB>
+void launch_forward(const RadialConvArgs& a, dim3 grid, hipStream_t s) {
+  if (a.nc <= 4)
+    launch_forward<NB, 1>(a, grid, s);
+  else if (a.nc <= 8)
+    launch_forward<NB, 2>(a, grid, s);
+  else
+    launch_forward<NB, kFGroups>(a, grid, s);
 }
 
 int prepare(RadialConvArgs& a, const float* v, const float* rf, const float* rbias, const float* rb, const float* w1,

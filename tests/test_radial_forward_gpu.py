@@ -13,7 +13,7 @@ DEGREES = [0, 1, 15, 16, 17, 33, 0, 100, 2]
 
 @pytest.mark.parametrize("basis", [4, 6, 8])
 @pytest.mark.parametrize("a0,orders", [(4, []), (0, [2]), (12, [1, 2, 2]), (16, [2, 1, 2, 1]), (20, [1] * 5 + [2] * 3),
-                                       (32, [2] * 15), (32, [1, 2] * 8)])
+                                       (32, [2] * 15), (32, [1, 2] * 8), (8, [2, 1, 1, 2, 2]), (28, [1] * 9)])
 def test_partial_and_mixed_groups_over_ragged_rows(a0, orders, basis, cuda):
     """Frequencies mixed within a group, tiles' columns in any order, dead copies in
     the last group, scalars short of a tile, rows of no edge to several tiles.
