@@ -1187,8 +1187,11 @@ def grouped_eligible(hp: HeadsPlan, h_dtype: torch.dtype, K: int) -> tuple[bool,
 def _together(meta: dict, h_g: Tensor) -> bool:
     """Whether a share of every head runs as one launch: float32 streams of
     several heads in the default group order (the heads of a group then run
-    together, sharing its phases and targets in the caches)."""
-    return h_g.dtype == torch.float32 and h_g.shape[0] > 1 and meta["group_order"] is None
+    together, sharing its phases and targets in the caches), as many heads and
+    groups as a launch takes."""
+    groups = -(-meta["group_source"].shape[0] // 8) * 8
+    return (h_g.dtype == torch.float32 and 1 < h_g.shape[0] <= 1024 and groups * h_g.shape[0] < 1 << 31
+            and meta["group_order"] is None)
 
 
 class FactoredHeadsGrouped(torch.autograd.Function):

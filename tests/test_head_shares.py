@@ -154,3 +154,12 @@ def test_padding_adds_at_most_its_share_of_the_memory(field, heads, shares, monk
     assert plan(nodes, 60 * nodes) == shares and plan(nodes + 100, 60 * (nodes + 100)) == 0
     assert plan(12285, 750_000) == shares  # 45x91, three samples
     assert plan(524_288, 63_000_000) == 0  # 256x512, four
+
+
+def test_heads_and_groups_beyond_a_launch_run_head_by_head():
+    def together(heads, groups):
+        meta = dict(group_order=None, group_source=torch.empty(1, dtype=torch.int64).expand(groups))
+        return fused_factored._together(meta, torch.empty(1, 1, 1).expand(heads, 1, 16))
+
+    assert not together(1, 100) and together(2, 100) and together(1024, 100) and not together(1025, 100)
+    assert together(8, (1 << 28) - 8) and not together(8, 1 << 28)
