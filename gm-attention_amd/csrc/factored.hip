@@ -881,7 +881,7 @@ __global__ __launch_bounds__(64) void factored_forward_mfma(FactArgs<float> a) {
 template <int NT>
 __global__ __launch_bounds__(64) void factored_backward_mfma(FactArgs<float> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nb = a.n_blocks, CV = 16 * NT, WP = CV + 1, wc2 = 2 * a.wc, d_out = a.d_out;
+  const int nb = a.n_blocks, CV = 16 * NT, WP = CV + 1, d_out = a.d_out;
   constexpr int ZP = 16 * NT + 4;
   int64_t* eid = reinterpret_cast<int64_t*>(smem);  // [kMT]
   Block* Bd = reinterpret_cast<Block*>(eid + kMT);  // [nb]
@@ -1188,7 +1188,7 @@ __global__ __launch_bounds__(64) void factored_forward_grouped(FactArgs<float> a
 template <int NT>
 __global__ __launch_bounds__(64) void factored_backward_grouped(FactArgs<float> a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int nb = a.n_blocks, CV = 16 * NT, WP = CV + 1, wc2 = 2 * a.wc, d_out = a.d_out;
+  const int nb = a.n_blocks, CV = 16 * NT, WP = CV + 1, d_out = a.d_out;
   int64_t* Tg = reinterpret_cast<int64_t*>(smem);                  // [kMT] targets
   Block* Bd = reinterpret_cast<Block*>(Tg + kMT);                  // [nb]
   float* Ph = reinterpret_cast<float*>(Bd + GM_FACT_MAX_BLOCKS);   // [kMT][kPhaseRow]

@@ -121,7 +121,8 @@ struct WalkArgs {
 // walked one by one, the wave's loop over every box was a chain of scalar loads
 // and each lane stored its own row's next element: 256x512 at three rings, 2048
 // boxes, 15.7M edges, degrees 0.97 ms and edges 1.45 ms; this form takes 0.22 and
-// 0.30 (the edges' 252 MB at 0.85 TB/s; float64 products bound both).  Sixteen targets a wave give a small box and 8192 waves.
+// 0.30 (the edges' 252 MB at 0.85 TB/s; float64 products bound both).  Sixteen
+// targets a wave give a small box and 8192 waves.
 template <bool kEdges>
 __global__ __launch_bounds__(kGeoTile) void geo_walk_kernel(WalkArgs a) {
   __shared__ double pts[kGeoTargets][3];
@@ -191,7 +192,6 @@ __global__ __launch_bounds__(kScanThreads) void geo_scan_kernel(int64_t* __restr
   __syncthreads();
   int64_t run = 0;
   for (int w = 0; w < wave; ++w) run += sums[w];
-#pragma unroll 4
   for (int64_t i = lo; i < hi; i += kWave) {
     int64_t v = i + lane < hi ? row_ptr[i + lane] : 0;
 #pragma unroll
