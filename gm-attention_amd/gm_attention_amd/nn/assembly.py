@@ -122,6 +122,16 @@ def _gather(tensors: Sequence[Tensor | None], codes: Tensor, made_on: int) -> Te
     return _native.signed_gather(tensors, codes)
 
 
+def _forms(plan: Plan, *params: Tensor | None) -> tuple:
+    out = _gather(params, plan.codes, plan.made_on)
+    return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.out_starts, plan.form_shapes))
+
+
+def _gradients(plan: Plan, *grads: Tensor | None) -> tuple:
+    out = _gather(_held(grads), plan.gradient_codes(), plan.back_made_on)
+    return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.in_starts, plan.shapes))
+
+
 class _Assemble(torch.autograd.Function):
     """The forms from the parameters; its gradient is :class:`_Transposed`, and that one's is this one."""
 
@@ -129,14 +139,13 @@ class _Assemble(torch.autograd.Function):
     def forward(ctx: Any, plan: Plan, *params: Tensor | None) -> tuple:
         ctx.plan = plan
         ctx.set_materialize_grads(False)
-        out = _gather(params, plan.codes, plan.made_on)
-        return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.out_starts, plan.form_shapes))
+        return _forms(plan, *params)
 
     @staticmethod
     def backward(ctx: Any, *grads: Tensor | None) -> tuple:
         if all(g is None for g in grads):
             return (None,) * len(ctx.needs_input_grad)
-        out = _Transposed.apply(ctx.plan, *grads)
+        out = (_Transposed.apply if torch.is_grad_enabled() else _gradients)(ctx.plan, *grads)
         return (None, *(g if need else None for g, need in zip(out, ctx.needs_input_grad[1:])))
 
 
@@ -145,14 +154,13 @@ class _Transposed(torch.autograd.Function):
     def forward(ctx: Any, plan: Plan, *grads: Tensor | None) -> tuple:
         ctx.plan = plan
         ctx.set_materialize_grads(False)
-        out = _gather(_held(grads), plan.gradient_codes(), plan.back_made_on)
-        return tuple(out[a:a + s.numel()].view(s) for a, s in zip(plan.in_starts, plan.shapes))
+        return _gradients(plan, *grads)
 
     @staticmethod
     def backward(ctx: Any, *grads: Tensor | None) -> tuple:
         if all(g is None for g in grads):
             return (None,) * len(ctx.needs_input_grad)
-        out = _Assemble.apply(ctx.plan, *_held(grads))
+        out = (_Assemble.apply if torch.is_grad_enabled() else _forms)(ctx.plan, *_held(grads))
         return (None, *(g if need else None for g, need in zip(out, ctx.needs_input_grad[1:])))
 
 
