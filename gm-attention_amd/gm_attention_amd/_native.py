@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import threading
 import weakref
 from pathlib import Path
 from typing import Any
@@ -187,6 +188,17 @@ def _require_device(*tensors: Tensor) -> None:
         _check(t.device == first.device, "every tensor must live on the same device")
 
 
+LOCK = threading.RLock()  # what is kept for edge sets and modules is found by one thread at a time
+
+
+def complete(device: torch.device) -> None:
+    """Waits for what this stream writes: the kernels follow kept tables
+    unchecked, and other streams and threads use them without an event of this
+    one's, so they are complete before anything else can see them."""
+    if device.type == "cuda":
+        torch.cuda.current_stream(device).synchronize()
+
+
 _HOST_DESC: dict[tuple, tuple[Any, Tensor]] = {}
 
 
@@ -233,9 +245,11 @@ def source_major(source: Tensor, row_ptr: Tensor) -> tuple[Tensor, Tensor, Tenso
         degrees = row_ptr[1:] - row_ptr[:-1]
         target = torch.repeat_interleave(torch.arange(n_nodes, device=device), degrees)
         result = (src_ptr.contiguous(), order.contiguous(), target.contiguous())
-    for stale in [k for k, (ref, _) in _GROUPS.items() if ref() is None]:
-        del _GROUPS[stale]
-    _GROUPS[key] = (weakref.ref(source), result)
+    complete(device)
+    with LOCK:
+        for stale in [k for k, (ref, _) in _GROUPS.items() if ref() is None]:
+            del _GROUPS[stale]
+        _GROUPS[key] = (weakref.ref(source), result)
     return result
 
 
@@ -260,11 +274,15 @@ def source_grouped_tables(source: Tensor, row_ptr: Tensor, transport: Tensor) ->
     inv[src_order] = torch.arange(source.shape[0], dtype=torch.int32, device=source.device)
     transport_s = transport.index_select(0, src_order).contiguous()
     result = (target_s.contiguous(), inv, transport_s)
-    for stale in [k for k, (a, b, _) in _GROUPED_TABLES.items() if a() is None or b() is None]:
-        del _GROUPED_TABLES[stale]
-    _GROUPED_TABLES[key] = (weakref.ref(source), weakref.ref(transport), result)
-    while len(_GROUPED_TABLES) > 8:
-        del _GROUPED_TABLES[next(iter(_GROUPED_TABLES))]
+    if source.is_cuda and torch.cuda.is_current_stream_capturing():
+        return result  # the graph's own: no numbers in them before its replay, and no waiting for them here
+    complete(source.device)
+    with LOCK:
+        for stale in [k for k, (a, b, _) in _GROUPED_TABLES.items() if a() is None or b() is None]:
+            del _GROUPED_TABLES[stale]
+        _GROUPED_TABLES[key] = (weakref.ref(source), weakref.ref(transport), result)
+        while len(_GROUPED_TABLES) > 8:
+            del _GROUPED_TABLES[next(iter(_GROUPED_TABLES))]
     return result
 
 

@@ -20,7 +20,6 @@ forward-mode derivatives, tracing and compiling.
 from __future__ import annotations
 
 import itertools
-import threading
 import weakref
 from collections.abc import Callable, Sequence
 from typing import Any
@@ -36,7 +35,6 @@ MAX_USES = 16  # uses of one parameter entry the gradient's padded table holds
 _ALIGN = 64  # entries a form starts at a multiple of (256 bytes: whole cache lines)
 _PLAIN = (Tensor, nn.Parameter)  # subclasses may hold their numbers elsewhere
 _OFFSET = (1 << 39) - 1  # of a code: its entry's offset in the tensor
-LOCK = threading.RLock()  # plans and their tables are found by one thread at a time
 #: Plans by the module whose parameters they assemble, then by name, device and
 #: shapes: beside the modules, so that these copy, pickle and list as if there
 #: were none, and gone with them.
@@ -46,14 +44,6 @@ _PLANS: weakref.WeakKeyDictionary[Any, dict[tuple, Plan]] = weakref.WeakKeyDicti
 def _starts(sizes: Sequence[int], align: int) -> list[int]:
     """Starts of consecutive ranges of ``sizes``, each rounded up to ``align``, then the total."""
     return list(itertools.accumulate((-(-n // align) * align for n in sizes), initial=0))
-
-
-def complete(device: torch.device) -> None:
-    """Waits for what this stream writes: the kernels follow a plan's tables
-    unchecked, and other streams and threads use them without an event of this
-    one's, so they are complete before anything else can see them."""
-    if device.type == "cuda":
-        torch.cuda.current_stream(device).synchronize()
 
 
 def stream_handle(device: torch.device) -> int:
@@ -85,7 +75,7 @@ class Plan:
         self.made_on = stream_handle(device)
         self.back: Tensor | None = None
         self.back_made_on = 0
-        complete(device)
+        _native.complete(device)
 
     @staticmethod
     def _code(starts: list[int], position: Tensor, negative: Tensor) -> Tensor:
@@ -98,7 +88,7 @@ class Plan:
     def gradient_codes(self) -> Tensor:
         """``(uses, parameter entries)``: entry p's j-th use among the forms' entries."""
         if self.back is None:
-            with LOCK:
+            with _native.LOCK:
                 if self.back is None:
                     codes = self.codes[0]
                     used = torch.nonzero(codes >= 0).squeeze(1)
@@ -109,7 +99,7 @@ class Plan:
                     table = torch.full((max(self.most, 1), self.in_starts[-1]), -1, dtype=torch.int64,
                                        device=at.device)
                     table[rank, at] = self._code(self.out_starts, used[order], (codes[order] & 1) == 1)
-                    complete(table.device)
+                    _native.complete(table.device)
                     self.back_made_on = stream_handle(table.device)
                     self.back = table
         return self.back
@@ -206,7 +196,7 @@ def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[
     if (plan is None or (graded and plan.back is None)) and torch.cuda.is_current_stream_capturing():
         return build(list(params))  # finding a plan waits on the host: a captured stream takes the construction
     if plan is None:
-        with LOCK:
+        with _native.LOCK:
             plans = _PLANS.setdefault(owner, {})
             plan = plans.get(key)
             if plan is None:

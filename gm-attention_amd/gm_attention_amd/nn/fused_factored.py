@@ -160,7 +160,7 @@ def source_groups(source_index: Tensor, key: tuple | None = None,
             held, groups = hit
             same = (owner is None) if held is None else (held() is not None and held() is owner)
             if same and groups[0].device == source_index.device:
-                with assembly.LOCK:
+                with _native.LOCK:
                     if key in _GROUPS:  # not dropped by another thread meanwhile
                         _GROUPS.move_to_end(key)
                 return groups
@@ -170,8 +170,8 @@ def source_groups(source_index: Tensor, key: tuple | None = None,
     group_ptr[1:] = torch.cumsum(counts, dim=0)
     result = (order.contiguous(), group_ptr.contiguous(), group_source.contiguous())
     if key is not None:
-        assembly.complete(source_index.device)  # the kernels follow them unchecked, on whatever stream finds them
-        with assembly.LOCK:
+        _native.complete(source_index.device)  # the kernels follow them unchecked, on whatever stream finds them
+        with _native.LOCK:
             _GROUPS[key] = (None if owner is None else weakref.ref(owner), result)
             while len(_GROUPS) > GROUP_CACHE_SIZE:
                 _GROUPS.popitem(last=False)
@@ -803,7 +803,7 @@ class _SignedGather(torch.autograd.Function):
             cols = torch.full((max(uses, 1), n), total, dtype=torch.int64, device=index.device)
             cols[rank, srt] = order
             found["cols"] = cols
-        assembly.complete(index.device)
+        _native.complete(index.device)
         return found
 
     @staticmethod
@@ -819,7 +819,7 @@ class _SignedGather(torch.autograd.Function):
     def backward(ctx: Any, *grads: Tensor) -> tuple:
         plan = ctx.plan
         if "order" not in plan:
-            with assembly.LOCK:
+            with _native.LOCK:
                 if "order" not in plan:
                     plan.update(_SignedGather._gradient_plan(plan["maps"], ctx.n))
         g = torch.cat([(gi if gi is not None else torch.zeros(sh, dtype=plan["sign"].dtype, device=plan["sign"].device))
@@ -1106,7 +1106,7 @@ STREAMS_KEPT, STREAMS_SHARE = 8, 1 / 128
 
 def release_streams() -> None:
     """Gives back every edge set's streams (:func:`grouped_streams`); a later call on a set makes its own again."""
-    with assembly.LOCK:
+    with _native.LOCK:
         _STREAMS.clear()
 
 
@@ -1138,7 +1138,7 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
            pt, dtype, phases)
     hit = _STREAMS.get(key)
     if hit is not None and hit[0]() is edges.edge_index:
-        with assembly.LOCK:
+        with _native.LOCK:
             if key in _STREAMS:  # not dropped by another thread meanwhile
                 _STREAMS.move_to_end(key)
         hit[1].outlive_queue()
@@ -1165,8 +1165,8 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
     if perm.is_cuda and torch.cuda.is_current_stream_capturing():
         return streams  # the graph's own: no numbers in them before its replay, and no waiting for them here
     streams.made_on = assembly.stream_handle(perm.device)
-    assembly.complete(perm.device)  # the kernels follow them unchecked, on whatever stream finds them
-    with assembly.LOCK:
+    _native.complete(perm.device)  # the kernels follow them unchecked, on whatever stream finds them
+    with _native.LOCK:
         _STREAMS[key] = (weakref.ref(edges.edge_index), streams)
         _STREAMS.move_to_end(key)
         _trim_streams()

@@ -80,7 +80,7 @@ def test_groups_and_streams_are_complete_before_they_are_kept(monkeypatch):
     """Another stream or thread that finds them waits for nothing."""
     kept = []
     monkeypatch.setattr(fused_factored, "_GROUPS", type(fused_factored._GROUPS)())
-    monkeypatch.setattr(fused_factored.assembly, "complete",
+    monkeypatch.setattr(fused_factored._native, "complete",
                         lambda device: kept.append((len(fused_factored._GROUPS), len(fused_factored._STREAMS))))
     edges, = _edges(1)
     _streams(edges)
@@ -101,3 +101,20 @@ def test_streams_found_behind_a_busy_stream_are_complete(cuda):
     assert got.made_on == stream.cuda_stream and _streams(edges, phases=True) is got  # on the default stream
     order = torch.argsort(edges.source_index, stable=True)
     assert torch.equal(got.perm, order) and torch.equal(got.target_g, edges.target_index[order])
+
+
+def test_the_transposed_grouping_is_complete_before_it_is_kept(monkeypatch):
+    native, kept = fused_factored._native, []
+    monkeypatch.setattr(native, "_GROUPS", {})
+    monkeypatch.setattr(native, "_GROUPED_TABLES", {})
+    monkeypatch.setattr(native, "complete",
+                        lambda device: kept.append((len(native._GROUPS), len(native._GROUPED_TABLES))))
+    edges, = _edges(1)
+    source, transport = edges.source_index.contiguous(), torch.view_as_real(edges.transport_phases).contiguous()
+    target_s, inv, _ = native.source_grouped_tables(source, edges.row_ptr, transport)
+    assert kept == [(0, 0), (1, 0)] and len(native._GROUPS) == len(native._GROUPED_TABLES) == 1
+    order = torch.argsort(source, stable=True)
+    assert torch.equal(target_s.long(), edges.target_index[order]) and torch.equal(order[inv.long()],
+                                                                                   torch.arange(order.numel()))
+    native.source_grouped_tables(source, edges.row_ptr, transport)
+    assert len(kept) == 2
