@@ -29,6 +29,8 @@ from gm_attention_amd.discretization.grid import SphericalGrid
 
 
 class SphericalDiscretization:
+    _exact_copies = 1  # samples whose edges follow each other, all with the lattice distances held
+
     def __init__(self, grid: SphericalGrid, frames: Tensor, edge_geometry: EdgeGeometry, coverage_radius: float,
                  exact_distances: Tensor | None = None) -> None:
         self.grid = grid
@@ -38,7 +40,6 @@ class SphericalDiscretization:
         # one sample's, kept where the builder computed them (8 of a coverage edge's 232 bytes): at 256x512 they are
         # 126 MB, and their copy to the host was 25 of the 36 ms that from_grid took on a GPU grid
         self._exact_distances = None if exact_distances is None else exact_distances.detach().to(torch.float64)
-        self._exact_copies = 1  # samples whose edges follow each other, all with these distances
         self._radius_cache: dict[float, EdgeGeometry] = {self._key(coverage_radius): edge_geometry}
 
     @staticmethod

@@ -931,7 +931,7 @@ def _padded_shares(kernel: Any, split: int, K: int, heads: int, size: tuple[int,
     4,640).  ``size`` is (nodes, edges): what the padding adds to the layer's
     memory is bounded (:data:`PADDED_SHARE`)."""
     env = (os.environ.get("GM_FACTORED_LANES", "1"), os.environ.get("GM_FACTORED_STATIC", "1"))
-    key = ("_padded_shares", split, K, env)
+    key = ("_padded_growth", split, K, env)
     held = kernel.__dict__.get(key)
     if held is None:
         held = (0, 0, 0)  # the shares, and the reals a head's rows (an edge) and mixes (a node) grow by

@@ -21,6 +21,13 @@ def test_samples_share_their_distances_and_follow_a_move():
         got = union.edges_within(0.5)
         assert torch.equal(got.edge_index, want.edge_index) and torch.equal(got.row_ptr, want.row_ptr)
 
+    saved = two.__getstate__() if hasattr(two, "__getstate__") else None
+    saved = dict(saved or two.__dict__)  # as pickled before distances were shared: repeated, and no count
+    saved["_exact_distances"] = saved["_exact_distances"].repeat(saved.pop("_exact_copies"))
+    older = SphericalDiscretization.__new__(SphericalDiscretization)
+    older.__dict__.update(saved, _radius_cache={})
+    assert torch.equal(older.edges_within(0.5).edge_index, two.edges_within(0.5).edge_index)
+
     class OnAnotherGpu:
         device = torch.device("cuda:0")
         moved_to = None
