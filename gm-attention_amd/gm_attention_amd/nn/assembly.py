@@ -13,8 +13,9 @@ construction's own, bit for bit (moves and sign changes only).
 Parameters the kernel does not take -- CPU tensors, other types and subclasses,
 parameters on several devices or another than the current one, or not
 contiguous -- go through the construction itself, as do parameters without a
-plan on a stream under capture, and all of them under functorch transforms,
-forward-mode derivatives, tracing and compiling.
+plan on a stream under capture or in a replica of a data-parallel step, and all
+of them under functorch transforms, forward-mode derivatives, tracing and
+compiling.
 """
 
 from __future__ import annotations
@@ -193,8 +194,11 @@ def assembled(owner: Any, name: str, params: Sequence[Tensor], build: Callable[[
     key = (name, params[0].device, tuple(p.shape for p in params))
     plan = _PLANS.get(owner, {}).get(key)
     graded = torch.is_grad_enabled() and any(p.requires_grad for p in params)
-    if (plan is None or (graded and plan.back is None)) and torch.cuda.is_current_stream_capturing():
-        return build(list(params))  # finding a plan waits on the host: a captured stream takes the construction
+    if (plan is None or (graded and plan.back is None)) and (
+            torch.cuda.is_current_stream_capturing() or owner.__dict__.get("_is_replica")):
+        # finding a plan waits on the host, which a captured stream cannot, and a replica of a
+        # data-parallel step is gone after it: these take the construction
+        return build(list(params))
     if plan is None:
         with _native.LOCK:
             plans = _PLANS.setdefault(owner, {})

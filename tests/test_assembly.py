@@ -158,6 +158,27 @@ def test_shapes_and_devices_have_plans_of_their_own(on_cpu):
     assert len(assembly._PLANS[owner]) == 2
 
 
+def test_replicas_of_a_data_parallel_step_find_no_plans(on_cpu):
+    from gm_attention_amd.nn.normalization import SO2LayerNorm
+
+    norm = SO2LayerNorm(SO2FieldType({0: 4, 1: 3}))
+    replica = norm._replicate_for_data_parallel()
+    replica.gamma = norm.gamma
+    got = replica.gamma_flat(torch.float32)
+    assert replica not in assembly._PLANS and torch.equal(got, norm.gamma_flat(torch.float32))
+
+
+def test_a_plan_found_in_inference_mode_trains(on_cpu):
+    owner, params = _Owner(), [p.requires_grad_(True) for p in _params()]
+    with torch.inference_mode():
+        assembly.assembled(owner, "x", params, _build)
+    got = assembly.assembled(owner, "x", params, _build)
+    up = [torch.randn_like(g) for g in got]
+    want = torch.autograd.grad(_build(params), params, up, allow_unused=True)
+    for g, w in zip(torch.autograd.grad(got, params, up), want):
+        assert torch.allclose(g, torch.zeros_like(g) if w is None else w, rtol=0, atol=1e-6)
+
+
 def test_second_derivatives_are_the_constructions(on_cpu):
     owner, params = _Owner(), [p.requires_grad_(True) for p in _params()]
     torch.manual_seed(2)
