@@ -199,6 +199,37 @@ def complete(device: torch.device) -> None:
         torch.cuda.current_stream(device).synchronize()
 
 
+def stream_handle(device: torch.device) -> int:
+    """The device's current stream, without the object ``torch.cuda.current_stream`` makes (a microsecond)."""
+    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
+
+
+class Made:
+    """Kept tensors and the stream that makes them.  Another stream that finds
+    them waits, on the GPU, for what that one had queued, and their memory
+    outlives what the other has queued.  (For what is made again and again, as
+    tables that a bounded cache drops: :func:`complete` stops the host.)"""
+
+    def __init__(self, *tensors: Tensor | None) -> None:
+        self.tensors = [t for t in tensors if t is not None]
+        self.device = self.tensors[0].device
+        self.handle = stream_handle(self.device)
+        self.event = None
+        if self.device.type == "cuda":
+            self.event = torch.cuda.Event()
+            self.event.record(torch.cuda.current_stream(self.device))
+
+    def found(self) -> None:
+        """The current stream reads them from here on."""
+        if stream_handle(self.device) == self.handle:
+            return
+        stream = torch.cuda.current_stream(self.device)
+        if not torch.cuda.is_current_stream_capturing():  # a capture begins after all that was queued before it
+            stream.wait_event(self.event)
+        for t in self.tensors:
+            t.record_stream(stream)
+
+
 _HOST_DESC: dict[tuple, tuple[Any, Tensor]] = {}
 
 
@@ -253,7 +284,7 @@ def source_major(source: Tensor, row_ptr: Tensor) -> tuple[Tensor, Tensor, Tenso
     return result
 
 
-_GROUPED_TABLES: dict[tuple, tuple[Any, Any, tuple[Tensor, Tensor, Tensor]]] = {}
+_GROUPED_TABLES: dict[tuple, tuple[Any, Any, tuple[Tensor, Tensor, Tensor], Made]] = {}
 
 
 def source_grouped_tables(source: Tensor, row_ptr: Tensor, transport: Tensor) -> tuple[Tensor, Tensor, Tensor]:
@@ -266,6 +297,7 @@ def source_grouped_tables(source: Tensor, row_ptr: Tensor, transport: Tensor) ->
            tuple(transport.shape))
     held = _GROUPED_TABLES.get(key)
     if held is not None and held[0]() is source and held[1]() is transport:
+        held[3].found()
         return held[2]
     _check(row_ptr.shape[0] - 1 < 2**31 and source.shape[0] < 2**31,
            "the source-grouped streams index nodes and edges in 32 bits")
@@ -276,11 +308,10 @@ def source_grouped_tables(source: Tensor, row_ptr: Tensor, transport: Tensor) ->
     result = (target_s.contiguous(), inv, transport_s)
     if source.is_cuda and torch.cuda.is_current_stream_capturing():
         return result  # the graph's own: no numbers in them before its replay, and no waiting for them here
-    complete(source.device)
     with LOCK:
-        for stale in [k for k, (a, b, _) in _GROUPED_TABLES.items() if a() is None or b() is None]:
+        for stale in [k for k, (a, b, *_) in _GROUPED_TABLES.items() if a() is None or b() is None]:
             del _GROUPED_TABLES[stale]
-        _GROUPED_TABLES[key] = (weakref.ref(source), weakref.ref(transport), result)
+        _GROUPED_TABLES[key] = (weakref.ref(source), weakref.ref(transport), result, Made(*result))
         while len(_GROUPED_TABLES) > 8:
             del _GROUPED_TABLES[next(iter(_GROUPED_TABLES))]
     return result

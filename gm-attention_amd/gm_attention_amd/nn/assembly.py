@@ -47,11 +47,6 @@ def _starts(sizes: Sequence[int], align: int) -> list[int]:
     return list(itertools.accumulate((-(-n // align) * align for n in sizes), initial=0))
 
 
-def stream_handle(device: torch.device) -> int:
-    """The device's current stream, without the object ``torch.cuda.current_stream`` makes (a microsecond)."""
-    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else 0
-
-
 class Plan:
     """Where every entry of a construction's forms comes from, found on the
     parameters' device and complete on return."""
@@ -73,7 +68,7 @@ class Plan:
         self.codes = torch.where(position < 0, -1, self._code(self.in_starts, position, flat < 0)).reshape(1, -1)
         counts = torch.bincount(position.clamp_min(-1) + 1, minlength=2)[1:]
         self.most = int(counts.max())  # uses of one parameter entry
-        self.made_on = stream_handle(device)
+        self.made_on = _native.stream_handle(device)
         self.back: Tensor | None = None
         self.back_made_on = 0
         _native.complete(device)
@@ -101,14 +96,14 @@ class Plan:
                                        device=at.device)
                     table[rank, at] = self._code(self.out_starts, used[order], (codes[order] & 1) == 1)
                     _native.complete(table.device)
-                    self.back_made_on = stream_handle(table.device)
+                    self.back_made_on = _native.stream_handle(table.device)
                     self.back = table
         return self.back
 
 
 def _gather(tensors: Sequence[Tensor | None], codes: Tensor, made_on: int) -> Tensor:
     """``signed_gather`` on the current stream; a table made on another one outlives what this has queued."""
-    if stream_handle(codes.device) != made_on:
+    if _native.stream_handle(codes.device) != made_on:
         codes.record_stream(torch.cuda.current_stream(codes.device))
     return _native.signed_gather(tensors, codes)
 

@@ -1077,15 +1077,7 @@ class GroupedStreams:
     pt: int
     zw_g: Tensor | None = None  # (E, 4): r e^{i phi}, e^{i gamma} (order-1 phases) in grouping order
     group_order: Tensor | None = None
-    made_on: int = 0  # the stream they were made on: their memory returns to it
-
-    def outlive_queue(self) -> None:
-        """Keeps their memory for what the current stream has queued, should they be dropped meanwhile."""
-        if assembly.stream_handle(self.perm.device) != self.made_on:
-            stream = torch.cuda.current_stream(self.perm.device)
-            for t in (self.perm, self.inv, self.rho_g, self.phase_g, self.target_g, self.zw_g):
-                if t is not None:
-                    t.record_stream(stream)
+    made: _native.Made | None = None
 
     def bytes(self, phases: bool = False) -> int:
         """Device memory of the streams (``perm`` is the grouping's own); ``phases``: with the phase rows they lack."""
@@ -1132,8 +1124,8 @@ def _trim_streams() -> None:
 def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, dtype: torch.dtype,
                     phases: bool = True) -> GroupedStreams:
     """The grouped streams of ``edges`` under ``order`` (with the phase rows
-    only where ``phases``), complete on return and cached while the edge set
-    lives."""
+    only where ``phases``), cached while the edge set lives: a stream that finds
+    another one's waits for them (the kernels follow them unchecked)."""
     key = (id(edges.edge_index), edges.edge_index.data_ptr(), int(edges.n_edges), order.data_ptr(), float(cutoff), pa,
            pt, dtype, phases)
     hit = _STREAMS.get(key)
@@ -1141,7 +1133,7 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
         with _native.LOCK:
             if key in _STREAMS:  # not dropped by another thread meanwhile
                 _STREAMS.move_to_end(key)
-        hit[1].outlive_queue()
+        hit[1].made.found()
         return hit[1]
     with torch.profiler.record_function("gm::kernel/group_streams"):
         perm = order
@@ -1164,8 +1156,7 @@ def grouped_streams(edges: Any, order: Tensor, cutoff: float, pa: int, pt: int, 
                                  pt, zw_g)
     if perm.is_cuda and torch.cuda.is_current_stream_capturing():
         return streams  # the graph's own: no numbers in them before its replay, and no waiting for them here
-    streams.made_on = assembly.stream_handle(perm.device)
-    _native.complete(perm.device)  # the kernels follow them unchecked, on whatever stream finds them
+    streams.made = _native.Made(perm, inv, rho_g, phase_g, streams.target_g, zw_g)
     with _native.LOCK:
         _STREAMS[key] = (weakref.ref(edges.edge_index), streams)
         _STREAMS.move_to_end(key)

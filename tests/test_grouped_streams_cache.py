@@ -76,45 +76,65 @@ def test_one_devices_bound_drops_nothing_of_another():
     assert len(_kept()) < len(sets) and next(iter(fused_factored._STREAMS)) == "other"
 
 
-def test_groups_and_streams_are_complete_before_they_are_kept(monkeypatch):
-    """Another stream or thread that finds them waits for nothing."""
-    kept = []
+def _recorded(monkeypatch):
+    """What is done about other streams, in order, with what the caches hold meanwhile."""
+    native, seen = fused_factored._native, []
     monkeypatch.setattr(fused_factored, "_GROUPS", type(fused_factored._GROUPS)())
-    monkeypatch.setattr(fused_factored._native, "complete",
-                        lambda device: kept.append((len(fused_factored._GROUPS), len(fused_factored._STREAMS))))
-    edges, = _edges(1)
-    _streams(edges)
-    assert kept == [(0, 0), (1, 0)] and len(fused_factored._GROUPS) == len(fused_factored._STREAMS) == 1
-    _streams(edges)
-    assert len(kept) == 2
-
-
-@pytest.mark.gpu
-def test_streams_found_behind_a_busy_stream_are_complete(cuda):
-    edges = problems.discretization(9, 18).edge_geometry.to(cuda, torch.float32)
-    torch.cuda.synchronize()
-    stream = torch.cuda.Stream()
-    with torch.cuda.stream(stream):
-        torch.cuda._sleep(50_000_000)
-        got = _streams(edges, phases=True)
-        assert stream.query()
-    assert got.made_on == stream.cuda_stream and _streams(edges, phases=True) is got  # on the default stream
-    order = torch.argsort(edges.source_index, stable=True)
-    assert torch.equal(got.perm, order) and torch.equal(got.target_g, edges.target_index[order])
-
-
-def test_the_transposed_grouping_is_complete_before_it_is_kept(monkeypatch):
-    native, kept = fused_factored._native, []
     monkeypatch.setattr(native, "_GROUPS", {})
     monkeypatch.setattr(native, "_GROUPED_TABLES", {})
-    monkeypatch.setattr(native, "complete",
-                        lambda device: kept.append((len(native._GROUPS), len(native._GROUPED_TABLES))))
+    caches = lambda: (len(fused_factored._GROUPS), len(fused_factored._STREAMS),  # noqa: E731
+                      len(native._GROUPS), len(native._GROUPED_TABLES))
+    monkeypatch.setattr(native, "complete", lambda device: seen.append(("complete", caches())))
+    made, found = native.Made.__init__, native.Made.found
+    monkeypatch.setattr(native.Made, "__init__", lambda self, *t: (seen.append(("made", caches())), made(self, *t))[1])
+    monkeypatch.setattr(native.Made, "found", lambda self: (seen.append(("found", caches())), found(self))[1])
+    return seen
+
+
+def test_groups_are_complete_and_streams_marked_before_they_are_kept(monkeypatch):
+    seen = _recorded(monkeypatch)
+    edges, = _edges(1)
+    _streams(edges)
+    assert seen == [("complete", (0, 0, 0, 0)), ("made", (1, 0, 0, 0))]
+    _streams(edges)
+    assert seen[2:] == [("found", (1, 1, 0, 0))]
+
+
+def test_the_transposed_grouping_is_complete_and_its_tables_marked_before_they_are_kept(monkeypatch):
+    seen = _recorded(monkeypatch)
+    native = fused_factored._native
     edges, = _edges(1)
     source, transport = edges.source_index.contiguous(), torch.view_as_real(edges.transport_phases).contiguous()
     target_s, inv, _ = native.source_grouped_tables(source, edges.row_ptr, transport)
-    assert kept == [(0, 0), (1, 0)] and len(native._GROUPS) == len(native._GROUPED_TABLES) == 1
+    assert seen == [("complete", (0, 0, 0, 0)), ("made", (0, 0, 1, 0))]
     order = torch.argsort(source, stable=True)
-    assert torch.equal(target_s.long(), edges.target_index[order]) and torch.equal(order[inv.long()],
-                                                                                   torch.arange(order.numel()))
+    assert torch.equal(target_s.long(), edges.target_index[order])
+    assert torch.equal(order[inv.long()], torch.arange(order.numel()))
     native.source_grouped_tables(source, edges.row_ptr, transport)
-    assert len(kept) == 2
+    assert seen[2:] == [("found", (0, 0, 1, 1))]
+
+
+@pytest.mark.gpu
+def test_streams_made_behind_a_busy_stream_are_waited_for_by_another(cuda):
+    native = fused_factored._native
+    edges = problems.discretization(9, 18).edge_geometry.to(cuda, torch.float32)
+    source, transport = edges.source_index.contiguous(), torch.view_as_real(edges.transport_phases).contiguous()
+    order = torch.argsort(source, stable=True)
+    native.source_major(source, edges.row_ptr)
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        fused_factored.groups_for(edges, edges.source_index)
+        torch.cuda._sleep(100_000_000)  # some tens of milliseconds ahead of the tables
+        got = _streams(edges, phases=True)
+        tables = native.source_grouped_tables(source, edges.row_ptr, transport)
+    with torch.cuda.stream(second):
+        assert _streams(edges, phases=True) is got
+        read = got.target_g.clone(), got.perm.clone()
+        again = native.source_grouped_tables(source, edges.row_ptr, transport)
+        assert again is tables
+        read += tuple(t.clone() for t in again)
+        second.synchronize()
+        assert first.query()  # the reads came after what made them
+    assert torch.equal(read[1], order) and torch.equal(read[0], edges.target_index[order])
+    assert torch.equal(read[2].long(), edges.target_index[order]) and torch.equal(read[4], transport[order])
