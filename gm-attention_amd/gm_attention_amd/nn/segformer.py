@@ -107,6 +107,8 @@ class GmSegformerBlock(nn.Module):
 def _transpose(edges, n_sources: int) -> tuple[Tensor, Tensor, Tensor]:
     """``(src_ptr, order, target[order])``: the edges grouped by source (stably),
     cached on the edge set."""
+    from gm_attention_amd import _native
+
     key = ("_low_pass_transpose", n_sources)
     hit = edges.__dict__.get(key)
     if hit is None:
@@ -115,6 +117,7 @@ def _transpose(edges, n_sources: int) -> tuple[Tensor, Tensor, Tensor]:
         src_ptr = torch.zeros(n_sources + 1, dtype=torch.int64, device=source.device)
         torch.cumsum(torch.bincount(source, minlength=n_sources), dim=0, out=src_ptr[1:])
         hit = (src_ptr, order.contiguous(), edges.target_index.index_select(0, order).contiguous())
+        _native.complete(source.device)
         edges.__dict__[key] = hit
     return hit
 

@@ -138,3 +138,16 @@ def test_streams_made_behind_a_busy_stream_are_waited_for_by_another(cuda):
         assert first.query()  # the reads came after what made them
     assert torch.equal(read[1], order) and torch.equal(read[0], edges.target_index[order])
     assert torch.equal(read[2].long(), edges.target_index[order]) and torch.equal(read[4], transport[order])
+
+
+def test_the_low_passes_transpose_is_complete_before_it_is_kept(monkeypatch):
+    from gm_attention_amd.nn import segformer
+
+    edges, = _edges(1)
+    kept = []
+    monkeypatch.setattr(fused_factored._native, "complete",
+                        lambda device: kept.append([k for k in edges.__dict__ if "_low_pass_transpose" in k]))
+    n = edges.row_ptr.shape[0] - 1
+    src_ptr, order, target = segformer._transpose(edges, n)
+    assert kept == [[]] and segformer._transpose(edges, n)[0] is src_ptr and len(kept) == 1
+    assert torch.equal(target, edges.target_index[order]) and int(src_ptr[-1]) == edges.n_edges
